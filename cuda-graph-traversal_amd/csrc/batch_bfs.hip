@@ -75,13 +75,7 @@ struct BatchArgs {
 };
 
 __device__ __forceinline__ void batch_sync(BatchCtl *ctl, u32 phase, u32 level) {
-    grid_sync(&ctl->bar, &ctl->bar.error);
-    if (threadIdx.x == 0 && blockIdx.x < kMaxTraceBlocks) {
-        BlockTrace *t = &ctl->trace[blockIdx.x];
-        st_relaxed(&t->barriers, ld_relaxed(&t->barriers) + 1);
-        st_relaxed(&t->phase, phase);
-        st_relaxed(&t->a, level);
-    }
+    grid_sync(&ctl->bar, ctl->trace, phase, level, 0);
 }
 
 // Wave-converged append of records (v, mask) for lanes with `want`; also the
@@ -448,6 +442,7 @@ __device__ void bu_heavy_fixup(const BatchArgs &a, u32 L, u64 alive_cur, int nxt
 
 __global__ __launch_bounds__(512) void batch_bfs_kernel(BatchArgs a) {
     BatchCtl *ctl = a.ctl;
+    grid_join(&ctl->bar);
     const u64 gtid = (u64)blockIdx.x * blockDim.x + threadIdx.x, gthreads = (u64)gridDim.x * blockDim.x;
     const u32 lane = lane_id();
     const u64 wave_gid = gtid / kWave, nwaves = gthreads / kWave;

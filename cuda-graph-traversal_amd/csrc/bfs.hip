@@ -40,13 +40,7 @@ struct BfsCtl {
 };
 
 __device__ __forceinline__ void bfs_sync(BfsCtl *ctl, u32 phase, u32 level) {
-    grid_sync(&ctl->bar, &ctl->bar.error);
-    if (threadIdx.x == 0 && blockIdx.x < kMaxTraceBlocks) {
-        BlockTrace *t = &ctl->trace[blockIdx.x];
-        st_relaxed(&t->barriers, ld_relaxed(&t->barriers) + 1);
-        st_relaxed(&t->phase, phase);
-        st_relaxed(&t->a, level);
-    }
+    grid_sync(&ctl->bar, ctl->trace, phase, level, 0);
 }
 
 struct BfsArgs {
@@ -117,6 +111,7 @@ __device__ __forceinline__ void td_visit(const BfsArgs &a, u32 u, u32 v, bool ac
 
 __global__ __launch_bounds__(512) void bfs_kernel(BfsArgs a) {
     BfsCtl *ctl = a.ctl;
+    grid_join(&ctl->bar);
     const u64 gtid = (u64)blockIdx.x * blockDim.x + threadIdx.x;
     const u64 gthreads = (u64)gridDim.x * blockDim.x;
     const u32 lane = lane_id();

@@ -91,14 +91,7 @@ struct SsspCtl {
 enum : u32 { kPhaseInit = 1, kPhaseLight = 2, kPhaseFused = 3, kPhaseHeavy = 4, kPhaseMin = 5, kPhaseCollect = 6 };
 
 __device__ __forceinline__ void sync_traced(SsspCtl *ctl, u32 phase, u32 a, u32 b) {
-    grid_sync(&ctl->bar, &ctl->bar.error);
-    if (threadIdx.x == 0 && blockIdx.x < kMaxTraceBlocks) {
-        BlockTrace *t = &ctl->trace[blockIdx.x];
-        st_relaxed(&t->barriers, ld_relaxed(&t->barriers) + 1);
-        st_relaxed(&t->phase, phase);
-        st_relaxed(&t->a, a);
-        st_relaxed(&t->b, b);
-    }
+    grid_sync(&ctl->bar, ctl->trace, phase, a, b);
 }
 
 // A row's bounds in one 16-byte record (one memory transaction per item):
@@ -614,6 +607,7 @@ __device__ __forceinline__ void pull_step(const SsspArgs &a, u32 x, f32 lo, f32 
 
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void sssp_kernel(SsspArgs a) {
     SsspCtl *ctl = a.ctl;
+    grid_join(&ctl->bar);
     const u64 gtid = (u64)blockIdx.x * blockDim.x + threadIdx.x, gthreads = (u64)gridDim.x * blockDim.x;
     const u32 lane = lane_id();
     __shared__ int slots[1024 / kWave][kWave];

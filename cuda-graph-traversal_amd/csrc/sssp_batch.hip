@@ -162,14 +162,7 @@ struct SsspBatchArgs {
 };
 
 __device__ __forceinline__ void bsync(SsspBatchCtl *ctl, u32 phase, u32 a, u32 b) {
-    grid_sync(&ctl->bar, &ctl->bar.error);
-    if (threadIdx.x == 0 && blockIdx.x < kMaxTraceBlocks) {
-        BlockTrace *t = &ctl->trace[blockIdx.x];
-        st_relaxed(&t->barriers, ld_relaxed(&t->barriers) + 1);
-        st_relaxed(&t->phase, phase);
-        st_relaxed(&t->a, a);
-        st_relaxed(&t->b, b);
-    }
+    grid_sync(&ctl->bar, ctl->trace, phase, a, b);
 }
 
 // Per-root bucket state, the same in every block (each block keeps its copy
@@ -917,6 +910,7 @@ __device__ __forceinline__ void hub_tier(const SsspBatchArgs &a, const u32 *hv, 
 
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void sssp_batch_kernel(SsspBatchArgs a) {
     SsspBatchCtl *ctl = a.ctl;
+    grid_join(&ctl->bar);
     const u64 gtid = (u64)blockIdx.x * blockDim.x + threadIdx.x, gthreads = (u64)gridDim.x * blockDim.x;
     const u32 lane = lane_id();
     __shared__ int slots[512 / kWave][kWave];
