@@ -74,9 +74,9 @@ inline bool failed() { return t_error_sink ? t_error_sink->status != 0 : ctx().s
 void release_library_resources();
 
 // Depth of every vertex from a parent array (bfs_compute_dist_from_pred's
-// semantics) into dist[n] on the library stream; `changed` is a device u32
-// the level loop uses. Blocking.
-void depth_from_pred(const Oned_Graph *g, const i64 *pred, i64 *dist, u64 root, u32 *changed);
+// semantics) into dist[n] on the library stream; `state` is a device u32
+// that the passes use. Blocking.
+void depth_from_pred(const Oned_Graph *g, const i64 *pred, i64 *dist, u64 root, u32 *state);
 
 // Distances (f32, -1.0f unreached, original ids) from the graph's highest-degree
 // vertex into dist_dev[n], by the single-root SSSP on temporary arena memory.

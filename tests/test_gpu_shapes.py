@@ -1,0 +1,73 @@
+"""Sizes at which the kernels change how they split their work: lengths around
+the edges of their tiers, remainders, the smallest and largest of a range.
+Everything is integer or bit-exact, so results equal the oracle's."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def sess():
+    import g500
+    s = g500.Session(arena_bytes=8 << 30)
+    yield s
+    s.close()
+
+
+@pytest.fixture
+def arena(sess):
+    m = sess.mark()
+    yield sess
+    sess.release(m)
+
+
+def build(arena, n, edges, weights=None):
+    edges = np.asarray(edges, np.uint64).reshape(-1, 2)
+    if weights is None:
+        weights = np.random.default_rng(len(edges)).random(len(edges)).astype(np.float32)
+    g = arena.csr(arena.upload_tuples(edges, weights), n)
+    import pyoracle
+    return g, pyoracle.csr(n, edges, weights)
+
+
+def two_stars(length):
+    """Vertices 0 and 1, both joined to 2 .. length + 1, and to each other: rows of length + 1, a second level of 2."""
+    leaves = np.arange(2, length + 2)
+    e = [np.stack([np.full(length, c), leaves], 1) for c in (0, 1)] + [np.array([[0, 1]])]
+    return length + 2, np.concatenate(e)
+
+
+@pytest.mark.parametrize("length", [1, 7, 8, 15, 16, 62, 63, 64, 1022, 1023, 1024, 1025, 5000])
+def test_depths_of_rows_of_every_tier(arena, oracle, length):
+    n, edges = two_stars(length)
+    n += 3  # isolated vertices at the end
+    g, ref = build(arena, n, edges)
+    b = arena.bfs_create(g)
+    for root in (0, 2):
+        arena.bfs(g, b, root)
+        pred = arena.bfs_pred(b)
+        trees = [pred.copy() for _ in range(6)]
+        trees[1][1] = n - 1          # a centre's parent is no neighbour of it
+        trees[2][0 if root else 2] = n + 5
+        trees[3][length + 1] = 0     # the last leaf hangs off a centre
+        trees[4][[0, 1]] = [1, 0]    # a cycle of the two centres
+        trees[5][n - 2] = 1          # an isolated vertex with a parent
+        for k, t in enumerate(trees):
+            arena.to_device(b.pred, t)
+            got = arena.bfs_depth(g, b, root)
+            assert np.array_equal(got, oracle.dist_from_pred(ref, t, root)), (length, root, k)
+
+
+@pytest.mark.parametrize("n", [2, 33, 34, 100, 4099])
+def test_depths_of_long_chains(arena, oracle, n):
+    order = np.random.default_rng(n).permutation(n)
+    g, ref = build(arena, n, np.stack([order[:-1], order[1:]], 1))
+    b = arena.bfs_create(g)
+    root = int(order[0])
+    arena.bfs(g, b, root)
+    assert np.array_equal(arena.bfs_depth(g, b, root), oracle.bfs(ref, root)[1])
+    pred = arena.bfs_pred(b)
+    pred[order[1]] = order[min(2, n - 1)]  # the chain hangs off a cycle (or a loop) next to the root
+    arena.to_device(b.pred, pred)
+    assert np.array_equal(arena.bfs_depth(g, b, root), oracle.dist_from_pred(ref, pred, root))
