@@ -71,7 +71,7 @@ struct BatchArgs {
     i32 nroots;
     f32 alpha, beta;
     u32 hub_degree;    // top-down: records above this degree go to the grid-wide hub list
-    u32 heavy_degree;  // bottom-up: vertices above this degree are split over the grid
+    u32 heavy_degree;  // bottom-up: rows of vertices above this degree are split over the grid
 };
 
 __device__ __forceinline__ void batch_sync(BatchCtl *ctl, u32 phase, u32 level) {
@@ -233,7 +233,9 @@ __device__ __forceinline__ u64 shfl_up64(u64 v, int o) {
 }
 
 __device__ __forceinline__ u64 uniform64(u64 v) {
-    return ((u64)__builtin_amdgcn_readfirstlane((u32)(v >> 32)) << 32) | __builtin_amdgcn_readfirstlane((u32)v);
+    // the builtin returns an int: without the casts the low half would sign-extend into the high one
+    return ((u64)(u32)__builtin_amdgcn_readfirstlane((u32)(v >> 32)) << 32) |
+           (u32)__builtin_amdgcn_readfirstlane((u32)v);
 }
 
 __device__ __forceinline__ bool frontier_bit(const u64 *fb, u32 v) { return (fb[v >> 6] >> (v & 63)) & 1; }
@@ -376,8 +378,11 @@ __device__ void bu_groups(const BatchArgs &a, u32 L, u64 alive_cur, int nxt, u64
     stage_flush();
 }
 
-// Heavy vertices with missing roots: their edge lists in 256-edge chunks over
-// the grid; each chunk ORs its finds into next[v].
+// Heavy vertices with missing roots: their rows' flattened space is cut into
+// spans of kHeavySpan entries over the grid; a wave walks the row pieces of
+// its span, ORs a piece's finds into next[v], and leaves a row as soon as its
+// missing roots are found here or were by another wave.
+constexpr u64 kHeavySpan = 16 * kHubChunk;
 __device__ void bu_heavy_chunks(const BatchArgs &a, u32 L, u64 alive_cur) {
     const u64 *fmc = a.fm[L & 1], *fbc = a.fb[L & 1];
     const u32 lane = lane_id();
@@ -388,26 +393,42 @@ __device__ void bu_heavy_chunks(const BatchArgs &a, u32 L, u64 alive_cur) {
     const u64 hb = 2 * a.n;
     const u32 *hv = a.hubs + hb, *hlen = a.hlen + hb;
     const u64 *hoff = a.hoff + hb;
-    u64 hi_idx = 0;
-    for (u64 c = wave_gid; c * kHubChunk < ht; c += nwaves) {
-        const u64 p = c * kHubChunk;
-        hi_idx = hub_locate(hoff, hi_idx, nh, p);
-        const u32 v = hv[hi_idx];
-        const u64 need = uniform64(alive_cur & ~a.seen[v]);
-        if (!need) continue;
-        if ((uniform64(ld_relaxed(&a.next[v])) & need) == need) continue;
-        const u64 b = a.rs[v] + (p - hoff[hi_idx]), e = a.rs[v] + hlen[hi_idx];
-        u64 acc = 0;
+    u64 i = 0;
+    for (u64 c = wave_gid; c * kHeavySpan < ht; c += nwaves) {
+        u64 p = c * kHeavySpan;
+        const u64 pend = min(p + kHeavySpan, ht);
+        for (i = hub_locate(hoff, i, nh, p); p < pend && i < nh; ++i) {  // padded ranges follow each other
+            const u32 v = hv[i], len = hlen[i];
+            const u64 off = hoff[i], r0 = a.rs[v];
+            const u64 next = off + ((u64)len + kHubChunk - 1) / kHubChunk * kHubChunk;
+            u64 need = uniform64(alive_cur & ~a.seen[v]);
+            if (need) need &= ~uniform64(ld_relaxed(&a.next[v]));
+            u64 acc = 0;
+            const u64 e = r0 + min((u64)len, pend - off);
+            for (u64 k = r0 + (p - off) + lane; need && k - lane < e; k += kSteps * kWave) {
+                u32 w[kSteps];
+                bool ok[kSteps];
+                u64 m = 0;
 #pragma unroll
-        for (u64 j = 0; j < kHubChunk; j += kWave) {
-            const u64 k = b + j + lane;
-            if (k < e) {
-                const u32 w = a.col[k];
-                if (frontier_bit(fbc, w)) acc |= fmc[w] & need;
+                for (int q = 0; q < kSteps; ++q) {
+                    ok[q] = k + (u64)q * kWave < e;
+                    w[q] = ok[q] ? a.col[k + (u64)q * kWave] : 0;
+                }
+#pragma unroll
+                for (int q = 0; q < kSteps; ++q) ok[q] = ok[q] && frontier_bit(fbc, w[q]);
+#pragma unroll
+                for (int q = 0; q < kSteps; ++q) m |= ok[q] ? fmc[w[q]] : 0;
+                m &= need;
+                if (!ballot(m != 0)) continue;
+                for (int o = 32; o > 0; o >>= 1) m |= shfl_xor64(m, o);
+                m = uniform64(m);
+                acc |= m;
+                need &= ~m;
             }
+            if (lane == 0 && acc) atomicOr((unsigned long long *)&a.next[v], (unsigned long long)acc);
+            p = next;
         }
-        for (int o = 32; o > 0; o >>= 1) acc |= shfl_xor64(acc, o);
-        if (lane == 0 && acc) atomicOr((unsigned long long *)&a.next[v], (unsigned long long)acc);
+        i = i ? i - 1 : 0;  // the next span starts at or after the last row walked
     }
 }
 
@@ -614,6 +635,20 @@ __global__ __launch_bounds__(256) void batch_depth_scatter(const u32 *__restrict
     }
 }
 
+// Degree above which a bottom-up level splits a vertex's row over the grid,
+// whatever the knob allows. The wave that owns 64 vertices of this degree
+// walks 64 times as many entries alone (the degree order puts them together),
+// so the bound grows with the number of vertex groups a wave has to amortise
+// that over; long rows cost a few dependent loads each, so it does not fall
+// below 256. 64 roots, ms at a bound of 256 / 512 / 1024 / 4096 / none:
+// S16 (1 group a wave at most) 1.02 / 1.08 / 2.18 / 4.89 / 7.49,
+// S21 (8) 2.35 / 2.40 / 3.41 / 6.22 / 23.9, S24 (64) 8.95 / 8.67 / 9.00 / 11.3 / 21.1,
+// S26 (256) 39.1 / 39.0 / 37.3 / 37.6 / 42.9.
+static u64 heavy_bound(u64 n, u64 nwaves) {
+    const u64 groups = (n / kWave + nwaves - 1) / nwaves;  // vertex groups per wave
+    return MAX((u64)256, MIN(8 * groups, (u64)1024));
+}
+
 bool bfs_batch_enqueue(const Oned_Graph *g, Bfs_Batch_State *b, const u64 *roots, i32 nroots, hipStream_t stream,
                        int grid) {
     Context &c = ctx();
@@ -666,10 +701,10 @@ bool bfs_batch_enqueue(const Oned_Graph *g, Bfs_Batch_State *b, const u64 *roots
     a.alpha = (f32)c.batch_alpha;
     a.beta = (f32)c.batch_beta;
     a.hub_degree = (u32)c.bfs_hub_degree;
-    a.heavy_degree = (u32)c.batch_heavy_degree;
     const int block = ctx().batch_bfs_block;
     if (grid <= 0) grid = cooperative_blocks((const void *)batch_bfs_kernel, block, 0);
     if (failed()) return false;
+    a.heavy_degree = (u32)MIN((u64)c.batch_heavy_degree, heavy_bound(n, (u64)grid * (u64)block / kWave));
     void *args[] = {&a};
     b->nroots = nroots;
     if (library) {

@@ -71,3 +71,25 @@ def test_depths_of_long_chains(arena, oracle, n):
     pred[order[1]] = order[min(2, n - 1)]  # the chain hangs off a cycle (or a loop) next to the root
     arena.to_device(b.pred, pred)
     assert np.array_equal(arena.bfs_depth(g, b, root), oracle.dist_from_pred(ref, pred, root))
+
+
+# bottom-up levels of the batched BFS: rows below and above the degree that is
+# split over the grid (256 on graphs of these sizes), and around the 4096-entry spans
+@pytest.mark.parametrize("length", [255, 256, 257, 4095, 4096, 4097, 8192, 20000])
+@pytest.mark.parametrize("nroots", [1, 5, 64])
+def test_batch_bfs_bottom_up_long_rows(arena, oracle, length, nroots):
+    n, edges = two_stars(length)
+    n += 7  # a tail of three vertices off the last leaf (the discovery log holds 8n records), four isolated ones
+    chain = np.stack([np.arange(n - 8, n - 5), np.arange(n - 7, n - 4)], 1)
+    g, ref = build(arena, n, np.concatenate([edges, chain]))
+    b = arena.batch_create(g)
+    rng = np.random.default_rng(length)
+    roots = np.concatenate([[n - 5, 0, 2, n - 1, n - 8], rng.integers(0, n, 59)])[:nroots]
+    old = arena.get_param("batch_alpha")
+    try:
+        arena.set_param("batch_alpha", 1e9)  # every level bottom-up
+        arena.batch(g, b, roots)
+    finally:
+        arena.set_param("batch_alpha", old)
+    for i in sorted({0, 1, 2, 3, 4, nroots - 1} & set(range(nroots))):
+        assert np.array_equal(arena.batch_depth(g, b, i), oracle.bfs(ref, int(roots[i]))[1]), (length, i)
