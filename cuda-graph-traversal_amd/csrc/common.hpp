@@ -110,6 +110,20 @@ inline void sync() { G500_HIP(hipStreamSynchronize(ctx().stream)); }
 // the CU's LDS without allocation rounding is never taken.
 int cooperative_blocks(const void *kernel, int block, size_t dyn_lds);
 
+// Grid of a persistent kernel for a launch of `work` (entries times roots, in
+// units that take a block about as long as a barrier takes per block): at most
+// `full`, the co-resident grid of `block` threads. Every step costs its share
+// of the work, which falls with the blocks, and a barrier, which grows with
+// them (2.6 us at 32 blocks of 512 threads, 6.7 us at 512), so the best grid
+// grows with the square root of the work. Measured on Kronecker graphs, us at
+// 16 / 32 / 64 / 128 / 256 / 512 blocks: SSSP S12 432 / 435 / 446 / 469 / 516 / 606,
+// S16 1089 / 928 / 879 / 931 / 994 / 1158, S20 - / 4217 / 3033 / 2344 / 2131 / 2257,
+// S22 - / - / 12151 / 7865 / 5422 / 4806; BFS S12 104 / 105 / 108 / 111 / 124 / 143,
+// S20 - / 547 / 401 / 348 / 369 / 418; batched SSSP, 32 roots, S12
+// 5595 / 5238 / 5135 / 5214 / 5719 / 6848, S20 - / - / 54580 / 38302 / 31711 / 29702;
+// batched BFS S16 1073 / 873 / 779 / 776 / 803 / 849, S22 - / - / 13815 / 7318 / 4217 / 3389.
+int persistent_grid(u64 work, int full, int block);
+
 // Launches a persistent kernel whose grid fits on the device at once. With
 // `cooperative`, uses a cooperative launch; if the runtime refuses it (the
 // cooperative queue is held by another process on the same device), or

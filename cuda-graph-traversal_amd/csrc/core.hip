@@ -1,5 +1,7 @@
 // Library context, errors, arenas, single-rank worker and control entry points.
 // Reference: src/base.cu:1-78, src/worker.cu:6-109.
+#include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <mutex>
 #include <string>
@@ -88,6 +90,12 @@ int cooperative_blocks(const void *kernel, int block, size_t dyn_lds) {
         return 1;
     }
     return per_cu * ctx().num_cus;
+}
+
+int persistent_grid(u64 work, int full, int block) {
+    // whole rounds over 8 XCDs; smaller blocks in proportion more
+    const f64 blocks = std::sqrt((f64)work) * 512.0 / block;
+    return (int)std::min<f64>(full, 8.0 * std::ceil(std::max(blocks, 1.0) / 8.0));
 }
 
 void launch_persistent(const void *kernel, int grid, int block, void **args, hipStream_t stream,

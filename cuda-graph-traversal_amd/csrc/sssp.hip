@@ -1050,7 +1050,8 @@ void oned_graph_sssp_run(Worker_State *ws, const Oned_Graph *g, Sssp_State *s, u
     a.delta = s->delta;
     a.dbound = g->rowstarts_s ? kPruneDistBound : __builtin_inff();
     const int block = ctx().sssp_block;
-    int grid = cooperative_blocks((const void *)sssp_kernel, block, 0);
+    const int grid =
+        persistent_grid(g->nlocaledges / 512, cooperative_blocks((const void *)sssp_kernel, block, 0), block);
     if (failed()) return;
     void *args[] = {&a};
     G500_HIP(hipMemsetAsync(s->ctl, 0, sizeof(SsspCtl), c.stream));

@@ -1730,6 +1730,10 @@ void sssp_batch_lags(const f32 *offsets, i32 nroots, f32 delta, u32 *lag, f32 *u
     }
 }
 
+static int launch_grid(const Oned_Graph *g, i32 nroots, int full) {
+    return persistent_grid(g->nlocaledges * (u64)nroots / 1024, full, ctx().batch_sssp_block);
+}
+
 bool sssp_batch_enqueue(const Oned_Graph *g, Sssp_Batch_State *s, const u64 *roots, const f32 *offsets, i32 nroots,
                         hipStream_t stream, int grid) {
     Context &c = ctx();
@@ -1831,13 +1835,14 @@ bool sssp_batch_enqueue(const Oned_Graph *g, Sssp_Batch_State *s, const u64 *roo
     a.dw[2] = wfar;
     const int block = ctx().batch_sssp_block;
     const size_t dyn = q_lds_bytes(block);
-    if (grid <= 0) grid = cooperative_blocks((const void *)sssp_batch_kernel, block, dyn);
+    const int full = grid > 0 ? grid : cooperative_blocks((const void *)sssp_batch_kernel, block, dyn);
     if (failed()) return false;
+    grid = launch_grid(g, nroots, full);
     void *args[] = {&a};
     s->nroots = nroots;
-    // the export's grid: as many blocks as the persistent grid holds waves / 4, at most one per 64 ids
+    // the export's grid: as many blocks as the full grid holds waves / 4, at most one per 64 ids
     const unsigned xgrid = (unsigned)std::max<u64>(1, std::min<u64>((n + kExportIds - 1) / kExportIds,
-                                                                     (u64)grid * (u64)block / 256));
+                                                                     (u64)full * (u64)block / 256));
     auto export_labels = [&]() {
         sssp_batch_export_kernel<<<xgrid, 256, 0, st>>>(a.lab, a.perm, a.iperm, n, nroots, a.dbound, a.dist, a.pred,
                                                         a.ctl);
@@ -1924,7 +1929,7 @@ void oned_graph_sssp_batch_run_offsets(Worker_State *ws, const Oned_Graph *g, Ss
         // where the blocks stood: the fewest and most grid barriers passed, with the phase and tags of each
         static SsspBatchCtl h;
         g500_copy_to_host(&h, s->ctl, sizeof(h));
-        const int nb = std::min(sssp_batch_grid(), kMaxTraceBlocks);
+        const int nb = std::min(launch_grid(g, nroots, sssp_batch_grid()), kMaxTraceBlocks);
         u32 lo = 0xFFFFFFFFu, hi = 0;
         int at_lo = 0, at_hi = 0;
         for (int b = 0; b < nb; ++b) {
