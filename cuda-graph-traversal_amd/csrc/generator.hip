@@ -123,45 +123,119 @@ G500_HD u64 scramble(u64 v, int lgN, u64 sum01, u64 mul0, u64 mul1) {
     return v;
 }
 
-// One block per 256-edge tile whose first edge index is a multiple of 256:
-// the state skip over bytes 1..7 of the edge index is uniform across the block
-// (scalar), each lane then applies the power for its low byte.
+// MRG step for residues: A1 z1 + A5 z5 < 2^59, so one fold (x mod 2^31 plus
+// x / 2^31) stays below 2^31 + 2^28 and one conditional subtraction reduces it.
+__device__ __forceinline__ u32 mrg_step(u32 z1, u32 z5) {
+    const u64 x = kA1 * z1 + kA5 * z5;
+    const u32 r = ((u32)x & kP) + (u32)(x >> 31);
+    return min(r, r - kP);
+}
+
+// Quadrants of an edge's levels (graph_generation.cu:114-143, :186-207): bit
+// strings of the source and target, one level per call, highest first.
+struct Quadrants {
+    u32 src = 0, tgt = 0;
+    bool same = true;      // src == tgt so far
+    bool rejected = false;
+    // u < 0x7FFFFFFF mod 10000 decides, by u mod 10000 < 1900 (B), < 3800 (C),
+    // < 9500 (A), else D; u below 3647 is rejected. u mod 10000 is compared as
+    // a fraction: with c = ceil(2^45 / 10000), u c mod 2^45 lies in
+    // [r, r + 0.072) 2^45 / 10000 for r = u mod 10000 (u (10000 c - 2^45) <
+    // 0.072 2^45), so bits 13..44 of u c compare like r with floor(t 2^32 / 10000).
+    __device__ __forceinline__ void level(u32 u) {
+        rejected |= u < 3647u;
+        const u64 p = (u64)u * 3518437209u;
+        const u32 f = __builtin_amdgcn_alignbit((u32)(p >> 32), (u32)p, 13);
+        const bool b = f < 816043786u;                          // 1900
+        const bool c = f - 816043786u < 1632087572u - 816043786u;  // 3800
+        const bool d = f >= 4080218931u;                        // 9500
+        const bool swap = same && c;  // no (1, 0) while the two are equal
+        same = same && !(b || c);
+        src = 2 * src + ((c && !swap) || d);
+        tgt = 2 * tgt + (b || d || swap);
+    }
+};
+
+// All levels from state st, and the weight's number. Levels run five at a time
+// so that the five state words keep their registers; a rejected number (4 in
+// 10^5 edges) is noticed at the end, and its edge is made again step by step.
+__device__ __forceinline__ void make_edge(Mrg_State st, int logN, u32 &src, u32 &tgt, u32 &wz) {
+    Quadrants q;
+    u32 a = st.z1, b = st.z2, c = st.z3, d = st.z4, e = st.z5;
+    int lvl = logN;
+    for (; lvl % 5; --lvl) {
+        const u32 n = mrg_step(a, e);
+        e = d;
+        d = c;
+        c = b;
+        b = a;
+        a = n;
+        q.level(n);
+    }
+    for (; lvl; lvl -= 5) {
+        e = mrg_step(a, e);
+        q.level(e);
+        d = mrg_step(e, d);
+        q.level(d);
+        c = mrg_step(d, c);
+        q.level(c);
+        b = mrg_step(c, b);
+        q.level(b);
+        a = mrg_step(b, a);
+        q.level(a);
+    }
+    wz = mrg_step(a, e);
+    if (q.rejected) {
+        q = Quadrants();
+        for (lvl = logN; lvl; --lvl) {
+            u32 u = mrg_next(st);
+            while (u < 3647u) u = mrg_next(st);
+            q.level(u);
+        }
+        wz = mrg_next(st);
+    }
+    src = q.src;
+    tgt = q.tgt;
+}
+
+// A block makes a run of consecutive 256-edge tiles whose first edge indexes
+// are multiples of 256. The state skip over bytes 1..7 of the edge index is
+// uniform across the block (scalar) and made once per run; each lane then
+// applies the power for its low byte, and one uniform power per further tile.
+// Bound by integer VALU: three 64-bit multiply-adds and about 17 other
+// operations a level. 250e6 edges of S24: 3.93 ms, 1.27 TB/s written (6.38 ms
+// with a skip per tile, state words moved at each level, a test for rejection
+// at each level and u mod 10000 computed in full). `tile_run` is 8, fewer when
+// that would leave CUs without blocks.
+constexpr i64 kTileRun = 8;
 __global__ __launch_bounds__(256) void kronecker_kernel(
     Mrg_State seed, const Mrg_Transition_Matrix *__restrict__ T, int logN, i64 start, i64 end,
     u64 sum01, u64 mul0, u64 mul1, Packed_Edge *__restrict__ edges, f32 *__restrict__ weights,
-    i64 tile_first, i64 tile_count) {
-    for (i64 t = blockIdx.x; t < tile_count; t += gridDim.x) {
-        const i64 tile = tile_first + t;
+    i64 tile_first, i64 tile_count, i64 tile_run) {
+    const Mrg_Transition_Matrix tile_step = T[9 * 256 + 1];
+    for (i64 t0 = (i64)blockIdx.x * tile_run; t0 < tile_count; t0 += (i64)gridDim.x * tile_run) {
         Mrg_State st = seed;
-        u64 hi = (u64)tile;
+        u64 hi = (u64)(tile_first + t0);
         for (int b = 9; hi; ++b, hi >>= 8) {
             const u32 byte = (u32)hi & 0xFF;
             if (byte) mrg_apply(T[b * 256 + byte], st);
         }
-        const i64 ei = tile * 256 + threadIdx.x;
-        if (ei < start || ei >= end) continue;
-        if (threadIdx.x) mrg_apply(T[8 * 256 + threadIdx.x], st);
-        // graph_generation.cu:114-143, :186-207: one quadrant per level,
-        // rejecting u < 0x7FFFFFFF mod 10000.
-        u64 src = 0, tgt = 0;
-        for (int lvl = logN - 1; lvl >= 0; --lvl) {
-            u32 u = mrg_next(st);
-            while (u < 3647u) u = mrg_next(st);
-            u %= 10000u;
-            u32 so, to;
-            if (u < 1900u) { so = 0; to = 1; }         // B
-            else if (u < 3800u) { so = 1; to = 0; }    // C
-            else if (u < 9500u) { so = 0; to = 0; }    // A
-            else { so = 1; to = 1; }                   // D
-            if (src == tgt && so > to) { so = 0; to = 1; }
-            src |= (u64)so << lvl;
-            tgt |= (u64)to << lvl;
+        mrg_apply(T[8 * 256 + threadIdx.x], st);  // the identity for thread 0
+        const i64 t1 = min(t0 + tile_run, tile_count);
+        for (i64 t = t0;;) {
+            const i64 ei = (tile_first + t) * 256 + threadIdx.x;
+            if (ei >= start && ei < end) {
+                u32 src, tgt, wz;
+                make_edge(st, logN, src, tgt, wz);
+                Packed_Edge e;
+                e.v0 = scramble(src, logN, sum01, mul0, mul1);
+                e.v1 = scramble(tgt, logN, sum01, mul0, mul1);
+                edges[ei - start] = e;
+                weights[ei - start] = (f32)wz * 0x1p-31f;  // graph_generation.cu:88-90
+            }
+            if (++t == t1) break;
+            mrg_apply(tile_step, st);
         }
-        Packed_Edge e;
-        e.v0 = scramble(src, logN, sum01, mul0, mul1);
-        e.v1 = scramble(tgt, logN, sum01, mul0, mul1);
-        edges[ei - start] = e;
-        weights[ei - start] = (f32)mrg_next(st) * 0x1p-31f;  // graph_generation.cu:88-90
     }
 }
 
@@ -214,11 +288,13 @@ void generate_kronecker_range(Worker_State *ws, u32 seed[5], u32 logN, i64 start
 
     const i64 tile_first = start_edge >> 8;
     const i64 tile_count = ((end_edge - 1) >> 8) - tile_first + 1;
-    i64 grid = c.gen_blocks > 0 ? c.gen_blocks : MIN(tile_count, (i64)c.num_cus * 2048);
+    const i64 tile_run = MAX((i64)1, MIN(kTileRun, tile_count / ((i64)c.num_cus * 16)));
+    const i64 runs = (tile_count + tile_run - 1) / tile_run;
+    i64 grid = c.gen_blocks > 0 ? c.gen_blocks : MIN(runs, (i64)c.num_cus * 2048);
     timer_start();
     kronecker_kernel<<<(unsigned)grid, 256, 0, c.stream>>>(
         st, c.d_mrg_table, (int)logN, start_edge, end_edge, val0 + val1, val0 | 0x4519840211493211ull,
-        val1 | 0x3050852102C843A5ull, tg->edges, tg->weights, tile_first, tile_count);
+        val1 | 0x3050852102C843A5ull, tg->edges, tg->weights, tile_first, tile_count, tile_run);
     G500_HIP(hipGetLastError());
     timer_stop();
 }

@@ -93,3 +93,14 @@ def test_batch_bfs_bottom_up_long_rows(arena, oracle, length, nroots):
         arena.set_param("batch_alpha", old)
     for i in sorted({0, 1, 2, 3, 4, nroots - 1} & set(range(nroots))):
         assert np.array_equal(arena.batch_depth(g, b, i), oracle.bfs(ref, int(roots[i]))[1]), (length, i)
+
+
+# edge ranges that end inside tiles and runs of tiles, every remainder of the levels (five at a time),
+# and enough edges that some take a rejected number (4 in 10^5)
+@pytest.mark.parametrize("scale,start,end", [(1, 0, 32), (2, 3, 61), (4, 0, 257), (6, 255, 1024), (18, 255, 1100001),
+                                             (21, 1, 20000001), (24, 2**28 - 9_000_000, 2**28)])
+def test_generator_runs_and_remainders(arena, oracle, scale, start, end):
+    e, w = arena.tuples_to_host(arena.generate(scale, 16, start=start, end=end))
+    eo, wo = oracle.kronecker(scale, 16, start=start, end=end)
+    assert np.array_equal(e, eo)
+    assert np.array_equal(w.view(np.uint32), wo.view(np.uint32))
