@@ -156,10 +156,31 @@ struct Quadrants {
     }
 };
 
-// All levels from state st, and the weight's number. Levels run five at a time
-// so that the five state words keep their registers; a rejected number (4 in
-// 10^5 edges) is noticed at the end, and its edge is made again step by step.
-__device__ __forceinline__ void make_edge(Mrg_State st, int logN, u32 &src, u32 &tgt, u32 &wz) {
+// All levels from state st, and the weight's number, one level at a time.
+__device__ __forceinline__ void make_edge_stepwise(const Mrg_State &st, int logN, u32 &src, u32 &tgt, u32 &wz) {
+    Quadrants q;
+    u32 a = st.z1, b = st.z2, c = st.z3, d = st.z4, e = st.z5;
+    for (int lvl = logN; lvl;) {
+        const u32 n = mrg_step(a, e);
+        e = d;
+        d = c;
+        c = b;
+        b = a;
+        a = n;
+        if (n >= 3647u) {
+            q.level(n);
+            --lvl;
+        }
+    }
+    wz = mrg_step(a, e);
+    src = q.src;
+    tgt = q.tgt;
+}
+
+// The same, five levels at a time so that the five state words keep their
+// registers; a rejected number (4 in 10^5 edges) is noticed at the end, and
+// its edge is made again.
+__device__ __forceinline__ void make_edge(const Mrg_State &st, int logN, u32 &src, u32 &tgt, u32 &wz) {
     Quadrants q;
     u32 a = st.z1, b = st.z2, c = st.z3, d = st.z4, e = st.z5;
     int lvl = logN;
@@ -185,17 +206,9 @@ __device__ __forceinline__ void make_edge(Mrg_State st, int logN, u32 &src, u32 
         q.level(a);
     }
     wz = mrg_step(a, e);
-    if (q.rejected) {
-        q = Quadrants();
-        for (lvl = logN; lvl; --lvl) {
-            u32 u = mrg_next(st);
-            while (u < 3647u) u = mrg_next(st);
-            q.level(u);
-        }
-        wz = mrg_next(st);
-    }
     src = q.src;
     tgt = q.tgt;
+    if (q.rejected) make_edge_stepwise(st, logN, src, tgt, wz);
 }
 
 // A block makes a run of consecutive 256-edge tiles whose first edge indexes
@@ -207,7 +220,11 @@ __device__ __forceinline__ void make_edge(Mrg_State st, int logN, u32 &src, u32 
 // with a skip per tile, state words moved at each level, a test for rejection
 // at each level and u mod 10000 computed in full). `tile_run` is 8, fewer when
 // that would leave CUs without blocks.
+// STEPWISE, for launches of up to two tiles per CU: those wait for their
+// slowest wave, and the few edges made again would be that (code not fetched
+// before): 65000 edges 8.7 us, 10.2 unrolled; 300000 edges 16.0 us, 14.8 unrolled.
 constexpr i64 kTileRun = 8;
+template <bool STEPWISE>
 __global__ __launch_bounds__(256) void kronecker_kernel(
     Mrg_State seed, const Mrg_Transition_Matrix *__restrict__ T, int logN, i64 start, i64 end,
     u64 sum01, u64 mul0, u64 mul1, Packed_Edge *__restrict__ edges, f32 *__restrict__ weights,
@@ -226,7 +243,8 @@ __global__ __launch_bounds__(256) void kronecker_kernel(
             const i64 ei = (tile_first + t) * 256 + threadIdx.x;
             if (ei >= start && ei < end) {
                 u32 src, tgt, wz;
-                make_edge(st, logN, src, tgt, wz);
+                if (STEPWISE) make_edge_stepwise(st, logN, src, tgt, wz);
+                else make_edge(st, logN, src, tgt, wz);
                 Packed_Edge e;
                 e.v0 = scramble(src, logN, sum01, mul0, mul1);
                 e.v1 = scramble(tgt, logN, sum01, mul0, mul1);
@@ -292,7 +310,8 @@ void generate_kronecker_range(Worker_State *ws, u32 seed[5], u32 logN, i64 start
     const i64 runs = (tile_count + tile_run - 1) / tile_run;
     i64 grid = c.gen_blocks > 0 ? c.gen_blocks : MIN(runs, (i64)c.num_cus * 2048);
     timer_start();
-    kronecker_kernel<<<(unsigned)grid, 256, 0, c.stream>>>(
+    auto *kernel = tile_count <= (i64)c.num_cus * 2 ? kronecker_kernel<true> : kronecker_kernel<false>;
+    kernel<<<(unsigned)grid, 256, 0, c.stream>>>(
         st, c.d_mrg_table, (int)logN, start_edge, end_edge, val0 + val1, val0 | 0x4519840211493211ull,
         val1 | 0x3050852102C843A5ull, tg->edges, tg->weights, tile_first, tile_count, tile_run);
     G500_HIP(hipGetLastError());
