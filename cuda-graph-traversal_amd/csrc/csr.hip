@@ -141,6 +141,223 @@ __global__ __launch_bounds__(256) void fill_kernel(const Packed_Edge *__restrict
     }
 }
 
+// ------------------------------------------------------- partition into rows
+// Rows filled through cursors in tuple order (degree_kernel, fill_kernel) cost
+// two random atomics and a random 8-byte write per entry: 34 ms of a 90 ms S23
+// construction (7.9 ms now). Large tuple lists are instead split by row in two or three
+// passes of at most kPartBins buckets per tile, high bits first: a block takes
+// a tile of entries, ranks them per bucket in LDS, reserves one run per bucket
+// with one atomic, and writes the runs from LDS in bucket order, so that
+// neighbouring lanes write neighbouring entries. The last pass's buckets are
+// the rows. Each pass is a histogram (4-8 bytes read per entry), a scan and a
+// scatter (12 read, 12 or 8 written); order inside a bucket does not matter,
+// the rows are sorted afterwards.
+constexpr int kPartThreads = 1024, kPartItems = 8, kPartTile = kPartThreads * kPartItems;
+constexpr u32 kPartBins = 2048;
+
+struct PartArgs {
+    const Packed_Edge *edges;  // pass 1: tuples (two entries each, loops dropped), else null
+    const f32 *ew;
+    const u32 *row_in, *col_in, *w_in;
+    u64 count;                 // tuples or entries
+    u64 n;
+    u32 shift;                 // bucket = row >> shift
+    u64 *next;                 // next free position per bucket (not the last pass)
+    const u64 *rs;             // last pass: row offsets
+    u32 *used;                 //   and entries placed per row
+    u32 *row_out, *col_out, *w_out;  // row_out null in the last pass
+};
+
+__device__ __forceinline__ u64 part_reserve(const PartArgs &a, u32 bucket, u32 k) {
+    return a.next ? atomicAdd((unsigned long long *)&a.next[bucket], (unsigned long long)k)
+                  : a.rs[bucket] + atomicAdd(&a.used[bucket], k);
+}
+
+template <bool TUPLES>
+__global__ __launch_bounds__(kPartThreads) void partition_kernel(PartArgs a) {
+    __shared__ u32 s_row[kPartTile], s_col[kPartTile], s_w[kPartTile];
+    __shared__ u32 bins[kPartBins];  // counts, then the bucket's first place in the tile
+    __shared__ u64 dst[kPartBins];   // the bucket's reserved run
+    __shared__ u32 wave_sum_[kPartThreads / kWave];
+    __shared__ u32 s_lo, s_hi;
+    const u32 tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+    constexpr u64 kPer = TUPLES ? kPartTile / 2 : kPartTile;
+    for (u64 t0 = (u64)blockIdx.x * kPer; t0 < a.count; t0 += (u64)gridDim.x * kPer) {
+        u32 row[kPartItems], col[kPartItems], w[kPartItems];
+        bool ok[kPartItems];
+        if (tid == 0) {
+            s_lo = ~0u;
+            s_hi = 0;
+        }
+        if (TUPLES) {
+#pragma unroll
+            for (int k = 0; k < kPartItems; k += 2) {
+                const u64 i = t0 + (u64)(k / 2) * kPartThreads + tid;
+                Packed_Edge e = {0, 0};
+                u32 wb = 0;
+                if (i < a.count) {
+                    e = a.edges[i];
+                    wb = __float_as_uint(a.ew[i]);
+                }
+                ok[k] = ok[k + 1] = e.v0 != e.v1 && e.v0 < a.n && e.v1 < a.n;
+                row[k] = col[k + 1] = (u32)e.v0;
+                row[k + 1] = col[k] = (u32)e.v1;
+                w[k] = w[k + 1] = wb;
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < kPartItems; ++k) {
+                const u64 i = t0 + (u64)k * kPartThreads + tid;
+                ok[k] = i < a.count;
+                row[k] = ok[k] ? a.row_in[i] : 0;
+                col[k] = ok[k] ? a.col_in[i] : 0;
+                w[k] = ok[k] ? a.w_in[i] : 0;
+            }
+        }
+        u32 lo = ~0u, hi = 0;
+#pragma unroll
+        for (int k = 0; k < kPartItems; ++k)
+            if (ok[k]) {
+                lo = min(lo, row[k] >> a.shift);
+                hi = max(hi, row[k] >> a.shift);
+            }
+        lo = wave_min(lo);
+        hi = ~wave_min(~hi);
+        __syncthreads();
+        if (lane == 0) {
+            atomicMin(&s_lo, lo);
+            atomicMax(&s_hi, hi);
+        }
+        __syncthreads();
+        lo = s_lo;
+        hi = s_hi;
+        if (lo > hi || hi - lo >= kPartBins) {
+            // no entries, or a stretch of almost empty buckets: entry by entry
+#pragma unroll
+            for (int k = 0; k < kPartItems; ++k)
+                if (ok[k]) {
+                    const u64 g = part_reserve(a, row[k] >> a.shift, 1);
+                    a.col_out[g] = col[k];
+                    a.w_out[g] = w[k];
+                    if (a.row_out) a.row_out[g] = row[k];
+                }
+            __syncthreads();  // s_lo and s_hi are set again by the next tile
+            continue;
+        }
+        const u32 nb = hi - lo + 1;
+        for (u32 b = tid; b < kPartBins; b += kPartThreads) bins[b] = 0;
+        __syncthreads();
+        u32 rank[kPartItems];
+#pragma unroll
+        for (int k = 0; k < kPartItems; ++k) rank[k] = ok[k] ? atomicAdd(&bins[(row[k] >> a.shift) - lo], 1u) : 0;
+        __syncthreads();
+        static_assert(kPartBins == 2 * kPartThreads, "two buckets per thread");
+        const u32 c0 = bins[2 * tid], c1 = bins[2 * tid + 1];
+        const u32 incl = wave_inclusive_scan(c0 + c1);
+        if (lane == kWave - 1) wave_sum_[wave] = incl;
+        __syncthreads();
+        u32 before = incl - c0 - c1, total = 0;
+        for (u32 i = 0; i < kPartThreads / kWave; ++i) {
+            before += i < wave ? wave_sum_[i] : 0u;
+            total += wave_sum_[i];
+        }
+        bins[2 * tid] = before;
+        bins[2 * tid + 1] = before + c0;
+        if (2 * tid < nb && c0) dst[2 * tid] = part_reserve(a, lo + 2 * tid, c0);
+        if (2 * tid + 1 < nb && c1) dst[2 * tid + 1] = part_reserve(a, lo + 2 * tid + 1, c1);
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kPartItems; ++k)
+            if (ok[k]) {
+                const u32 p = bins[(row[k] >> a.shift) - lo] + rank[k];
+                s_row[p] = row[k];
+                s_col[p] = col[k];
+                s_w[p] = w[k];
+            }
+        __syncthreads();
+        for (u32 p = tid; p < total; p += kPartThreads) {
+            const u32 r = s_row[p], b = (r >> a.shift) - lo;
+            const u64 g = dst[b] + (p - bins[b]);
+            a.col_out[g] = s_col[p];
+            a.w_out[g] = s_w[p];
+            if (a.row_out) a.row_out[g] = r;
+        }
+        __syncthreads();
+    }
+}
+
+// Entries per bucket of pass 1, from the tuples; flags endpoints out of range.
+__global__ __launch_bounds__(1024) void partition_count_tuples(const Packed_Edge *__restrict__ edges, u64 ne, u64 n,
+                                                               u32 shift, u32 *__restrict__ counts,
+                                                               u32 *__restrict__ bad) {
+    __shared__ u32 h[kPartBins];
+    for (u32 b = threadIdx.x; b < kPartBins; b += blockDim.x) h[b] = 0;
+    __syncthreads();
+    for (u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x; i < ne; i += (u64)gridDim.x * blockDim.x) {
+        const Packed_Edge e = edges[i];
+        if (e.v0 >= n || e.v1 >= n) {
+            atomicOr(bad, 1u);
+            continue;
+        }
+        if (e.v0 == e.v1) continue;
+        atomicAdd(&h[(u32)(e.v0 >> shift)], 1u);
+        atomicAdd(&h[(u32)(e.v1 >> shift)], 1u);
+    }
+    __syncthreads();
+    for (u32 b = threadIdx.x; b < kPartBins; b += blockDim.x)
+        if (h[b]) atomicAdd(&counts[b], h[b]);
+}
+
+// Entries per bucket of a later pass, from the rows of the pass before: a
+// block's tile lies in few parents, so its buckets are counted in LDS.
+constexpr u32 kCountBins = 4096;
+constexpr int kCountItems = 16;
+__global__ __launch_bounds__(1024) void partition_count_rows(const u32 *__restrict__ rows, u64 count, u32 shift,
+                                                             u32 *__restrict__ counts) {
+    __shared__ u32 h[kCountBins];
+    __shared__ u32 s_lo, s_hi;
+    constexpr u64 kPer = 1024 * kCountItems;
+    for (u64 t0 = (u64)blockIdx.x * kPer; t0 < count; t0 += (u64)gridDim.x * kPer) {
+        if (threadIdx.x == 0) {
+            s_lo = ~0u;
+            s_hi = 0;
+        }
+        for (u32 b = threadIdx.x; b < kCountBins; b += blockDim.x) h[b] = 0;
+        u32 b[kCountItems], lo = ~0u, hi = 0;
+#pragma unroll
+        for (int k = 0; k < kCountItems; ++k) {
+            const u64 i = t0 + (u64)k * 1024 + threadIdx.x;
+            b[k] = i < count ? rows[i] >> shift : 0u;
+        }
+        auto valid = [&](int k) { return t0 + (u64)k * 1024 + threadIdx.x < count; };
+#pragma unroll
+        for (int k = 0; k < kCountItems; ++k)
+            if (valid(k)) {
+                lo = min(lo, b[k]);
+                hi = max(hi, b[k]);
+            }
+        lo = wave_min(lo);
+        hi = ~wave_min(~hi);
+        __syncthreads();
+        if (lane_id() == 0) {
+            atomicMin(&s_lo, lo);
+            atomicMax(&s_hi, hi);
+        }
+        __syncthreads();
+        lo = s_lo;
+        hi = s_hi;
+        const bool narrow = hi - lo < kCountBins;
+#pragma unroll
+        for (int k = 0; k < kCountItems; ++k)
+            if (valid(k)) atomicAdd(narrow ? &h[b[k] - lo] : &counts[b[k]], 1u);
+        __syncthreads();
+        if (narrow)
+            for (u32 q = threadIdx.x; q <= hi - lo; q += blockDim.x)
+                if (h[q]) atomicAdd(&counts[lo + q], h[q]);
+        __syncthreads();
+    }
+}
+
 // ------------------------------------------------------------------ row sort
 struct SortLists {
     u32 n1, n2, n3;       // rows in tiers 1..3
@@ -780,6 +997,180 @@ void build_traversal_copy(Worker_State *ws, Oned_Graph *g) {
     if (c.sssp_prune && !failed()) build_sssp_copy(ws, g, nlong, hc[0]);
 }
 
+// Tuple lists below this take the direct path, where the partition's launches
+// cost more than scattered accesses in cache. Whole construction, direct /
+// partition, us: 48 Ki tuples (3000 uniform vertices) 490 / 520, S12 (64 Ki)
+// 876 / 800, S14 1259 / 1045, S16 2346 / 1762, S18 5046 / 3673, S20 14348 / 11278,
+// S22 47674 / 34400.
+constexpr u64 kPartitionTuples = 1ull << 16;
+
+// Exclusive scan of counts[0, n) into offsets[0, n], the total last.
+static void scan_counts(const u32 *counts, u64 n, u64 *tiles, u64 *offsets, hipStream_t s) {
+    const u64 ntiles = (n + kScanTile - 1) / kScanTile;
+    scan_tile_sums<<<(unsigned)ntiles, kScanBlock, 0, s>>>(counts, n, tiles);
+    scan_tile_offsets<<<1, 1024, 0, s>>>(tiles, ntiles, offsets, n);
+    scan_write<<<(unsigned)ntiles, kScanBlock, 0, s>>>(counts, n, tiles, offsets);
+    G500_HIP(hipGetLastError());
+}
+static u64 scan_tile_bytes(u64 n) { return ((n + kScanTile - 1) / kScanTile + 1) * sizeof(u64); }
+
+static bool bad_endpoints(u64 n) {
+    fail("oned_graph_from_tuple_graph: tuple endpoint outside [0, %llu)", (unsigned long long)n);
+    return false;
+}
+
+// Row offsets, columns and weights (rows unsorted) through per-row cursors.
+static bool fill_direct(Worker_State *ws, const Tuple_Graph *tg, Oned_Graph *g) {
+    Context &c = ctx();
+    const hipStream_t s = c.stream;
+    const u64 n = g->nlocalverts, ne = tg->edges_size;
+    const u64 mark = ws->gpu_arena.used;
+    u32 *deg = (u32 *)arena_alloc(ws, n * sizeof(u32), "CSR degrees");
+    u64 *tiles = (u64 *)arena_alloc(ws, scan_tile_bytes(n) + 16, "CSR scan tiles");
+    if (failed()) return false;
+    u32 *bad = (u32 *)((u8 *)tiles + scan_tile_bytes(n));
+    G500_HIP(hipMemsetAsync(deg, 0, n * sizeof(u32), s));
+    G500_HIP(hipMemsetAsync(bad, 0, sizeof(u32), s));
+    if (ne) degree_kernel<<<grid_for(ne, 256, (u64)c.num_cus * 64), 256, 0, s>>>(tg->edges, ne, n, deg, bad);
+    scan_counts(deg, n, tiles, g->rowstarts, s);
+    u64 m = 0;
+    u32 hbad = 0;
+    G500_HIP(hipMemcpyAsync(&m, g->rowstarts + n, sizeof(u64), hipMemcpyDeviceToHost, s));
+    G500_HIP(hipMemcpyAsync(&hbad, bad, sizeof(u32), hipMemcpyDeviceToHost, s));
+    sync();
+    if (hbad) return bad_endpoints(n);
+    if (failed()) return false;
+    // the scratch moves above the column and weight arrays, to be released afterwards
+    ws->gpu_arena.used = mark;
+    g->nlocaledges = m;
+    g->column = (u32 *)arena_alloc(ws, m * sizeof(u32), "CSR columns");
+    g->weights = (f32 *)arena_alloc(ws, m * sizeof(f32), "CSR weights");
+    const u64 mark_fill = ws->gpu_arena.used;
+    u32 *cursor = (u32 *)arena_alloc(ws, n * sizeof(u32), "CSR cursors");
+    if (failed()) return false;
+    G500_HIP(hipMemsetAsync(cursor, 0, n * sizeof(u32), s));
+    if (ne)
+        fill_kernel<<<grid_for(ne, 256, (u64)c.num_cus * 64), 256, 0, s>>>(tg->edges, tg->weights, ne, n,
+                                                                          g->rowstarts, cursor, g->column,
+                                                                          g->weights);
+    G500_HIP(hipGetLastError());
+    ws->gpu_arena.used = mark_fill;
+    return !failed();
+}
+
+// Whether the partition path is taken: large lists, whose counts fit 32 bits,
+// when the arena has room for its scratch (16 bytes an entry beside the
+// columns and weights; the copies built later need as much).
+static bool partition_pays(const Worker_State *ws, u64 n, u64 ne) {
+    const u64 room = ws->gpu_arena.reserved - ws->gpu_arena.used;
+    return ne >= kPartitionTuples && 2 * ne < (1ull << 32) && 2 * ne * 24 + n * 5 + (64ull << 20) <= room;
+}
+
+// The same arrays by partition (see partition_kernel).
+static bool fill_partitioned(Worker_State *ws, const Tuple_Graph *tg, Oned_Graph *g) {
+    Context &c = ctx();
+    const hipStream_t s = c.stream;
+    const u64 n = g->nlocalverts, ne = tg->edges_size;
+    const u64 mark = ws->gpu_arena.used;
+    u32 bits = 1;
+    while (bits < 32 && (1ull << bits) < n) ++bits;
+    // two passes up to 2^18 rows, else three; at most 11 bits each
+    const u32 d1 = bits <= 18 ? (bits + 1) / 2 : (bits + 2) / 3;
+    const u32 shift1 = bits - d1, shift2 = bits <= 18 ? 0 : shift1 / 2;
+    const u64 nb1 = ((n - 1) >> shift1) + 1, nb2 = ((n - 1) >> shift2) + 1;
+    // pass 1's counts, whose sum is the number of entries
+    std::vector<u32> h(nb1 + 1);
+    std::vector<u64> first(nb1 + 1);
+    u32 *count1 = (u32 *)arena_alloc(ws, (kPartBins + 1) * sizeof(u32), "CSR partition counts");
+    if (failed()) return false;
+    G500_HIP(hipMemsetAsync(count1, 0, (kPartBins + 1) * sizeof(u32), s));
+    partition_count_tuples<<<(unsigned)c.num_cus * 2, 1024, 0, s>>>(tg->edges, ne, n, shift1, count1,
+                                                                   count1 + kPartBins);
+    G500_HIP(hipGetLastError());
+    G500_HIP(hipMemcpyAsync(h.data(), count1, nb1 * sizeof(u32), hipMemcpyDeviceToHost, s));
+    G500_HIP(hipMemcpyAsync(&h[nb1], count1 + kPartBins, sizeof(u32), hipMemcpyDeviceToHost, s));
+    sync();
+    if (failed()) return false;
+    if (h[nb1]) return bad_endpoints(n);
+    u64 m = 0;
+    for (u64 b = 0; b < nb1; ++b) {
+        first[b] = m;
+        m += h[b];
+    }
+    ws->gpu_arena.used = mark;
+    g->nlocaledges = m;
+    g->column = (u32 *)arena_alloc(ws, m * sizeof(u32), "CSR columns");
+    g->weights = (f32 *)arena_alloc(ws, m * sizeof(f32), "CSR weights");
+    const u64 mark_fill = ws->gpu_arena.used;
+    u64 *next1 = (u64 *)arena_alloc(ws, nb1 * sizeof(u64), "CSR partition offsets");
+    u32 *deg = (u32 *)arena_alloc(ws, n * sizeof(u32), "CSR degrees");
+    u64 *tiles = (u64 *)arena_alloc(ws, scan_tile_bytes(n), "CSR scan tiles");
+    // the last pass's input, and pass 1's rows when there are three
+    u32 *row2 = (u32 *)arena_alloc(ws, m * sizeof(u32), "CSR partition rows");
+    u32 *col2 = (u32 *)arena_alloc(ws, m * sizeof(u32), "CSR partition columns");
+    u32 *w2 = (u32 *)arena_alloc(ws, m * sizeof(u32), "CSR partition weights");
+    u32 *row1 = shift2 ? (u32 *)arena_alloc(ws, m * sizeof(u32), "CSR partition rows") : nullptr;
+    u64 *next2 = shift2 ? (u64 *)arena_alloc(ws, (nb2 + 1) * sizeof(u64), "CSR partition offsets") : nullptr;
+    if (failed()) return false;
+    const unsigned max_blocks = (unsigned)c.num_cus;  // a block's LDS fills a CU
+    const unsigned count_blocks = grid_for(m, 1024 * kCountItems, (u64)c.num_cus * 4);
+    auto pass = [&](auto tuples, PartArgs a) {
+        constexpr bool kTuples = decltype(tuples)::value;
+        partition_kernel<kTuples><<<grid_for(a.count, kTuples ? kPartTile / 2 : kPartTile, max_blocks), kPartThreads,
+                                    0, s>>>(a);
+    };
+    PartArgs a = {};
+    a.edges = tg->edges;
+    a.ew = tg->weights;
+    a.count = ne;
+    a.n = n;
+    a.shift = shift1;
+    a.next = next1;
+    G500_HIP(hipMemcpyAsync(next1, first.data(), nb1 * sizeof(u64), hipMemcpyHostToDevice, s));
+    if (shift2) {
+        a.row_out = row1;
+        a.col_out = g->column;
+        a.w_out = (u32 *)g->weights;
+        pass(std::true_type(), a);
+        G500_HIP(hipMemsetAsync(deg, 0, nb2 * sizeof(u32), s));
+        partition_count_rows<<<count_blocks, 1024, 0, s>>>(row1, m, shift2, deg);
+        scan_counts(deg, nb2, tiles, next2, s);
+        a.edges = nullptr;
+        a.row_in = row1;
+        a.col_in = g->column;
+        a.w_in = (const u32 *)g->weights;
+        a.count = m;
+        a.shift = shift2;
+        a.next = next2;
+    }
+    a.row_out = row2;
+    a.col_out = col2;
+    a.w_out = w2;
+    if (shift2) pass(std::false_type(), a);
+    else pass(std::true_type(), a);
+    G500_HIP(hipMemsetAsync(deg, 0, n * sizeof(u32), s));
+    partition_count_rows<<<count_blocks, 1024, 0, s>>>(row2, m, 0, deg);
+    scan_counts(deg, n, tiles, g->rowstarts, s);
+    G500_HIP(hipMemsetAsync(deg, 0, n * sizeof(u32), s));
+    a.edges = nullptr;
+    a.row_in = row2;
+    a.col_in = col2;
+    a.w_in = w2;
+    a.count = m;
+    a.shift = 0;
+    a.next = nullptr;
+    a.rs = g->rowstarts;
+    a.used = deg;
+    a.row_out = nullptr;
+    a.col_out = g->column;
+    a.w_out = (u32 *)g->weights;
+    pass(std::false_type(), a);
+    G500_HIP(hipGetLastError());
+    sync();  // `first` is read by the copy
+    ws->gpu_arena.used = mark_fill;
+    return !failed();
+}
+
 }  // namespace g500
 
 using namespace g500;
@@ -798,52 +1189,19 @@ Oned_Graph oned_graph_from_tuple_graph(Worker_State *ws, Tuple_Graph *tg, u64 ng
         return g;
     }
     const u64 ne = tg->edges_size;
-    const u64 mark = ws->gpu_arena.used;  // scratch above this mark is released at the end
     g.rowstarts = (u64 *)arena_alloc(ws, (n + 1) * sizeof(u64), "CSR row offsets");
     if (failed()) return g;
-    // Scratch: degrees/cursors, scan tile sums, sort lists.
-    const u64 mark_scratch = ws->gpu_arena.used;
-    u32 *deg = (u32 *)arena_alloc(ws, n * sizeof(u32), "CSR degrees");
-    const u64 ntiles = (n + kScanTile - 1) / kScanTile;
-    u64 *tiles = (u64 *)arena_alloc(ws, (ntiles + 1) * sizeof(u64), "CSR scan tiles");
-    if (failed()) return g;
-    u32 *bad = (u32 *)(tiles + ntiles);
-    timer_start();
     const hipStream_t s = c.stream;
-    G500_HIP(hipMemsetAsync(deg, 0, n * sizeof(u32), s));
-    G500_HIP(hipMemsetAsync(bad, 0, sizeof(u32), s));
-    if (ne) degree_kernel<<<grid_for(ne, 256, (u64)c.num_cus * 64), 256, 0, s>>>(tg->edges, ne, n, deg, bad);
-    scan_tile_sums<<<(unsigned)ntiles, kScanBlock, 0, s>>>(deg, n, tiles);
-    scan_tile_offsets<<<1, 1024, 0, s>>>(tiles, ntiles, g.rowstarts, n);
-    scan_write<<<(unsigned)ntiles, kScanBlock, 0, s>>>(deg, n, tiles, g.rowstarts);
-    G500_HIP(hipGetLastError());
-    u64 m = 0;
-    u32 hbad = 0;
-    G500_HIP(hipMemcpyAsync(&m, g.rowstarts + n, sizeof(u64), hipMemcpyDeviceToHost, s));
-    G500_HIP(hipMemcpyAsync(&hbad, bad, sizeof(u32), hipMemcpyDeviceToHost, s));
-    sync();
-    if (hbad) fail("oned_graph_from_tuple_graph: tuple endpoint outside [0, %llu)", (unsigned long long)n);
-    if (failed()) return g;
-    // Column / weight arrays are allocated below the scratch so that the
-    // scratch can be released afterwards: move the scratch region up.
-    ws->gpu_arena.used = mark_scratch;
-    g.nlocaledges = m;
-    g.column = (u32 *)arena_alloc(ws, m * sizeof(u32), "CSR columns");
-    g.weights = (f32 *)arena_alloc(ws, m * sizeof(f32), "CSR weights");
+    timer_start();
+    if (!(partition_pays(ws, n, ne) ? fill_partitioned(ws, tg, &g) : fill_direct(ws, tg, &g))) return g;
     const u64 mark_sort = ws->gpu_arena.used;
-    u32 *cursor = (u32 *)arena_alloc(ws, n * sizeof(u32), "CSR cursors");
     SortLists *L = (SortLists *)arena_alloc(ws, sizeof(SortLists), "sort lists");
     u32 *t1 = (u32 *)arena_alloc(ws, n * sizeof(u32), "sort tier 1");
     u32 *t2 = (u32 *)arena_alloc(ws, n * sizeof(u32), "sort tier 2");
     u32 *t3 = (u32 *)arena_alloc(ws, n * sizeof(u32), "sort tier 3");
     u64 *t3_off = (u64 *)arena_alloc(ws, n * sizeof(u64), "sort tier 3 offsets");
     if (failed()) return g;
-    G500_HIP(hipMemsetAsync(cursor, 0, n * sizeof(u32), s));
     G500_HIP(hipMemsetAsync(L, 0, sizeof(SortLists), s));
-    if (ne)
-        fill_kernel<<<grid_for(ne, 256, (u64)c.num_cus * 64), 256, 0, s>>>(tg->edges, tg->weights, ne, n,
-                                                                          g.rowstarts, cursor, g.column,
-                                                                          g.weights);
     classify_rows<<<grid_for(n, 256, (u64)c.num_cus * 16), 256, 0, s>>>(g.rowstarts, n, L, t1, t2, t3, t3_off);
     sort_rows_thread<<<grid_for(n, 256, (u64)c.num_cus * 32), 256, 0, s>>>(g.rowstarts, n, g.column, g.weights);
     G500_HIP(hipGetLastError());
@@ -872,7 +1230,6 @@ Oned_Graph oned_graph_from_tuple_graph(Worker_State *ws, Tuple_Graph *tg, u64 ng
     ws->gpu_arena.used = mark_sort;  // release the scratch
     if (c.relabel) build_traversal_copy(ws, &g);
     timer_stop();
-    (void)mark;
     return g;
 }
 

@@ -104,3 +104,38 @@ def test_generator_runs_and_remainders(arena, oracle, scale, start, end):
     eo, wo = oracle.kronecker(scale, 16, start=start, end=end)
     assert np.array_equal(e, eo)
     assert np.array_equal(w.view(np.uint32), wo.view(np.uint32))
+
+
+def csr_equal(arena, g, ref):
+    rs, col, w = arena.csr_to_host(g)
+    assert np.array_equal(rs, ref.rowstarts)
+    assert np.array_equal(col, ref.column)
+    assert np.array_equal(w.view(np.uint32), ref.weights.view(np.uint32))
+
+
+# tuple lists large enough for the partition: vertex counts around its digit
+# splits (two passes up to 2^18, three above), one so sparse that a tile spans
+# more buckets than it ranks, a hub with half of all entries, and loops
+@pytest.mark.parametrize("n", [3, 255, 1000, 2**18 - 1, 2**18, 2**18 + 1, 700001, 2**22 + 5, 3 * 10**7])
+def test_csr_partition(arena, oracle, n):
+    rng = np.random.default_rng(n)
+    ne = 2**20 + 4097
+    e = rng.integers(0, n, (ne, 2))
+    if n == 2**18:
+        e[: ne // 2, 0] = n - 1
+    if n == 1000:
+        e[:5000, 1] = e[:5000, 0]
+    if n == 3 * 10**7:  # a dense corner and rows far apart
+        e[: ne // 2] %= 4096
+    g, ref = build(arena, n, e)
+    csr_equal(arena, g, ref)
+
+
+@pytest.mark.parametrize("ne", [2**16 - 1, 2**16])
+def test_csr_partition_rejects_endpoints_out_of_range(arena, ne):
+    import g500
+    e = np.random.default_rng(1).integers(0, 5000, (ne, 2)).astype(np.uint64)
+    e[ne // 3, 1] = 5000
+    tg = arena.upload_tuples(e, np.ones(ne, np.float32))
+    with pytest.raises(g500.LibraryError, match="outside"):
+        arena.csr(tg, 5000)
