@@ -287,8 +287,8 @@ constexpr u64 kHubChunk = 256;
 constexpr int kHubCountShift = 38;
 constexpr u64 kHubTotalMask = (1ull << kHubCountShift) - 1;
 
-__device__ __forceinline__ u64 hub_count(u64 packed) { return packed >> kHubCountShift; }
-__device__ __forceinline__ u64 hub_total(u64 packed) { return packed & kHubTotalMask; }
+__host__ __device__ __forceinline__ u64 hub_count(u64 packed) { return packed >> kHubCountShift; }
+__host__ __device__ __forceinline__ u64 hub_total(u64 packed) { return packed & kHubTotalMask; }
 
 // Wave-converged append of (v, len) for lanes with `want`; returns the lane's
 // slot (~0 when it appended nothing).

@@ -2,14 +2,13 @@
 // Reference: src/traversal.cu:15-73 (degree / rowstart / fill kernels),
 // :342-410 (oned_graph_from_tuple_graph, oned_graph_is_vertex_isolated).
 //
-// Steps: (1) degree histogram with u32 device atomics, self-loops skipped;
-// (2) three-phase exclusive scan into u64 row offsets; (3) fill of both
-// directions of every non-loop tuple edge through per-row cursors; (4) each
-// row sorted ascending by the key (f32 weight bits << 32 | column), which
-// makes the CSR deterministic and puts light edges first in every row. Rows
-// are sorted by one of four tiers: a thread (<= 16 entries), a wave
-// (<= 64), a block in LDS (<= 4096), or a block-wide LSD radix sort through a
-// scratch buffer (longer rows).
+// Steps: (1) both directions of every non-loop tuple edge are put in row order,
+// small lists through a degree histogram and per-row cursors, large ones by a
+// partition in passes; (2) a three-phase exclusive scan of the row lengths
+// gives u64 row offsets; (3) each row is sorted ascending by the key
+// (f32 weight bits << 32 | column), which makes the CSR deterministic and puts
+// light edges first in every row. Rows are sorted by a thread (<= 16 entries) or a wave (<= 512); longer ones are
+// split by weight into bins that a wave sorts.
 #include <algorithm>
 #include <cstdio>
 #include <vector>
@@ -359,35 +358,74 @@ __global__ __launch_bounds__(1024) void partition_count_rows(const u32 *__restri
 }
 
 // ------------------------------------------------------------------ row sort
+// Tiers by row length: 2..16 a thread, 17..64 / 128 / 256 / 512 a wave with 1
+// / 2 / 4 / 8 entries per lane; longer rows are split by weight into bins of
+// about kBinEntries, which a wave sorts too (see the long rows below).
+constexpr int kWaveTiers = 4;            // 64 << t entries
+constexpr u32 kLongRow = 512;            // rows above it are long
+constexpr u32 kSegBlock = 4096;          // longest segment that one block sorts in LDS
 struct SortLists {
-    u32 n1, n2, n3;       // rows in tiers 1..3
-    u32 pad;
-    u64 scratch_total;    // entries of tier-3 rows
-    u64 notisolated;
+    CounterLine<u32> n[kWaveTiers];      // rows per wave tier
+    CounterLine<u64> longs;              // packed hub counter of the long rows
+    CounterLine<u64> long_entries;       // their entries
+    CounterLine<u64> huge_entries;       //   of those above kSegBlock
+    CounterLine<u32> nblock, nradix;     // segments for the block and radix sorts
+    CounterLine<u64> notisolated;
+};
+// Rows of a tier's list are at least `least` entries long, so M entries have
+// at most this many of them.
+static u64 tier_cap(u64 n, u64 m, u64 least) { return MIN(n, m / least + 1); }
+
+struct TierLists {
+    u32 *rows[kWaveTiers];
+    u32 *long_row, *long_len;
+    u64 *long_off;
+    u64 long_cap;
 };
 
-__global__ __launch_bounds__(256) void classify_rows(const u64 *__restrict__ rs, u64 n, SortLists *L,
-                                                     u32 *__restrict__ t1, u32 *__restrict__ t2,
-                                                     u32 *__restrict__ t3, u64 *__restrict__ t3_off) {
-    u32 local_nonzero = 0;
-    const u64 stride = (u64)gridDim.x * blockDim.x;
-    const u64 nround = (n + stride - 1) / stride * stride;  // every lane runs the same trip count
-    for (u64 v = (u64)blockIdx.x * blockDim.x + threadIdx.x; v < nround; v += stride) {
-        u64 d = v < n ? rs[v + 1] - rs[v] : 0;
-        local_nonzero += d > 0;
-        bool a = d > 16 && d <= 64, b = d > 64 && d <= 4096, c = d > 4096;
-        u32 s1 = wave_append(&L->n1, a);
-        u32 s2 = wave_append(&L->n2, b);
-        u32 s3 = wave_append(&L->n3, c);
-        if (a) t1[s1] = (u32)v;
-        if (b) t2[s2] = (u32)v;
-        if (c) {
-            t3[s3] = (u32)v;
-            t3_off[s3] = atomicAdd((unsigned long long *)&L->scratch_total, (unsigned long long)d);
+// The lists are staged in LDS per tile of rows, one atomic per list and tile
+// (one per wave and list on neighbouring counters took 3.4 ms at S23, this 0.6).
+constexpr int kClassifyTile = 1024;
+__global__ __launch_bounds__(1024) void classify_rows(const u64 *__restrict__ rs, u64 n, SortLists *L, TierLists t,
+                                                      u32 *__restrict__ error) {
+    __shared__ u32 stage[kWaveTiers][kClassifyTile];
+    __shared__ u32 cnt[kWaveTiers], base[kWaveTiers];
+    u32 nonzero = 0;
+    u64 longs = 0, huge = 0;
+    for (u64 v0 = (u64)blockIdx.x * kClassifyTile; v0 < n; v0 += (u64)gridDim.x * kClassifyTile) {
+        if (threadIdx.x < kWaveTiers) cnt[threadIdx.x] = 0;
+        __syncthreads();
+        for (int k = 0; k < kClassifyTile; k += 1024) {
+            const u64 v = v0 + k + threadIdx.x;
+            const u64 d = v < n ? rs[v + 1] - rs[v] : 0;
+            nonzero += d > 0;
+            const bool is_long = d > kLongRow;
+            if (is_long) {
+                longs += d;
+                huge += d > kSegBlock ? d : 0;
+            }
+            hub_append(&L->longs.v, t.long_row, t.long_off, t.long_len, is_long, (u32)v, (u32)d, t.long_cap, error);
+            if (d > 16 && !is_long) {
+                const int tier = d <= 64 ? 0 : d <= 128 ? 1 : d <= 256 ? 2 : 3;
+                stage[tier][atomicAdd(&cnt[tier], 1u)] = (u32)v;
+            }
         }
+        __syncthreads();
+        if (threadIdx.x < kWaveTiers)
+            base[threadIdx.x] = cnt[threadIdx.x] ? atomicAdd(&L->n[threadIdx.x].v, cnt[threadIdx.x]) : 0;
+        __syncthreads();
+        for (int q = 0; q < kWaveTiers; ++q)
+            for (u32 i = threadIdx.x; i < cnt[q]; i += 1024) t.rows[q][base[q] + i] = stage[q][i];
+        __syncthreads();
     }
-    u32 tot = wave_sum(local_nonzero);
-    if (lane_id() == 0 && tot) atomicAdd((unsigned long long *)&L->notisolated, (unsigned long long)tot);
+    const u32 tot = wave_sum(nonzero);
+    longs = wave_sum(longs);
+    huge = wave_sum(huge);
+    if (lane_id() == 0) {
+        if (tot) atomicAdd((unsigned long long *)&L->notisolated.v, (unsigned long long)tot);
+        if (longs) atomicAdd((unsigned long long *)&L->long_entries.v, (unsigned long long)longs);
+        if (huge) atomicAdd((unsigned long long *)&L->huge_entries.v, (unsigned long long)huge);
+    }
 }
 
 // Tier 0: rows of 2..16 entries, one thread each, bitonic network in registers.
@@ -425,46 +463,103 @@ __global__ __launch_bounds__(256) void sort_rows_thread(const u64 *__restrict__ 
     }
 }
 
-// Tier 1: rows of 17..64 entries, one wave each, bitonic across lanes.
-__global__ __launch_bounds__(256) void sort_rows_wave(const u64 *__restrict__ rs, const u32 *__restrict__ rows,
-                                                      const SortLists *L, u32 *__restrict__ col,
-                                                      f32 *__restrict__ cw) {
-    const u32 count = L->n1;
-    const int lane = lane_id();
-    const u32 waves = gridDim.x * (blockDim.x / kWave);
-    for (u32 r = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave; r < count; r += waves) {
-        const u32 v = rows[r];
-        const u64 b = rs[v];
-        const u32 d = (u32)(rs[v + 1] - b);
-        u64 x = (u32)lane < d ? make_key(col[b + lane], cw[b + lane]) : ~0ull;
+// Ascending bitonic sort of a wave's 64 E keys, E per lane, key p in lane p / E:
+// strides below E stay in a lane's registers, the others are 21 lane exchanges
+// of each key for any E.
+template <int E>
+__device__ __forceinline__ void wave_sort(u64 (&x)[E]) {
+    const u32 lane = lane_id();
 #pragma unroll
-        for (int size = 2; size <= kWave; size <<= 1)
+    for (int size = 2; size <= kWave * E; size <<= 1)
 #pragma unroll
-            for (int stride = size / 2; stride > 0; stride >>= 1) {
-                u64 y = shfl_xor64(x, stride);
-                const bool up = (lane & size) == 0, lower = (lane & stride) == 0;
-                x = (lower == up) ? (x < y ? x : y) : (x < y ? y : x);
+        for (int stride = size / 2; stride > 0; stride >>= 1) {
+            if (stride >= E) {
+                const bool lower = (lane & (u32)(stride / E)) == 0;
+                const bool up = (lane * E & (u32)size) == 0;  // size > stride >= E: the lane alone decides
+#pragma unroll
+                for (int i = 0; i < E; ++i) {
+                    const u64 y = shfl_xor64(x[i], stride / E);
+                    x[i] = (lower == up) ? (x[i] < y ? x[i] : y) : (x[i] < y ? y : x[i]);
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < E; ++i) {
+                    const int j = i ^ stride;
+                    if (j > i) {
+                        const bool up = ((lane * E + (u32)i) & (u32)size) == 0;
+                        if ((x[i] > x[j]) == up) {
+                            const u64 t = x[i];
+                            x[i] = x[j];
+                            x[j] = t;
+                        }
+                    }
+                }
             }
-        if ((u32)lane < d) {
-            col[b + lane] = (u32)x;
-            cw[b + lane] = __uint_as_float((u32)(x >> 32));
+        }
+}
+
+// Sorts src[0, len) (len <= 64 E) into dst; they may be the same place.
+template <int E>
+__device__ __forceinline__ void wave_sort_segment(const u32 *src_col, const u32 *src_w, u32 *col, u32 *w, u32 len) {
+    const u32 lane = lane_id();
+    u64 x[E];
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+        const u32 p = (u32)i * kWave + lane;
+        x[i] = p < len ? ((u64)src_w[p] << 32) | src_col[p] : ~0ull;
+    }
+    wave_sort(x);
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+        const u32 p = lane * E + (u32)i;
+        if (p < len) {
+            col[p] = (u32)x[i];
+            w[p] = (u32)(x[i] >> 32);
         }
     }
 }
 
-// Tier 2: rows of 65..4096 entries, one 256-thread block each, bitonic in LDS.
-__global__ __launch_bounds__(256) void sort_rows_block(const u64 *__restrict__ rs, const u32 *__restrict__ rows,
-                                                       const SortLists *L, u32 *__restrict__ col,
-                                                       f32 *__restrict__ cw) {
-    __shared__ u64 keys[4096];
-    const u32 count = L->n2;
+// Rows of the wave tiers, in place, the longest first.
+struct TierCounts {
+    u32 n[kWaveTiers];
+};
+__global__ __launch_bounds__(256) void sort_rows_wave(const u64 *__restrict__ rs, TierLists t, TierCounts k, u32 *col,
+                                                      u32 *w) {
+    const u32 waves = gridDim.x * (blockDim.x / kWave);
+    u32 r = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+    auto tier = [&](auto entries, int q) {
+        for (; r < k.n[q]; r += waves) {
+            const u32 v = t.rows[q][r];
+            const u64 b = rs[v];
+            wave_sort_segment<decltype(entries)::value>(col + b, w + b, col + b, w + b, (u32)(rs[v + 1] - b));
+        }
+        r -= k.n[q];
+    };
+    static_assert(kWaveTiers == 4, "one call per tier");
+    tier(std::integral_constant<int, 8>(), 3);
+    tier(std::integral_constant<int, 4>(), 2);
+    tier(std::integral_constant<int, 2>(), 1);
+    tier(std::integral_constant<int, 1>(), 0);
+}
+
+// Segments that a wave does not sort: a block's bitonic sort in LDS up to
+// kSegBlock entries, a block's radix sort above. They are whole long rows, or
+// bins of rows whose weights are far from evenly spread (many equal ones).
+struct Segment {
+    u64 at;       // in the columns and weights
+    u64 scratch;  // in the scratch pair (radix)
+    u32 len, pad;
+};
+__global__ __launch_bounds__(256) void sort_segments_block(const Segment *__restrict__ segs, const u32 *__restrict__ nsegs,
+                                                           u32 *__restrict__ col, u32 *__restrict__ w) {
+    __shared__ u64 keys[kSegBlock];
+    const u32 count = *nsegs;
     for (u32 r = blockIdx.x; r < count; r += gridDim.x) {
-        const u32 v = rows[r];
-        const u64 b = rs[v];
-        const u32 d = (u32)(rs[v + 1] - b);
+        const u64 b = segs[r].at;
+        const u32 d = segs[r].len;
         u32 P = 128;
         while (P < d) P <<= 1;
-        for (u32 i = threadIdx.x; i < P; i += 256) keys[i] = i < d ? make_key(col[b + i], cw[b + i]) : ~0ull;
+        for (u32 i = threadIdx.x; i < P; i += 256) keys[i] = i < d ? ((u64)w[b + i] << 32) | col[b + i] : ~0ull;
         __syncthreads();
         for (u32 size = 2; size <= P; size <<= 1)
             for (u32 stride = size >> 1; stride > 0; stride >>= 1) {
@@ -481,16 +576,16 @@ __global__ __launch_bounds__(256) void sort_rows_block(const u64 *__restrict__ r
             }
         for (u32 i = threadIdx.x; i < d; i += 256) {
             col[b + i] = (u32)keys[i];
-            cw[b + i] = __uint_as_float((u32)(keys[i] >> 32));
+            w[b + i] = (u32)(keys[i] >> 32);
         }
         __syncthreads();
     }
 }
 
-// Tier 3: rows longer than 4096 entries, one 1024-thread block each, stable
-// LSD radix sort on 8-bit digits ping-ponging between the row (column /
+// Segments longer than kSegBlock entries, one 1024-thread block each, stable
+// LSD radix sort on 8-bit digits ping-ponging between the segment (column /
 // weight-bit arrays) and a scratch pair. Digits cover the column bits, then
-// the 30 significant weight bits.
+// the weight bits.
 constexpr int kRadixBlock = 1024;
 constexpr int kRadixWaves = kRadixBlock / kWave;
 
@@ -498,21 +593,18 @@ __device__ __forceinline__ u32 digit_of(u32 lo, u32 hi, int shift) {
     return shift < 32 ? (lo >> shift) & 0xFF : (hi >> (shift - 32)) & 0xFF;
 }
 
-__global__ __launch_bounds__(kRadixBlock) void sort_rows_radix(
-    const u64 *__restrict__ rs, const u32 *__restrict__ rows, const u64 *__restrict__ row_off,
-    const SortLists *L, u32 *__restrict__ col, u32 *__restrict__ wbits, u32 *__restrict__ s_lo,
-    u32 *__restrict__ s_hi, int col_passes) {
+__global__ __launch_bounds__(kRadixBlock) void sort_segments_radix(
+    const Segment *__restrict__ segs, const u32 *__restrict__ nsegs, u32 *__restrict__ col, u32 *__restrict__ wbits,
+    u32 *__restrict__ s_lo, u32 *__restrict__ s_hi, int col_passes) {
     __shared__ u32 base[256];
     __shared__ u32 wcnt[kRadixWaves][256];
-    const u32 count = L->n3;
     const int lane = lane_id(), wave = threadIdx.x / kWave;
     const int npass = col_passes + 4;
+    const u32 count = *nsegs;
     for (u32 r = blockIdx.x; r < count; r += gridDim.x) {
-        const u32 v = rows[r];
-        const u64 b = rs[v];
-        const u32 d = (u32)(rs[v + 1] - b);
-        u32 *a_lo = col + b, *a_hi = wbits + b;
-        u32 *b_lo = s_lo + row_off[r], *b_hi = s_hi + row_off[r];
+        const u32 d = segs[r].len;
+        u32 *a_lo = col + segs[r].at, *a_hi = wbits + segs[r].at;
+        u32 *b_lo = s_lo + segs[r].scratch, *b_hi = s_hi + segs[r].scratch;
         for (int pass = 0; pass < npass; ++pass) {
             const int shift = pass < col_passes ? 8 * pass : 32 + 8 * (pass - col_passes);
             const u32 *src_lo = (pass & 1) ? b_lo : a_lo, *src_hi = (pass & 1) ? b_hi : a_hi;
@@ -583,6 +675,219 @@ __global__ __launch_bounds__(kRadixBlock) void sort_rows_radix(
             }
         }
         __syncthreads();
+    }
+}
+
+// ----------------------------------------------------------------- long rows
+// Rows above kLongRow entries (three quarters of the entries at S23) are split
+// by weight: row r of d entries has K = ceil(d / kBinEntries) bins, linear in
+// the weight between the row's smallest and largest (a monotone map, so the
+// bins are in order), its entries are scattered by bin into scratch, and a
+// wave sorts each bin into the row. Rows with negative or non-finite weights
+// are one bin. Rows lie in a flattened space padded to kHubChunk entries
+// (hub_append); chunk c of it stands for 256 entries of its row and, for the
+// row's first K chunks, for a bin. Before, rows of 65..4096 entries were
+// sorted by a block's bitonic sort in LDS and longer ones by one block's
+// radix sort each: 20 ms at S23, now 5.3 with the wave tiers.
+constexpr u32 kBinEntries = 384;  // on average; a wave sorts up to 512 (six deviations above it for uniform weights)
+constexpr int kLongBlock = 512, kLongChunks = 4;  // a wave takes 4 chunks, a block a span of 32
+constexpr u64 kLongSpan = (u64)kLongChunks * (kLongBlock / kWave);
+constexpr u32 kLongBins = 8192;  // bins counted in LDS per span
+
+struct LongRows {
+    const u64 *rs;
+    const u32 *row, *len;
+    const u64 *off;
+    u64 nrows, nchunks;
+    u32 *chunk_row;    // [nchunks] slot of the row
+    u32 *wlo, *whi;    // [nrows] smallest and largest weight bits
+    u32 *count;        // [nchunks] entries per bin
+    u64 *bin_off;      // [nchunks + 1] the bin's place in the scratch
+    u32 *used;         // [nchunks] entries placed
+    u32 *col, *w;      // the CSR
+    u32 *s_col, *s_w;  // scratch
+};
+
+__device__ __forceinline__ u32 long_bins(u32 len) { return (len + kBinEntries - 1) / kBinEntries; }
+
+// The slot of every chunk's row; clears the row's weight range.
+__global__ __launch_bounds__(256) void long_chunk_rows(LongRows a) {
+    const u64 wave = ((u64)blockIdx.x * blockDim.x + threadIdx.x) / kWave, nw = (u64)gridDim.x * blockDim.x / kWave;
+    for (u64 r = wave; r < a.nrows; r += nw) {
+        const u64 c0 = a.off[r] / kHubChunk, k = (a.len[r] + kHubChunk - 1) / kHubChunk;
+        for (u64 c = lane_id(); c < k; c += kWave) a.chunk_row[c0 + c] = (u32)r;
+        if (lane_id() == 0) {
+            a.wlo[r] = ~0u;
+            a.whi[r] = 0;
+        }
+    }
+}
+
+// A lane's 4 entries of chunk c (false beyond the row's end).
+struct LongChunk {
+    u64 at[4];
+    bool ok[4];
+};
+__device__ __forceinline__ u32 long_chunk(const LongRows &a, u64 c, LongChunk &k) {
+    const u32 r = a.chunk_row[c];
+    const u32 in_row = (u32)(c * kHubChunk - a.off[r]) + lane_id(), len = a.len[r];
+    const u64 b = a.rs[a.row[r]];
+#pragma unroll
+    for (u32 q = 0; q < 4; ++q) {
+        k.ok[q] = in_row + q * kWave < len;
+        k.at[q] = b + in_row + q * kWave;
+    }
+    return r;
+}
+
+__global__ __launch_bounds__(256) void long_weight_range(LongRows a) {
+    const u64 wave = ((u64)blockIdx.x * blockDim.x + threadIdx.x) / kWave, nw = (u64)gridDim.x * blockDim.x / kWave;
+    for (u64 c = wave; c < a.nchunks; c += nw) {
+        LongChunk k;
+        const u32 r = long_chunk(a, c, k);
+        u32 lo = ~0u, hi = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (k.ok[q]) {
+                const u32 wb = a.w[k.at[q]];
+                lo = min(lo, wb);
+                hi = max(hi, wb);
+            }
+        lo = wave_min(lo);
+        hi = ~wave_min(~hi);
+        if (lane_id() == 0) {  // a plain read may be stale, the wrong way only for skipping nothing
+            if (lo < ld_relaxed(&a.wlo[r])) atomicMin(&a.wlo[r], lo);
+            if (hi > ld_relaxed(&a.whi[r])) atomicMax(&a.whi[r], hi);
+        }
+    }
+}
+
+// Bin of a weight in its row: first bin, bins, and the linear map.
+struct LongMap {
+    u32 first, bins;
+    f32 lo, scale;
+    __device__ __forceinline__ u32 bin(u32 wb) const {
+        return first + min((u32)((__uint_as_float(wb) - lo) * scale), bins - 1);
+    }
+};
+__device__ __forceinline__ LongMap long_map(const LongRows &a, u32 r) {
+    LongMap m;
+    m.first = (u32)(a.off[r] / kHubChunk);
+    m.bins = long_bins(a.len[r]);
+    const u32 lo = a.wlo[r], hi = a.whi[r];
+    m.lo = __uint_as_float(lo);
+    m.scale = (f32)m.bins / (__uint_as_float(hi) - m.lo);
+    if (hi >= 0x7F800000u || !(m.scale < 1e30f)) {  // negative or not finite, or (almost) all equal: one bin
+        m.lo = 0.0f;
+        m.scale = 0.0f;
+        m.bins = 1;
+    }
+    return m;
+}
+
+// Counts (SCATTER false) or places (true) the entries of a span of chunks by
+// bin. The bins of the span's rows are ranked in LDS, one global atomic per
+// bin, unless a span meets rows of more bins than that.
+template <bool SCATTER>
+__global__ __launch_bounds__(kLongBlock) void long_bin_kernel(LongRows a) {
+    __shared__ u32 h[kLongBins];
+    const u32 wave = threadIdx.x / kWave;
+    for (u64 c0 = (u64)blockIdx.x * kLongSpan; c0 < a.nchunks; c0 += (u64)gridDim.x * kLongSpan) {
+        const u64 c1 = min(c0 + kLongSpan, a.nchunks);
+        const u32 r0 = a.chunk_row[c0], r1 = a.chunk_row[c1 - 1];
+        const u32 lo = (u32)(a.off[r0] / kHubChunk), hi = (u32)(a.off[r1] / kHubChunk) + long_bins(a.len[r1]);
+        const bool lds = hi - lo <= kLongBins;
+        if (lds)
+            for (u32 b = threadIdx.x; b < hi - lo; b += kLongBlock) h[b] = 0;
+        __syncthreads();
+        u32 bin[kLongChunks][4], rank[kLongChunks][4], wb[kLongChunks][4], cv[kLongChunks][4];
+        bool ok[kLongChunks][4];
+#pragma unroll
+        for (int g = 0; g < kLongChunks; ++g) {
+            const u64 c = c0 + (u64)wave * kLongChunks + g;
+            LongChunk k;
+            u32 r = 0;
+            if (c < c1) r = long_chunk(a, c, k);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                ok[g][q] = c < c1 && k.ok[q];
+                wb[g][q] = ok[g][q] ? a.w[k.at[q]] : 0;
+                if (SCATTER) cv[g][q] = ok[g][q] ? a.col[k.at[q]] : 0;
+            }
+            if (c < c1) {
+                const LongMap m = long_map(a, r);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) bin[g][q] = ok[g][q] ? m.bin(wb[g][q]) : 0;
+            }
+        }
+        u32 *cnt = SCATTER ? a.used : a.count;
+#pragma unroll
+        for (int g = 0; g < kLongChunks; ++g)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                rank[g][q] = ok[g][q] ? atomicAdd(lds ? &h[bin[g][q] - lo] : &cnt[bin[g][q]], 1u) : 0;
+        __syncthreads();
+        if (lds)
+            for (u32 b = threadIdx.x; b < hi - lo; b += kLongBlock)
+                if (h[b]) h[b] = atomicAdd(&cnt[lo + b], h[b]);
+        __syncthreads();
+        if (SCATTER) {
+#pragma unroll
+            for (int g = 0; g < kLongChunks; ++g)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (ok[g][q]) {
+                        const u64 p = a.bin_off[bin[g][q]] + rank[g][q] + (lds ? h[bin[g][q] - lo] : 0u);
+                        a.s_col[p] = cv[g][q];
+                        a.s_w[p] = wb[g][q];
+                    }
+            __syncthreads();
+        }
+    }
+}
+
+// Sorts every bin into its row; a bin too long for a wave is copied there and
+// listed for the block and radix sorts.
+__global__ __launch_bounds__(256) void long_sort_bins(LongRows a, SortLists *L, Segment *__restrict__ block_segs,
+                                                      Segment *__restrict__ radix_segs) {
+    const u32 lane = lane_id();
+    const u64 wave = ((u64)blockIdx.x * blockDim.x + threadIdx.x) / kWave, nw = (u64)gridDim.x * blockDim.x / kWave;
+    for (u64 c = wave; c < a.nchunks; c += nw) {
+        const u32 len = a.count[c];
+        if (!len) continue;
+        const u32 r = a.chunk_row[c];
+        const u64 from = a.bin_off[c];
+        const u64 to = a.rs[a.row[r]] + (from - a.bin_off[a.off[r] / kHubChunk]);
+        if (len <= 4 * kWave) {
+            wave_sort_segment<4>(a.s_col + from, a.s_w + from, a.col + to, a.w + to, len);
+        } else if (len <= 8 * kWave) {
+            wave_sort_segment<8>(a.s_col + from, a.s_w + from, a.col + to, a.w + to, len);
+        } else {
+            for (u32 i = lane; i < len; i += kWave) {
+                a.col[to + i] = a.s_col[from + i];
+                a.w[to + i] = a.s_w[from + i];
+            }
+            if (lane == 0) {
+                const Segment s = {to, from, len, 0};
+                if (len <= kSegBlock) block_segs[atomicAdd(&L->nblock.v, 1u)] = s;
+                else radix_segs[atomicAdd(&L->nradix.v, 1u)] = s;
+            }
+        }
+    }
+}
+
+// Few long rows, or no room for the scratch of them all: each is a segment of its own
+// (scratch places in list order for those above kSegBlock entries).
+__global__ __launch_bounds__(256) void long_rows_as_segments(LongRows a, SortLists *L, Segment *__restrict__ block_segs,
+                                                             Segment *__restrict__ radix_segs, u64 *scratch_used) {
+    for (u64 r = (u64)blockIdx.x * blockDim.x + threadIdx.x; r < a.nrows; r += (u64)gridDim.x * blockDim.x) {
+        Segment s = {a.rs[a.row[r]], 0, a.len[r], 0};
+        if (s.len <= kSegBlock) {
+            block_segs[atomicAdd(&L->nblock.v, 1u)] = s;
+        } else {
+            s.scratch = atomicAdd((unsigned long long *)scratch_used, (unsigned long long)s.len);
+            radix_segs[atomicAdd(&L->nradix.v, 1u)] = s;
+        }
     }
 }
 
@@ -1171,6 +1476,100 @@ static bool fill_partitioned(Worker_State *ws, const Tuple_Graph *tg, Oned_Graph
     return !failed();
 }
 
+// Fewer entries in long rows than this are sorted as whole rows, in fewer
+// launches. Whole construction, whole rows / bins, us: S10 646 / 690, S14 (2.5e5
+// entries in long rows) 1088 / 928, S15 1359 / 1155, S16 1745 / 1393.
+constexpr u64 kLongMin = 1 << 17;
+
+// Sorts every row by (weight bits, column) and counts the rows with entries.
+static bool sort_rows(Worker_State *ws, Oned_Graph *g) {
+    Context &c = ctx();
+    const hipStream_t s = c.stream;
+    const u64 n = g->nlocalverts, m = g->nlocaledges;
+    const u64 mark = ws->gpu_arena.used;
+    u32 *col = g->column, *w = (u32 *)g->weights;
+    SortLists *L = (SortLists *)arena_alloc(ws, sizeof(SortLists) + 256, "sort lists");
+    TierLists t;
+    for (int q = 0; q < kWaveTiers; ++q)
+        t.rows[q] = (u32 *)arena_alloc(ws, tier_cap(n, m, q ? 32u << q : 17) * sizeof(u32), "sort tier");
+    t.long_cap = tier_cap(n, m, kLongRow + 1);
+    t.long_row = (u32 *)arena_alloc(ws, t.long_cap * sizeof(u32), "long rows");
+    t.long_len = (u32 *)arena_alloc(ws, t.long_cap * sizeof(u32), "long row lengths");
+    t.long_off = (u64 *)arena_alloc(ws, t.long_cap * sizeof(u64), "long row offsets");
+    Segment *block_segs = (Segment *)arena_alloc(ws, tier_cap(m, m, kLongRow + 1) * sizeof(Segment), "block segments");
+    Segment *radix_segs = (Segment *)arena_alloc(ws, tier_cap(m, m, kSegBlock + 1) * sizeof(Segment), "radix segments");
+    if (failed()) return false;
+    u32 *error = (u32 *)(L + 1);
+    G500_HIP(hipMemsetAsync(L, 0, sizeof(SortLists) + 256, s));
+    classify_rows<<<grid_for(n, kClassifyTile, (u64)c.num_cus * 2), 1024, 0, s>>>(g->rowstarts, n, L, t, error);
+    sort_rows_thread<<<grid_for(n, 256, (u64)c.num_cus * 32), 256, 0, s>>>(g->rowstarts, n, col, g->weights);
+    G500_HIP(hipGetLastError());
+    SortLists h;
+    G500_HIP(hipMemcpyAsync(&h, L, sizeof(h), hipMemcpyDeviceToHost, s));
+    sync();
+    if (failed()) return false;
+    g->notisolated = h.notisolated.v;
+    TierCounts k;
+    u64 nwave = 0;
+    for (int q = 0; q < kWaveTiers; ++q) nwave += k.n[q] = h.n[q].v;
+    if (nwave)
+        sort_rows_wave<<<grid_for(nwave * kWave, 256, (u64)c.num_cus * 32), 256, 0, s>>>(g->rowstarts, t, k, col, w);
+    LongRows a = {};
+    a.nrows = hub_count(h.longs.v);
+    a.nchunks = hub_total(h.longs.v) / kHubChunk;
+    if (a.nrows) {
+        a.rs = g->rowstarts;
+        a.row = t.long_row;
+        a.len = t.long_len;
+        a.off = t.long_off;
+        a.col = col;
+        a.w = w;
+        const u64 per_chunk = 3 * sizeof(u32) + sizeof(u64), slack = 16 * 256 + scan_tile_bytes(a.nchunks);
+        const u64 room = ws->gpu_arena.reserved - ws->gpu_arena.used;
+        const bool bins = h.long_entries.v >= kLongMin && h.long_entries.v * 8 + a.nchunks * per_chunk + a.nrows * 8 + slack <= room;
+        const u64 scratch = MAX(bins ? h.long_entries.v : h.huge_entries.v, (u64)1);
+        a.s_col = (u32 *)arena_alloc(ws, scratch * sizeof(u32), "sort scratch");
+        a.s_w = (u32 *)arena_alloc(ws, scratch * sizeof(u32), "sort scratch");
+        if (failed()) return false;
+        if (bins) {
+            a.chunk_row = (u32 *)arena_alloc(ws, a.nchunks * sizeof(u32), "long row chunks");
+            a.count = (u32 *)arena_alloc(ws, a.nchunks * sizeof(u32), "long row bin counts");
+            a.used = (u32 *)arena_alloc(ws, a.nchunks * sizeof(u32), "long row bins filled");
+            a.bin_off = (u64 *)arena_alloc(ws, (a.nchunks + 1) * sizeof(u64), "long row bin offsets");
+            a.wlo = (u32 *)arena_alloc(ws, a.nrows * sizeof(u32), "long row weights");
+            a.whi = (u32 *)arena_alloc(ws, a.nrows * sizeof(u32), "long row weights");
+            u64 *tiles = (u64 *)arena_alloc(ws, scan_tile_bytes(a.nchunks), "long row scan tiles");
+            if (failed()) return false;
+            const unsigned waves = grid_for(a.nchunks * kWave, 256, (u64)c.num_cus * 32);
+            const unsigned spans = grid_for(a.nchunks, (int)kLongSpan, (u64)c.num_cus * 8);
+            long_chunk_rows<<<grid_for(a.nrows * kWave, 256, (u64)c.num_cus * 16), 256, 0, s>>>(a);
+            G500_HIP(hipMemsetAsync(a.count, 0, a.nchunks * sizeof(u32), s));
+            G500_HIP(hipMemsetAsync(a.used, 0, a.nchunks * sizeof(u32), s));
+            long_weight_range<<<waves, 256, 0, s>>>(a);
+            long_bin_kernel<false><<<spans, kLongBlock, 0, s>>>(a);
+            scan_counts(a.count, a.nchunks, tiles, a.bin_off, s);
+            long_bin_kernel<true><<<spans, kLongBlock, 0, s>>>(a);
+            long_sort_bins<<<waves, 256, 0, s>>>(a, L, block_segs, radix_segs);
+        } else {
+            long_rows_as_segments<<<grid_for(a.nrows, 256, 1024), 256, 0, s>>>(a, L, block_segs, radix_segs,
+                                                                              (u64 *)(error + 2));
+        }
+        G500_HIP(hipGetLastError());
+        // the kernels read how many segments there are: waiting for the counts would cost more than an empty launch
+        sort_segments_block<<<(unsigned)MIN(a.nrows, (u64)c.num_cus * 16), 256, 0, s>>>(block_segs, &L->nblock.v, col,
+                                                                                        w);
+        if (bins || h.huge_entries.v) {
+            int bits = 1;
+            while (bits < 32 && (1ull << bits) < n) ++bits;
+            sort_segments_radix<<<(unsigned)MIN(a.nrows, (u64)c.num_cus * 2), kRadixBlock, 0, s>>>(
+                radix_segs, &L->nradix.v, col, w, a.s_col, a.s_w, (bits + 7) / 8);
+        }
+    }
+    G500_HIP(hipGetLastError());
+    ws->gpu_arena.used = mark;  // release the scratch
+    return !failed();
+}
+
 }  // namespace g500
 
 using namespace g500;
@@ -1191,43 +1590,9 @@ Oned_Graph oned_graph_from_tuple_graph(Worker_State *ws, Tuple_Graph *tg, u64 ng
     const u64 ne = tg->edges_size;
     g.rowstarts = (u64 *)arena_alloc(ws, (n + 1) * sizeof(u64), "CSR row offsets");
     if (failed()) return g;
-    const hipStream_t s = c.stream;
     timer_start();
     if (!(partition_pays(ws, n, ne) ? fill_partitioned(ws, tg, &g) : fill_direct(ws, tg, &g))) return g;
-    const u64 mark_sort = ws->gpu_arena.used;
-    SortLists *L = (SortLists *)arena_alloc(ws, sizeof(SortLists), "sort lists");
-    u32 *t1 = (u32 *)arena_alloc(ws, n * sizeof(u32), "sort tier 1");
-    u32 *t2 = (u32 *)arena_alloc(ws, n * sizeof(u32), "sort tier 2");
-    u32 *t3 = (u32 *)arena_alloc(ws, n * sizeof(u32), "sort tier 3");
-    u64 *t3_off = (u64 *)arena_alloc(ws, n * sizeof(u64), "sort tier 3 offsets");
-    if (failed()) return g;
-    G500_HIP(hipMemsetAsync(L, 0, sizeof(SortLists), s));
-    classify_rows<<<grid_for(n, 256, (u64)c.num_cus * 16), 256, 0, s>>>(g.rowstarts, n, L, t1, t2, t3, t3_off);
-    sort_rows_thread<<<grid_for(n, 256, (u64)c.num_cus * 32), 256, 0, s>>>(g.rowstarts, n, g.column, g.weights);
-    G500_HIP(hipGetLastError());
-    SortLists hl;
-    G500_HIP(hipMemcpyAsync(&hl, L, sizeof(hl), hipMemcpyDeviceToHost, s));
-    sync();
-    if (failed()) return g;
-    g.notisolated = hl.notisolated;
-    if (hl.n1)
-        sort_rows_wave<<<grid_for((u64)hl.n1 * kWave, 256, (u64)c.num_cus * 32), 256, 0, s>>>(
-            g.rowstarts, t1, L, g.column, g.weights);
-    if (hl.n2)
-        sort_rows_block<<<(unsigned)MIN((u64)hl.n2, (u64)c.num_cus * 16), 256, 0, s>>>(g.rowstarts, t2, L,
-                                                                                       g.column, g.weights);
-    if (hl.n3) {
-        u32 *s_lo = (u32 *)arena_alloc(ws, hl.scratch_total * sizeof(u32), "radix scratch");
-        u32 *s_hi = (u32 *)arena_alloc(ws, hl.scratch_total * sizeof(u32), "radix scratch");
-        if (failed()) return g;
-        int bits = 1;
-        while (bits < 32 && (1ull << bits) < n) ++bits;
-        const int col_passes = (bits + 7) / 8;
-        sort_rows_radix<<<(unsigned)MIN((u64)hl.n3, (u64)c.num_cus * 2), kRadixBlock, 0, s>>>(
-            g.rowstarts, t3, t3_off, L, g.column, (u32 *)g.weights, s_lo, s_hi, col_passes);
-    }
-    G500_HIP(hipGetLastError());
-    ws->gpu_arena.used = mark_sort;  // release the scratch
+    if (!sort_rows(ws, &g)) return g;
     if (c.relabel) build_traversal_copy(ws, &g);
     timer_stop();
     return g;

@@ -139,3 +139,31 @@ def test_csr_partition_rejects_endpoints_out_of_range(arena, ne):
     tg = arena.upload_tuples(e, np.ones(ne, np.float32))
     with pytest.raises(g500.LibraryError, match="outside"):
         arena.csr(tg, 5000)
+
+
+# rows at the edges of the sort's tiers, with evenly spread weights and with
+# weights that put many entries, or all, into one bin; with `bulk`, a long row
+# more, enough that long rows are sorted in bins
+@pytest.mark.parametrize("weights", ["uniform", "equal", "two", "wide", "negative", "infinite"])
+@pytest.mark.parametrize("bulk", [0, 150000])
+def test_csr_row_sort_tiers(arena, oracle, weights, bulk):
+    rng = np.random.default_rng(5)
+    lengths = [2, 15, 16, 17, 63, 64, 65, 127, 128, 129, 255, 256, 257, 384, 511, 512, 513, 768, 769, 1025, 4095, 4096,
+               4097, 9000] + ([bulk] if bulk else [])
+    n = 30000
+    e = np.concatenate([np.stack([np.full(d, i), rng.integers(len(lengths), n, d)], 1)
+                        for i, d in enumerate(lengths)])
+    e = e[rng.permutation(len(e))]
+    w = rng.random(len(e)).astype(np.float32)
+    if weights == "equal":
+        w[:] = 0.25
+    elif weights == "two":
+        w = np.where(w < 0.5, np.float32(0.1), np.float32(0.9))
+    elif weights == "wide":
+        w = np.exp(60 * w - 40).astype(np.float32)
+    elif weights == "negative":
+        w -= np.float32(0.5)
+    elif weights == "infinite":
+        w[::97] = np.inf
+    g, ref = build(arena, n, e, w)
+    csr_equal(arena, g, ref)
