@@ -167,3 +167,29 @@ def test_csr_row_sort_tiers(arena, oracle, weights, bulk):
         w[::97] = np.inf
     g, ref = build(arena, n, e, w)
     csr_equal(arena, g, ref)
+
+
+# the SSSP copy: weights on and next to the steps of the 8-bit hub table, above
+# its range and infinite, rows on both sides of a wave, and a graph with few
+# entries per vertex in an arena without room for that table
+@pytest.mark.parametrize("n,ne,tight", [(40, 300, False), (2000, 30000, False), (9000, 200000, False),
+                                        (1 << 20, 3000, True)])
+def test_sssp_copy_of_step_weights(arena, oracle, n, ne, tight):
+    from test_gpu_pipeline import check_sssp_copy
+    rng = np.random.default_rng(ne)
+    e = np.minimum(rng.integers(0, n, (ne, 2)), rng.integers(0, n, (ne, 2)) * rng.integers(0, 2, (ne, 2)))
+    step = (rng.integers(0, 300, ne) / 127).astype(np.float32)
+    w = (step + rng.choice([0.0, 2.0**-10, 2.0**-20, -2.0**-20], ne)).astype(np.float32)
+    w = np.where(rng.random(ne) < 0.5, w / 8, w).astype(np.float32)
+    w = np.maximum(w, np.float32(0))
+    w[::501] = np.inf
+    tg = arena.upload_tuples(e, w)
+    a, m = arena.ws.gpu_arena, 2 * ne
+    saved = a.reserved
+    if tight:
+        a.reserved = a.used + 176 * n + 24 * m + (9 << 20)
+    try:
+        g = arena.csr(tg, n)
+    finally:
+        a.reserved = saved
+    check_sssp_copy(arena, g)
