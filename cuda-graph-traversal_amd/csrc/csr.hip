@@ -550,7 +550,8 @@ struct Segment {
     u64 scratch;  // in the scratch pair (radix)
     u32 len, pad;
 };
-__global__ __launch_bounds__(256) void sort_segments_block(const Segment *__restrict__ segs, const u32 *__restrict__ nsegs,
+constexpr u32 kSegThreads = 1024;
+__global__ __launch_bounds__(kSegThreads) void sort_segments_block(const Segment *__restrict__ segs, const u32 *__restrict__ nsegs,
                                                            u32 *__restrict__ col, u32 *__restrict__ w) {
     __shared__ u64 keys[kSegBlock];
     const u32 count = *nsegs;
@@ -559,11 +560,11 @@ __global__ __launch_bounds__(256) void sort_segments_block(const Segment *__rest
         const u32 d = segs[r].len;
         u32 P = 128;
         while (P < d) P <<= 1;
-        for (u32 i = threadIdx.x; i < P; i += 256) keys[i] = i < d ? ((u64)w[b + i] << 32) | col[b + i] : ~0ull;
+        for (u32 i = threadIdx.x; i < P; i += kSegThreads) keys[i] = i < d ? ((u64)w[b + i] << 32) | col[b + i] : ~0ull;
         __syncthreads();
         for (u32 size = 2; size <= P; size <<= 1)
             for (u32 stride = size >> 1; stride > 0; stride >>= 1) {
-                for (u32 t = threadIdx.x; t < P / 2; t += 256) {
+                for (u32 t = threadIdx.x; t < P / 2; t += kSegThreads) {
                     const u32 i = 2 * stride * (t / stride) + (t % stride), j = i + stride;
                     const bool up = (i & size) == 0;
                     const u64 a = keys[i], c = keys[j];
@@ -574,7 +575,7 @@ __global__ __launch_bounds__(256) void sort_segments_block(const Segment *__rest
                 }
                 __syncthreads();
             }
-        for (u32 i = threadIdx.x; i < d; i += 256) {
+        for (u32 i = threadIdx.x; i < d; i += kSegThreads) {
             col[b + i] = (u32)keys[i];
             w[b + i] = (u32)(keys[i] >> 32);
         }
@@ -966,35 +967,119 @@ __global__ __launch_bounds__(kRelabelBlock) void relabel_scatter(const u64 *__re
     }
 }
 
-// Rows of the traversal copy: a lane per row up to kWave entries, a block per
-// longer row (they come first: rows are in decreasing degree order).
-__global__ __launch_bounds__(256) void relabel_rows_lane(const u64 *__restrict__ rs, const u32 *__restrict__ col,
-                                                         const f32 *__restrict__ w, const u32 *__restrict__ perm,
-                                                         const u32 *__restrict__ iperm, const u64 *__restrict__ rs_t,
-                                                         u64 first, u64 n, u32 *__restrict__ col_t,
-                                                         f32 *__restrict__ w_t) {
-    for (u64 p = first + (u64)blockIdx.x * blockDim.x + threadIdx.x; p < n; p += (u64)gridDim.x * blockDim.x) {
-        const u32 v = iperm[p];
-        const u64 b = rs[v], e = rs[v + 1], o = rs_t[p];
-        for (u64 k = b; k < e; ++k) {
-            col_t[o + (k - b)] = perm[col[k]];
-            w_t[o + (k - b)] = w[k];
+// Largest row p of [0, n) with rs[p] <= k (rows before it may be empty).
+__device__ __forceinline__ u64 row_at(const u64 *rs, u64 n, u64 k) {
+    u64 lo = 0, hi = n;
+    while (hi - lo > 1) {
+        const u64 mid = lo + (hi - lo) / 2;
+        if (rs[mid] <= k) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Rows of the traversal copy. Bound by the gather of the columns' new ids
+// (4 random bytes an entry); what remains is to keep many of them in flight:
+// a lane per short row and a block per longer one took 7.5 ms at S23, this 4.2.
+struct RelabelArgs {
+    const u64 *rs;
+    const u32 *col;
+    const f32 *w;
+    const u32 *perm, *iperm;
+    const u64 *rs_t;
+    u32 *col_t;
+    f32 *w_t;
+    u64 nlong, n;
+    u64 span;  // entries of a wave's piece of the long rows
+    u32 per;   // short rows per wave
+};
+
+// Rows longer than a wave, [0, nlong): spans of the copy's entries, a wave
+// walks the row pieces of its span.
+constexpr int kRelabelSteps = 8;
+__global__ __launch_bounds__(256) void relabel_rows_long(RelabelArgs a) {
+    const u32 lane = lane_id();
+    const u64 wave = ((u64)blockIdx.x * blockDim.x + threadIdx.x) / kWave, nw = (u64)gridDim.x * blockDim.x / kWave;
+    const u64 total = a.rs_t[a.nlong];
+    for (u64 s0 = wave * a.span; s0 < total; s0 += nw * a.span) {
+        const u64 s1 = min(s0 + a.span, total);
+        u64 p = row_at(a.rs_t, a.nlong, s0);
+        for (u64 k = s0; k < s1; ++p) {
+            const u64 e = min(a.rs_t[p + 1], s1);
+            const u64 from = a.rs[a.iperm[p]] - a.rs_t[p];  // source position - copy's position
+            for (; k < e; k += kRelabelSteps * kWave) {
+                u32 c[kRelabelSteps];
+                f32 wk[kRelabelSteps];
+#pragma unroll
+                for (int q = 0; q < kRelabelSteps; ++q) {
+                    const u64 i = k + (u64)q * kWave + lane;
+                    c[q] = i < e ? a.col[from + i] : 0;
+                    wk[q] = i < e ? a.w[from + i] : 0.0f;
+                }
+#pragma unroll
+                for (int q = 0; q < kRelabelSteps; ++q) c[q] = a.perm[c[q]];
+#pragma unroll
+                for (int q = 0; q < kRelabelSteps; ++q) {
+                    const u64 i = k + (u64)q * kWave + lane;
+                    if (i < e) {
+                        a.col_t[i] = c[q];
+                        a.w_t[i] = wk[q];
+                    }
+                }
+            }
+            k = e;
         }
     }
 }
 
-__global__ __launch_bounds__(256) void relabel_rows_block(const u64 *__restrict__ rs, const u32 *__restrict__ col,
-                                                          const f32 *__restrict__ w, const u32 *__restrict__ perm,
-                                                          const u32 *__restrict__ iperm, const u64 *__restrict__ rs_t,
-                                                          u64 count, u32 *__restrict__ col_t, f32 *__restrict__ w_t) {
-    for (u64 p = blockIdx.x; p < count; p += gridDim.x) {
-        const u32 v = iperm[p];
-        const u64 b = rs[v], e = rs[v + 1], o = rs_t[p];
-        for (u64 k = b + threadIdx.x; k < e; k += blockDim.x) {
-            col_t[o + (k - b)] = perm[col[k]];
-            w_t[o + (k - b)] = w[k];
+// The other rows: a wave takes `per` of them and gives each G lanes, the power
+// of two that holds the longest (neighbours have the same length in this order).
+__global__ __launch_bounds__(256) void relabel_rows_short(RelabelArgs a) {
+    const u32 lane = lane_id();
+    const u64 wave = ((u64)blockIdx.x * blockDim.x + threadIdx.x) / kWave, nw = (u64)gridDim.x * blockDim.x / kWave;
+    for (u64 p0 = a.nlong + wave * a.per; p0 < a.n; p0 += nw * a.per) {
+        const bool mine = lane < a.per && p0 + lane < a.n;
+        const u64 to = mine ? a.rs_t[p0 + lane] : 0;
+        const u32 len = mine ? (u32)(a.rs_t[p0 + lane + 1] - to) : 0;
+        const u64 from = len ? a.rs[a.iperm[p0 + lane]] : 0;
+        const u32 longest = ~wave_min(~len);
+        if (!longest) continue;
+        u32 G = 1;
+        while (G < longest) G <<= 1;
+        const u32 step = kWave / G, k = lane & (G - 1);
+        for (u32 r = 0; r < a.per; r += 4 * step) {  // four groups of rows in flight
+            u32 c[4];
+            f32 wk[4];
+            u64 o[4];
+            bool in[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const u32 j = r + (u32)q * step + lane / G, js = j & (kWave - 1);
+                const u32 lj = __shfl(len, (int)js);
+                const u64 f = shfl64(from, (int)js);
+                o[q] = shfl64(to, (int)js) + k;
+                in[q] = j < (u32)kWave && k < lj;
+                c[q] = in[q] ? a.col[f + k] : 0;
+                wk[q] = in[q] ? a.w[f + k] : 0.0f;
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) c[q] = a.perm[c[q]];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (in[q]) {
+                    a.col_t[o[q]] = c[q];
+                    a.w_t[o[q]] = wk[q];
+                }
         }
     }
+}
+
+// Units of a kernel's work that one wave takes at a time: `most`, halved down
+// to `least` while that leaves waves of the chip without any.
+static u64 wave_share(u64 units, u64 least, u64 most) {
+    u64 share = most;
+    while (share > least && units / share < (u64)ctx().num_cus * 32) share /= 2;
+    return share;
 }
 
 // ---------------------------------------------------------------- SSSP copy
@@ -1157,17 +1242,6 @@ __device__ __forceinline__ void put_bits(u64 *bits, u64 k, u64 mask) {
     if (s && mask >> (64 - s)) atomicOr((unsigned long long *)&bits[(k >> 6) + 1], (unsigned long long)(mask >> (64 - s)));
 }
 
-// Largest row p of [0, n) with rs[p] <= k (rows before it may be empty).
-__device__ __forceinline__ u64 row_at(const u64 *rs, u64 n, u64 k) {
-    u64 lo = 0, hi = n;
-    while (hi - lo > 1) {
-        const u64 mid = lo + (hi - lo) / 2;
-        if (rs[mid] <= k) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
-
 // Rows longer than a wave, [0, nlong): the entries in spans over the grid, a
 // wave walks the row pieces of its span, so that a row's own table row is
 // read once per piece and the longest rows spread over the chip.
@@ -1292,14 +1366,6 @@ __global__ __launch_bounds__(256) void prune_compact(const u32 *__restrict__ col
                 w_s[at] = wk[i];
             }
     }
-}
-
-// Units of a kernel's work that one wave takes at a time: `most`, halved down
-// to `least` while that leaves waves of the chip without any.
-static u64 wave_share(u64 units, u64 least, u64 most) {
-    u64 share = most;
-    while (share > least && units / share < (u64)ctx().num_cus * 32) share /= 2;
-    return share;
 }
 
 // Exclusive scan of counts[0, n) into offsets[0, n], the total last.
@@ -1449,13 +1515,12 @@ void build_traversal_copy(Worker_State *ws, Oned_Graph *g) {
     sync();
     u64 nlong = 0;
     for (u32 k = 0; k < kDegKeys - 1 - (u32)kWave; ++k) nlong += hc[k];
+    const RelabelArgs a = {g->rowstarts, g->column, g->weights, g->perm, g->iperm, g->rowstarts_t, g->column_t,
+                           g->weights_t, nlong, n, wave_share(m, 512, 4096), (u32)wave_share(n - nlong, 1, kWave)};
     if (nlong)
-        relabel_rows_block<<<(unsigned)MIN(nlong, (u64)c.num_cus * 8), 256, 0, s>>>(
-            g->rowstarts, g->column, g->weights, g->perm, g->iperm, g->rowstarts_t, nlong, g->column_t,
-            g->weights_t);
-    relabel_rows_lane<<<grid_for(n - nlong, 256, (u64)c.num_cus * 32), 256, 0, s>>>(
-        g->rowstarts, g->column, g->weights, g->perm, g->iperm, g->rowstarts_t, nlong, n, g->column_t,
-        g->weights_t);
+        relabel_rows_long<<<grid_for(m / a.span * kWave + kWave, 256, (u64)c.num_cus * 16), 256, 0, s>>>(a);
+    if (nlong < n)
+        relabel_rows_short<<<grid_for((n - nlong) / a.per * kWave + kWave, 256, (u64)c.num_cus * 16), 256, 0, s>>>(a);
     G500_HIP(hipGetLastError());
     sync();
     ws->gpu_arena.used = mark;
@@ -1706,7 +1771,7 @@ static bool sort_rows(Worker_State *ws, Oned_Graph *g) {
         }
         G500_HIP(hipGetLastError());
         // the kernels read how many segments there are: waiting for the counts would cost more than an empty launch
-        sort_segments_block<<<(unsigned)MIN(a.nrows, (u64)c.num_cus * 16), 256, 0, s>>>(block_segs, &L->nblock.v, col,
+        sort_segments_block<<<(unsigned)MIN(a.nrows, (u64)c.num_cus * 4), kSegThreads, 0, s>>>(block_segs, &L->nblock.v, col,
                                                                                         w);
         if (bins || h.huge_entries.v) {
             int bits = 1;
