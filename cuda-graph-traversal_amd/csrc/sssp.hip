@@ -23,7 +23,8 @@
 // fl(d_u + w) >= fl(lo + delta) = hi: heavy relaxations never land back in
 // the current bucket. Per bucket:
 //   light steps: queued vertices relax their light edges; vertices lowered
-//     below hi are queued for the next step (de-duplicated per queue);
+//     below hi are queued for the next step (de-duplicated per queue), or, in
+//     short queues, relaxed at once by the wave that lowered them;
 //   one fused dense step: every vertex of the bucket relaxes its heavy edges
 //     (short rows inline, longer rows through a wave list and a hub list in a
 //     second phase), and every vertex already in the next bucket
@@ -354,6 +355,39 @@ __device__ __forceinline__ void walk_segments(const SsspArgs &a, const Target &t
     }
 }
 
+// Relaxes the light entries of the vertices that this wave has staged for the
+// next step and not spilled, up to kLocalRounds times, instead of leaving them
+// to that step: in the tails of the buckets most queues hold a few vertices,
+// and a step there is a barrier, its counters and a chain of loads. Any order
+// of relaxations reaches the same distances. A staged vertex is popped by
+// clearing its stamp before its distance is read, so that whoever lowers it
+// after the read finds the stamp clear and queues it again.
+// Callers do so when the step's queue is shrinking and holds no more vertices
+// than the grid has waves (a fused step: when its bucket had no more); a
+// growing queue belongs on all waves. us at delta 0.05, without / with (light
+// steps): S10 462 (15) / 408 (8), S14 769 (28) / 669 (12), S18 1562 (52) / 1295 (19),
+// S20 2402 (62) / 1928 (25), S22 3769 (64) / 3253 (26), S24 8668 (66) / 8295 (32);
+// without the conditions S12 568 / 593, S14 771 / 836.
+constexpr int kLocalRounds = 8;
+__device__ __forceinline__ void local_rounds(const SsspArgs &a, const Target &t, u64 &improved, volatile int *slot,
+                                             Stage &sq) {
+    for (int round = 0; round < kLocalRounds && sq.n[0]; ++round) {
+        const u32 n = sq.n[0];
+        const bool mine = lane_id() < n;
+        const u32 u = mine ? ((volatile u32 *)sq.L->v[sq.w][0])[lane_id()] : 0;
+        sq.n[0] = 0;
+        u64 b = 0, e = 0;
+        u32 was = 0;
+        if (mine) {
+            was = atomicExch(&a.stamp[u], 0u);
+            segment<true>(a, u, b, e);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(was)::"memory");
+        const f32 du = mine ? __uint_as_float(ld_relaxed(&a.dl[u])) : 0.f;
+        walk_segments(a, t, u, du, b, (u32)(e - b), improved, slot, sq);
+    }
+}
+
 // Vertices list[0, count) of work tier 0 (64 vertices per wave, segments
 // walked together) or 1 (a wave each).
 template <bool LIGHT>
@@ -609,6 +643,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void s
     SsspCtl *ctl = a.ctl;
     grid_join(&ctl->bar);
     const u64 gtid = (u64)blockIdx.x * blockDim.x + threadIdx.x, gthreads = (u64)gridDim.x * blockDim.x;
+    const u64 nwaves = gthreads / kWave;
     const u32 lane = lane_id();
     __shared__ int slots[1024 / kWave][kWave];
     volatile int *slot = slots[threadIdx.x / kWave];
@@ -624,6 +659,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void s
         sq.slot = t.slot;
     };
     u64 improved = 0;
+    u64 prev_total = 0;              // light-queue items of the step before (the same in every thread)
     u64 bucket_items = 0;            // light-queue items of the current bucket (the same in every thread)
     u64 settled_total = 0;           // vertices settled so far (the same in every thread)
     u32 x = 0;                       // step
@@ -711,6 +747,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void s
             for (int tier = 0; tier < 2; ++tier)
                 process_tier<true>(a, a.fq[x & 1][tier], cnt[tier], tier, t, improved, slot, sq);
             process_hubs<true>(a, a.fq[x & 1][2], a.fq_off[x & 1], a.fq_len[x & 1], hub, t, improved, sq);
+            if (total < prev_total && total <= nwaves) local_rounds(a, t, improved, slot, sq);
+            prev_total = total;
             stage_flush(a, sq);
             sync_traced(ctl, kPhaseLight, __float_as_uint(lo), x);
             tick(0);
@@ -764,6 +802,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void s
                            &ctl->bar.error);
                 walk_segments(a, t, (u32)v, dv, b, mine && len <= kSmall ? len : 0, improved, slot, sq);
             });
+            if (bucket_items <= nwaves) local_rounds(a, t, improved, slot, sq);
             stage_flush(a, sq);
             {  // the block sums its waves' settled counts and makes one atomic (every thread is here)
                 __shared__ u64 bset;
@@ -780,6 +819,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void s
             if (nmed || hub_count(hh)) {  // second phase of the same step: longer heavy rows
                 process_tier<false>(a, a.hq1, min(nmed, (u32)a.n), 1, t, improved, slot, sq);
                 process_hubs<false>(a, a.hqh, a.hq_off, a.hq_len, hh, t, improved, sq);
+                if (bucket_items <= nwaves) local_rounds(a, t, improved, slot, sq);
                 stage_flush(a, sq);
                 sync_traced(ctl, kPhaseHeavy, __float_as_uint(lo), x);
             }
