@@ -43,32 +43,79 @@ __global__ __launch_bounds__(256) void validate_init_kernel(const i64 *__restric
 
 __device__ __forceinline__ i64 wrap_inc(i64 x) { return (i64)((u64)x + 1u); }
 
-// Rules 3-6 over every CSR entry, one wave per source row
-// (graph500_runner.cu:111-153).
+// Rules 3-6 over every CSR entry (graph500_runner.cu:111-153). A wave takes
+// `per` source rows; 8 lanes walk each row of up to kValidateLong entries,
+// eight rows at a time, and the whole wave each longer one, with kValidateSteps
+// entries of a lane in flight: their depths are random reads, which bound it.
+// The reference also confirms d from an entry (s, d) with pred[d] == s; the
+// rows are symmetric, so d's own row holds s and confirms it there, and the
+// entries' parents need no reads. 700001 uniform vertices, 15.4e6 entries:
+// 385 us with one row per wave, one entry per lane and both reads, now 121.
+constexpr u32 kValidateLong = 128;
+constexpr int kValidateSteps = 4;
 __global__ __launch_bounds__(256) void validate_edges_kernel(const u64 *__restrict__ rs, const u32 *__restrict__ col,
                                                              const i64 *__restrict__ pred, const i64 *__restrict__ dist,
-                                                             u32 *__restrict__ confirmed, u64 *__restrict__ errors, u64 n) {
+                                                             u32 *__restrict__ confirmed, u64 *__restrict__ errors, u64 n,
+                                                             u32 per) {
     const u32 lane = lane_id();
     const u64 wave = ((u64)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
     const u64 nw = (u64)gridDim.x * blockDim.x / kWave;
     u64 err = 0;
-    for (u64 s = wave; s < n; s += nw) {
-        const i64 sp = pred[s], sd = dist[s];
-        const u64 b = rs[s], e = rs[s + 1];
+    // entries k, k + stride, ... of source s (this lane's share of a row of len entries from b)
+    auto walk = [&](u64 s, i64 sp, i64 sd, u64 b, u32 len, u32 first, u32 stride) {
         bool self_ok = false;
-        for (u64 k = b + lane; k < e; k += kWave) {
-            const u64 d = col[k];
-            if (d == s) {
-                ++err;
-                continue;
+        for (u32 k = first; k < len; k += kValidateSteps * stride) {
+            u64 d[kValidateSteps];
+            i64 dd[kValidateSteps];
+            bool in[kValidateSteps];
+#pragma unroll
+            for (int q = 0; q < kValidateSteps; ++q) {
+                in[q] = k + (u32)q * stride < len;
+                d[q] = in[q] ? col[b + k + (u32)q * stride] : s;
             }
-            const i64 dp = pred[d], dd = dist[d];
-            if ((sd == -1 && dd != -1) || (sd != -1 && dd == -1)) ++err;
-            if (sd >= 0 && dd >= 0 && (wrap_inc(sd) < dd || wrap_inc(dd) < sd)) ++err;
-            if (sp == (i64)d) self_ok = true;
-            if (dp == (i64)s) confirm(confirmed, d);
+#pragma unroll
+            for (int q = 0; q < kValidateSteps; ++q) dd[q] = dist[d[q]];
+#pragma unroll
+            for (int q = 0; q < kValidateSteps; ++q) {
+                if (!in[q]) continue;
+                if (d[q] == s) {
+                    ++err;
+                    continue;
+                }
+                if ((sd == -1 && dd[q] != -1) || (sd != -1 && dd[q] == -1)) ++err;
+                if (sd >= 0 && dd[q] >= 0 && (wrap_inc(sd) < dd[q] || wrap_inc(dd[q]) < sd)) ++err;
+                if (sp == (i64)d[q]) self_ok = true;
+            }
         }
-        if (ballot(self_ok) && lane == 0) confirm(confirmed, s);
+        return self_ok;
+    };
+    for (u64 s0 = wave * per; s0 < n; s0 += nw * per) {
+        const u64 s = s0 + lane;
+        const bool mine = lane < per && s < n;
+        const i64 sp = mine ? pred[s] : -1, sd = mine ? dist[s] : -1;
+        const u64 b = mine ? rs[s] : 0;
+        const u32 len = mine ? (u32)(rs[s + 1] - b) : 0;
+        for (u64 todo = ballot(len > 0 && len <= kValidateLong); todo;) {
+            int j = -1;
+#pragma unroll
+            for (u32 q = 0; q < 8; ++q) {
+                const int jq = todo ? __ffsll((unsigned long long)todo) - 1 : -1;
+                todo &= todo - 1;
+                if (lane >> 3 == q) j = jq;
+            }
+            const int js = j < 0 ? 0 : j;
+            const u32 lj = __shfl(len, js);
+            const bool ok = walk(s0 + js, (i64)shfl64((u64)sp, js), (i64)shfl64((u64)sd, js), shfl64(b, js),
+                                 j < 0 ? 0 : lj, lane & 7u, 8);
+            const u32 any = (u32)(ballot(ok) >> (lane & ~7u)) & 0xFFu;
+            if (any && (lane & 7u) == 0) confirm(confirmed, s0 + js);
+        }
+        for (u64 todo = ballot(len > kValidateLong); todo; todo &= todo - 1) {
+            const int j = __ffsll((unsigned long long)todo) - 1;
+            const bool ok = walk(s0 + j, (i64)shfl64((u64)sp, j), (i64)shfl64((u64)sd, j), shfl64(b, j), __shfl(len, j),
+                                 lane, kWave);
+            if (ballot(ok) && lane == 0) confirm(confirmed, s0 + j);
+        }
     }
     err = wave_sum(err);
     if (lane == 0 && err) atomicAdd((unsigned long long *)errors, (unsigned long long)err);
@@ -225,10 +272,13 @@ static u64 validate_enqueue(const Oned_Graph *g, const i64 *pred, const i64 *dis
     Context &c = ctx();
     const u64 n = g->nlocalverts, nwords = (n + 31) / 32;
     const hipStream_t s = c.stream;
-    const unsigned gv = grid_for(n, 256, (u64)c.num_cus * 32), ge = grid_for(n * kWave, 256, (u64)c.num_cus * 32);
+    const unsigned gv = grid_for(n, 256, (u64)c.num_cus * 32);
+    u32 per = kWave;  // source rows per wave, fewer on graphs that would leave waves idle
+    while (per > 1 && n / per < (u64)c.num_cus * 32) per /= 2;
+    const unsigned ge = grid_for((n + per - 1) / per * kWave, 256, (u64)c.num_cus * 32);
     validate_clear_kernel<<<grid_for(nwords, 256, (u64)c.num_cus * 8), 256, 0, s>>>(confirmed, nwords, errors);
     validate_init_kernel<<<gv, 256, 0, s>>>(pred, dist, confirmed, errors, n, root);
-    validate_edges_kernel<<<ge, 256, 0, s>>>(g->rowstarts, g->column, pred, dist, confirmed, errors, n);
+    validate_edges_kernel<<<ge, 256, 0, s>>>(g->rowstarts, g->column, pred, dist, confirmed, errors, n, per);
     validate_confirmed_kernel<<<gv, 256, 0, s>>>(pred, dist, confirmed, errors, n, root);
     G500_HIP(hipGetLastError());
     u64 h = 0;
