@@ -112,7 +112,7 @@ __device__ __forceinline__ void append_record(const BatchArgs &a, bool want, u32
 // Folds per-lane edge counts and masks into the slot's counters.
 __device__ __forceinline__ void flush_level(const BatchArgs &a, int slot, u64 edges, u64 alive) {
     edges = wave_sum(edges);
-    for (int o = 32; o > 0; o >>= 1) alive |= shfl_xor64(alive, o);
+    alive = wave_or(alive);
     if (lane_id() == 0) {
         if (edges) atomicAdd((unsigned long long *)&a.ctl->fedges[slot], (unsigned long long)edges);
         if (alive) atomicOr((unsigned long long *)&a.ctl->alive[slot], (unsigned long long)alive);
@@ -227,9 +227,12 @@ __device__ void compact_touched(const BatchArgs &a, int slot, int buf) {
     flush_level(a, slot, edges, alive);
 }
 
-__device__ __forceinline__ u64 shfl_up64(u64 v, int o) {
-    u32 lo = __shfl_up((u32)v, o), hi = __shfl_up((u32)(v >> 32), o);
-    return ((u64)hi << 32) | lo;
+// One step of a segmented OR scan: lanes whose source lane has the same owner
+// (owners do not decrease over the lanes) take its value too.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ void owner_or_step(u64 &x, int owner) {
+    const u64 y = lane_before<CTRL, ROWS>((u64)0, x);
+    if (lane_before<CTRL, ROWS>(-1, owner) == owner) x |= y;
 }
 
 __device__ __forceinline__ u64 uniform64(u64 v) {
@@ -310,7 +313,7 @@ __device__ void bu_groups(const BatchArgs &a, u32 L, u64 alive_cur, int nxt, u64
         }
         if (!need) deg = 0;
         const u32 incl = wave_inclusive_scan(deg);
-        const u32 off = incl - deg, total = __shfl(incl, kWave - 1);
+        const u32 off = incl - deg, total = wave_last(incl);
         const u64 shift = base - (u64)off;  // CSR position of concatenated position e: shift + e
         u64 acc = 0;
         u64 done = ballot(deg == 0);
@@ -346,12 +349,12 @@ __device__ void bu_groups(const BatchArgs &a, u32 L, u64 alive_cur, int nxt, u64
                 if (!ballot(mq[q] != 0)) continue;
                 u64 x = mq[q];
                 const int j = jq[q];
-#pragma unroll
-                for (int o = 1; o < kWave; o <<= 1) {
-                    const u64 y = shfl_up64(x, o);
-                    const int yj = __shfl_up(j, o);
-                    if ((int)lane >= o && yj == j) x |= y;
-                }
+                owner_or_step<kDppShr + 1, 0xF>(x, j);
+                owner_or_step<kDppShr + 2, 0xF>(x, j);
+                owner_or_step<kDppShr + 4, 0xF>(x, j);
+                owner_or_step<kDppShr + 8, 0xF>(x, j);
+                owner_or_step<kDppBcast15, 0xA>(x, j);
+                owner_or_step<kDppBcast31, 0xC>(x, j);
                 const u64 got = shfl64(x, lastq[q]);
                 if (interq[q]) acc |= got;
             }
@@ -420,8 +423,7 @@ __device__ void bu_heavy_chunks(const BatchArgs &a, u32 L, u64 alive_cur) {
                 for (int q = 0; q < kSteps; ++q) m |= ok[q] ? fmc[w[q]] : 0;
                 m &= need;
                 if (!ballot(m != 0)) continue;
-                for (int o = 32; o > 0; o >>= 1) m |= shfl_xor64(m, o);
-                m = uniform64(m);
+                m = wave_or(m);
                 acc |= m;
                 need &= ~m;
             }

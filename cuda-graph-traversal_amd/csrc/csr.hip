@@ -39,31 +39,16 @@ __global__ __launch_bounds__(256) void degree_kernel(const Packed_Edge *__restri
     }
 }
 
-__device__ __forceinline__ u64 shfl_up64(u64 v, int d) {
-    u32 lo = __shfl_up((u32)v, d), hi = __shfl_up((u32)(v >> 32), d);
-    return ((u64)hi << 32) | lo;
-}
-
 // Exclusive scan over the block; *total receives the block sum.
 template <int BLOCK>
 __device__ __forceinline__ u64 block_exclusive_scan(u64 v, u64 *total) {
     __shared__ u64 wtot[BLOCK / kWave];
     const int lane = lane_id(), wave = threadIdx.x / kWave;
-    u64 x = v;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-        u64 y = shfl_up64(x, o);
-        if (lane >= o) x += y;
-    }
+    const u64 x = wave_inclusive_scan(v);
     if (lane == kWave - 1) wtot[wave] = x;
     __syncthreads();
     if (wave == 0) {
-        u64 t = lane < BLOCK / kWave ? wtot[lane] : 0;
-#pragma unroll
-        for (int o = 1; o < BLOCK / kWave; o <<= 1) {
-            u64 y = shfl_up64(t, o);
-            if (lane >= o) t += y;
-        }
+        const u64 t = wave_inclusive_scan(lane < BLOCK / kWave ? wtot[lane] : (u64)0);
         if (lane < BLOCK / kWave) wtot[lane] = t;
     }
     __syncthreads();
@@ -599,7 +584,7 @@ __global__ __launch_bounds__(kRadixBlock) void sort_segments_radix(
     u32 *__restrict__ s_lo, u32 *__restrict__ s_hi, int col_passes) {
     __shared__ u32 base[256];
     __shared__ u32 wcnt[kRadixWaves][256];
-    const int lane = lane_id(), wave = threadIdx.x / kWave;
+    const int wave = threadIdx.x / kWave;
     const int npass = col_passes + 4;
     const u32 count = *nsegs;
     for (u32 r = blockIdx.x; r < count; r += gridDim.x) {
@@ -617,11 +602,7 @@ __global__ __launch_bounds__(kRadixBlock) void sort_segments_radix(
             __syncthreads();
             if (threadIdx.x < 256) {  // exclusive scan of the 256 bins, 4 waves
                 u32 x = base[threadIdx.x];
-                u32 incl = x;
-                for (int o = 1; o < kWave; o <<= 1) {
-                    u32 y = __shfl_up(incl, o);
-                    if (lane >= o) incl += y;
-                }
+                const u32 incl = wave_inclusive_scan(x);
                 wcnt[0][threadIdx.x] = incl;  // staging of wave-inclusive sums
             }
             __syncthreads();

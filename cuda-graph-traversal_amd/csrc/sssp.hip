@@ -323,7 +323,7 @@ __device__ __forceinline__ void walk_segments(const SsspArgs &a, const Target &t
                                               u64 &improved, volatile int *slot, Stage &sq) {
     if (!ballot(len != 0)) return;
     const u32 incl = wave_inclusive_scan(len);
-    const u32 off = incl - len, total = __shfl(incl, kWave - 1);
+    const u32 off = incl - len, total = wave_last(incl);
     const u32 lane = lane_id();
     for (u32 c = 0; c < total; c += kQ * kWave) {
         bool act[kQ];
@@ -956,10 +956,7 @@ __global__ __launch_bounds__(256) void hub_kernel(const u64 *__restrict__ rs, u6
     u64 m = 0;
     for (u64 v = (u64)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (u64)gridDim.x * blockDim.x)
         m = max(m, (MIN(rs[v + 1] - rs[v], (u64)0xFFFFFFFFu) << 32) | (0xFFFFFFFFu - (u32)v));
-    for (int o = 32; o > 0; o >>= 1) {
-        const u32 lo = __shfl_xor((u32)m, o), hi = __shfl_xor((u32)(m >> 32), o);
-        m = max(m, ((u64)hi << 32) | lo);
-    }
+    m = wave_last(wave_scan(m, (u64)0, [](u64 x, u64 y) { return y > x ? y : x; }));
     if (lane_id() == 0 && m) atomicMax((unsigned long long *)best, (unsigned long long)m);
 }
 

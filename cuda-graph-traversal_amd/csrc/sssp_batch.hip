@@ -448,7 +448,7 @@ __device__ __forceinline__ void relax_commit_push(const SsspBatchArgs &a, const 
             out[h] = cand < below[h] ? 1u << r[h] : 0u;
         }
     }
-    if (ballot(nimp != 0)) improved += wave_sum((u64)nimp);
+    if (ballot(nimp != 0)) improved += wave_sum(nimp);
     u64 any = 0;
 #pragma unroll
     for (int h = 0; h < R; ++h) any |= ballot(out[h] != 0);
@@ -736,7 +736,7 @@ __device__ __forceinline__ void group_tier(const SsspBatchArgs &a, u32 *pend, co
         }
         const u32 pairs = (u32)(e - b) * (u32)__popc(M);
         const u32 incl = wave_inclusive_scan(pairs);
-        const u32 off = incl - pairs, total = __shfl(incl, kWave - 1);
+        const u32 off = incl - pairs, total = wave_last(incl);
         {
             const u64 nitems = (u64)__popcll(ballot(M != 0)), nent = wave_sum((u64)(e - b));
             if (lane == 0) work_add(wk, nitems, nent, total);
@@ -1221,9 +1221,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void s
                 }
                 if (c == kDefer - 1) {  // far-class sources per root of the window (pull flushes read them)
                     const u32 hf = (H && len) ? H : 0u;
-                    u32 any = hf;
-#pragma unroll
-                    for (int o = 32; o >= 1; o >>= 1) any |= __shfl_xor(any, o);
+                    u32 any = wave_last(wave_scan(hf, 0u, [](u32 x, u32 y) { return x | y; }));
                     while (any) {
                         const int r = __ffs(any) - 1;
                         any &= any - 1;
