@@ -148,9 +148,13 @@ __global__ __launch_bounds__(512) void bfs_kernel(BfsArgs a) {
     u64 t_prev = gtid == 0 ? wall_clock64() : 0;
     for (u32 L = 0;; ++L) {
         const int cur = L % 3, nxt = (L + 1) % 3, clr = (L + 2) % 3;
+        // the level's words from the memory side, in one round trip
         const u64 nf = ld64(&ctl->fcount[cur]);
         const u64 mf = ld64(&ctl->fedges[cur]);
-        if (nf == 0 || ld_relaxed(&ctl->bar.error) || L >= 0x7FFFFFFFu) break;
+        u32 nq = ld_relaxed(&ctl->qlen[cur]);
+        u64 hp = ld_relaxed(&ctl->hcnt[cur]);
+        const u32 error = ld_relaxed(&ctl->bar.error);
+        if (nf == 0 || error || L >= 0x7FFFFFFFu) break;
         const u64 m_unexplored = a.m_total > m_explored + mf ? a.m_total - m_explored - mf : 0;
         bool next_bu = bottom_up;
         if (!bottom_up) next_bu = m_unexplored > 0 && (f32)mf > (f32)m_unexplored / a.alpha;
@@ -174,8 +178,7 @@ __global__ __launch_bounds__(512) void bfs_kernel(BfsArgs a) {
         if (next_bu && !bottom_up) {  // frontier queue -> bitmap
             for (u64 w = gtid; w < a.nwords; w += gthreads) fbc[w] = 0;
             bfs_sync(ctl, 2, L);
-            const u32 nq = ld_relaxed(&ctl->qlen[cur]);
-            const u64 nh = hub_count(ld_relaxed(&ctl->hcnt[cur]));
+            const u64 nh = hub_count(hp);
             const u32 *hc = a.hubs[L & 1];
             for (u64 i = gtid; i < (u64)nq + nh; i += gthreads) {
                 const u32 v = i < nq ? qc[i] : hc[i - nq];
@@ -205,14 +208,14 @@ __global__ __launch_bounds__(512) void bfs_kernel(BfsArgs a) {
                 }
             }
             bfs_sync(ctl, 4, L);
+            nq = ld_relaxed(&ctl->qlen[cur]);
+            hp = ld_relaxed(&ctl->hcnt[cur]);
         }
         bottom_up = next_bu;
 
         u32 cnt = 0;
         u64 edges = 0;
         if (!bottom_up) {
-            const u32 nq = ld_relaxed(&ctl->qlen[cur]);
-            const u64 hp = ld_relaxed(&ctl->hcnt[cur]);
             const u64 nh = hub_count(hp), ht = hub_total(hp);
             const u32 *hc = a.hubs[L & 1];
             const u64 *ho = a.hoff[L & 1];
