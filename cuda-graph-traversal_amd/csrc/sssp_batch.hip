@@ -1358,17 +1358,21 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void s
                 Queue q = read_queue(x + 1);
                 check_queue(q);
                 const bool next_empty = q.total == 0 && q.nnext == 0;
-                bool fl[kDefer], anyf = false;
+                bool fl[kDefer], anyf = false, by_empty = false;
                 u64 items = 0;
 #pragma unroll
                 for (int c = 0; c < kDefer; ++c) {
                     // due when some root's next bucket reaches past fl(epoch_r + W_c)
-                    bool due = next_empty;
+                    bool due = false;
                     for (int r = 0; r < a.nroots && !due; ++r) due = rbk.b[2][r] > rbk.ep[c][r] + a.dw[c];
-                    fl[c] = lpending[c] && due;
+                    fl[c] = lpending[c] && (due || next_empty);
+                    by_empty = by_empty || (fl[c] && !due);
                     anyf = anyf || fl[c];
                     if (fl[c]) items += (u64)lc[c][0] + lc[c][1] + hub_count(lh[c]);
                 }
+                // The flush fills the queue whose emptiness may have called for it:
+                // no block starts before every block has read it as empty.
+                if (by_empty) bsync(ctl, 10, gb, x);
                 if (anyf) {
                     // the far class is pulled when its window's items are a large share of the graph
                     constexpr int cf = kDefer - 1;
