@@ -382,9 +382,15 @@ struct Probe {
     u32 v, cb, cur;  // target, candidate distance bits, probe as read
 };
 // Relaxation rounds a lane has in flight: group tier, and the wave and hub
-// tiers (one item's row, so a round costs fewer registers there).
-constexpr int kRounds = 4;
-constexpr int kWideRounds = 8;
+// tiers (one item's row, so a round costs fewer registers there). With four
+// waves on a SIMD the kernel has 128 registers a lane and spills what does not
+// fit; more rounds spill more than their loads in flight hide (4 and 8 rounds
+// 188 spilled registers, 2 and 4 113). ms at 7 roots S12 / 7 roots S19 /
+// 32 roots S22: 4, 8 rounds 2.16 / 9.65 / 35.8; 4, 4 1.95 / 8.7 / 35.4; 2, 4
+// 1.87 / 8.5 / 35.2; 2, 2 1.85 / 8.6 / 36.6; 2, 5 1.88 / 8.6 / 35.7; 1, 2
+// 1.81 / 8.7 / 37.1.
+constexpr int kRounds = 2;
+constexpr int kWideRounds = 4;
 
 // Branch-free, so that the loads of both relaxations of a lane are issued
 // before the first one is waited for: an inactive lane reads entry 0 (valid
