@@ -1369,8 +1369,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void s
 #pragma unroll
                 for (int c = 0; c < kDefer; ++c) {
                     // due when some root's next bucket reaches past fl(epoch_r + W_c)
-                    bool due = false;
-                    for (int r = 0; r < a.nroots && !due; ++r) due = rbk.b[2][r] > rbk.ep[c][r] + a.dw[c];
+                    // (lane r looks at root r)
+                    const bool due = ballot(lane < (u32)a.nroots && rbk.b[2][lane % kBatchRoots] >
+                                                                   rbk.ep[c][lane % kBatchRoots] + a.dw[c]) != 0;
                     fl[c] = lpending[c] && (due || next_empty);
                     by_empty = by_empty || (fl[c] && !due);
                     anyf = anyf || fl[c];
@@ -1390,9 +1391,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void s
                     u32 elig = 0;  // roots that settled at least pull_ratio * nact sources in the window
                     if (fl[cf] && a.pull_ratio > 0.0f) {
                         const f32 need = a.pull_ratio * (f32)a.nact;
-                        for (int r = 0; r < a.nroots; ++r)
-                            if (((a.pull_roots >> r) & 1u) && (f32)ld_relaxed(&ctl->wcnt[wq.ls[cf]][r]) >= need)
-                                elig |= 1u << r;
+                        elig = (u32)ballot(lane < (u32)a.nroots && ((a.pull_roots >> (lane % kBatchRoots)) & 1u) &&
+                                           (f32)ld_relaxed(&ctl->wcnt[wq.ls[cf]][lane % kBatchRoots]) >= need);
                     }
                     const bool pull = elig != 0u;
                     // the window's other roots are pushed, their masks kept for the pull (cleared after it)
