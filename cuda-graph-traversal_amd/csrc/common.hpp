@@ -124,6 +124,14 @@ int cooperative_blocks(const void *kernel, int block, size_t dyn_lds);
 // batched BFS S16 1073 / 873 / 779 / 776 / 803 / 849, S22 - / - / 13815 / 7318 / 4217 / 3389.
 int persistent_grid(u64 work, int full, int block);
 
+// Kernel and grid of a persistent kernel that is built for four waves a SIMD
+// (packed) and for two, with twice the registers each (roomy).
+struct PersistentLaunch {
+    const void *kernel;
+    int grid, full;  // full: packed blocks that the device holds at once
+};
+PersistentLaunch pick_persistent(const void *packed, const void *roomy, u64 work, int block, size_t dyn_lds);
+
 // Launches a persistent kernel whose grid fits on the device at once. With
 // `cooperative`, uses a cooperative launch; if the runtime refuses it (the
 // cooperative queue is held by another process on the same device), or

@@ -98,6 +98,23 @@ int persistent_grid(u64 work, int full, int block) {
     return (int)std::min<f64>(full, 8.0 * std::ceil(std::max(blocks, 1.0) / 8.0));
 }
 
+// The SSSP kernels hold about 200 registers a lane where four waves on a SIMD
+// get 128 each, and spill the rest; two waves a SIMD spill nothing but are half
+// as many. A grid that needs no more than the roomy blocks loses nothing by
+// them, and a somewhat larger one less than the spills cost it. us, packed ->
+// roomy, by the blocks wanted: SSSP S12 338 -> 316, S16 695 -> 675, S19 1555 ->
+// 1490; batched, 7 roots S12 (16 blocks) 1850 -> 1690, 32 roots S16 (256) 5690 ->
+// 5400, 7 roots S19 (344) 8360 -> 7920; past the line 32 roots over 300001
+// uniform vertices (416) 6450 -> 6880, 16 roots S19 (512) 6650 -> 7370, 32 roots
+// S22 35300 -> 41000.
+PersistentLaunch pick_persistent(const void *packed, const void *roomy, u64 work, int block, size_t dyn_lds) {
+    const int want = persistent_grid(work, 1 << 30, block);
+    const int most = cooperative_blocks(roomy, block, dyn_lds);
+    if (want <= most + most / 2) return {roomy, std::min(want, most), 2 * most};
+    const int full = cooperative_blocks(packed, block, dyn_lds);
+    return {packed, std::min(want, full), full};
+}
+
 void launch_persistent(const void *kernel, int grid, int block, void **args, hipStream_t stream,
                        bool cooperative, size_t dyn_lds) {
     Context &c = ctx();

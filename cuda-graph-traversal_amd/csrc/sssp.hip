@@ -639,7 +639,9 @@ __device__ __forceinline__ void pull_step(const SsspArgs &a, u32 x, f32 lo, f32 
     sync_traced(ctl, kPhaseHeavy, lo_b, x);
 }
 
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void sssp_kernel(SsspArgs a) {
+// WAVES: waves that share a SIMD's registers (4 or 2, see pick_persistent).
+template <int WAVES>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WAVES))) void sssp_kernel(SsspArgs a) {
     SsspCtl *ctl = a.ctl;
     grid_join(&ctl->bar);
     const u64 gtid = (u64)blockIdx.x * blockDim.x + threadIdx.x, gthreads = (u64)gridDim.x * blockDim.x;
@@ -1102,20 +1104,20 @@ void oned_graph_sssp_run(Worker_State *ws, const Oned_Graph *g, Sssp_State *s, u
     a.delta = s->delta;
     a.dbound = g->rowstarts_s ? kPruneDistBound : __builtin_inff();
     const int block = ctx().sssp_block;
-    const int grid =
-        persistent_grid(g->nlocaledges / 512, cooperative_blocks((const void *)sssp_kernel, block, 0), block);
+    const PersistentLaunch pl = pick_persistent((const void *)sssp_kernel<4>, (const void *)sssp_kernel<2>,
+                                                g->nlocaledges / 512, block, 0);
     if (failed()) return;
     void *args[] = {&a};
     G500_HIP(hipMemsetAsync(s->ctl, 0, sizeof(SsspCtl), c.stream));
     timer_start();
-    launch_persistent((const void *)sssp_kernel, grid, block, args);
+    launch_persistent(pl.kernel, pl.grid, block, args);
     timer_stop();
     static SsspCtl h;
     g500_copy_to_host(&h, s->ctl, sizeof(h));
     if (h.bar.error) {
         u32 lo = 0xFFFFFFFFu, hi = 0;
         int at_lo = 0, at_hi = 0;
-        for (int b = 0; b < MIN(grid, kMaxTraceBlocks); ++b) {
+        for (int b = 0; b < MIN(pl.grid, kMaxTraceBlocks); ++b) {
             if (h.trace[b].barriers < lo) { lo = h.trace[b].barriers; at_lo = b; }
             if (h.trace[b].barriers > hi) { hi = h.trace[b].barriers; at_hi = b; }
         }
@@ -1123,7 +1125,7 @@ void oned_graph_sssp_run(Worker_State *ws, const Oned_Graph *g, Sssp_State *s, u
         fail("SSSP kernel error %u (1 barrier timeout, 2 hub list overflow, 4 bad queue entry, 8 queue overflow, "
              "16 bucket invariant, 32 distance at or above 2048 on the pruned SSSP copy: build with sssp_prune 0); %d blocks; barriers passed min %u (block %d phase %u tags %u/%u) max %u "
              "(block %d phase %u tags %u/%u)",
-             h.bar.error, grid, lo, at_lo, tl.phase, tl.a, tl.b, hi, at_hi, th.phase, th.a, th.b);
+             h.bar.error, pl.grid, lo, at_lo, tl.phase, tl.a, tl.b, hi, at_hi, th.phase, th.a, th.b);
     }
 }
 

@@ -932,7 +932,9 @@ __device__ __forceinline__ void hub_tier(const SsspBatchArgs &a, const u32 *hv, 
     }
 }
 
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void sssp_batch_kernel(SsspBatchArgs a) {
+// WAVES: waves that share a SIMD's registers (4 or 2, see pick_persistent).
+template <int WAVES>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WAVES))) void sssp_batch_kernel(SsspBatchArgs a) {
     SsspBatchCtl *ctl = a.ctl;
     grid_join(&ctl->bar);
     const u64 gtid = (u64)blockIdx.x * blockDim.x + threadIdx.x, gthreads = (u64)gridDim.x * blockDim.x;
@@ -1770,8 +1772,15 @@ void sssp_batch_lags(const f32 *offsets, i32 nroots, f32 delta, u32 *lag, f32 *u
     }
 }
 
-static int launch_grid(const Oned_Graph *g, i32 nroots, int full) {
-    return persistent_grid(g->nlocaledges * (u64)nroots / 1024, full, ctx().batch_sssp_block);
+// Kernel and grid of a batch; `grid`: a serving slot's share of the resident
+// blocks, 0 for the whole device.
+static PersistentLaunch pick_launch(const Oned_Graph *g, i32 nroots, int grid) {
+    const int block = ctx().batch_sssp_block;
+    const void *packed = (const void *)sssp_batch_kernel<4>, *roomy = (const void *)sssp_batch_kernel<2>;
+    const u64 work = g->nlocaledges * (u64)nroots / 1024;
+    // slots share the CUs: their share was counted in packed blocks
+    if (grid > 0) return {packed, persistent_grid(work, grid, block), grid};
+    return pick_persistent(packed, roomy, work, block, q_lds_bytes(block));
 }
 
 bool sssp_batch_enqueue(const Oned_Graph *g, Sssp_Batch_State *s, const u64 *roots, const f32 *offsets, i32 nroots,
@@ -1875,14 +1884,13 @@ bool sssp_batch_enqueue(const Oned_Graph *g, Sssp_Batch_State *s, const u64 *roo
     a.dw[2] = wfar;
     const int block = ctx().batch_sssp_block;
     const size_t dyn = q_lds_bytes(block);
-    const int full = grid > 0 ? grid : cooperative_blocks((const void *)sssp_batch_kernel, block, dyn);
+    const PersistentLaunch pl = pick_launch(g, nroots, grid);
     if (failed()) return false;
-    grid = launch_grid(g, nroots, full);
     void *args[] = {&a};
     s->nroots = nroots;
     // the export's grid: as many blocks as the full grid holds waves / 4, at most one per 64 ids
     const unsigned xgrid = (unsigned)std::max<u64>(1, std::min<u64>((n + kExportIds - 1) / kExportIds,
-                                                                     (u64)full * (u64)block / 256));
+                                                                     (u64)pl.full * (u64)block / 256));
     auto export_labels = [&]() {
         sssp_batch_export_kernel<<<xgrid, 256, 0, st>>>(a.lab, a.perm, a.iperm, n, nroots, a.dbound, a.dist, a.pred,
                                                         a.ctl);
@@ -1890,11 +1898,11 @@ bool sssp_batch_enqueue(const Oned_Graph *g, Sssp_Batch_State *s, const u64 *roo
     };
     if (library) {
         timer_start();
-        launch_persistent((const void *)sssp_batch_kernel, grid, block, args, nullptr, true, dyn);
+        launch_persistent(pl.kernel, pl.grid, block, args, nullptr, true, dyn);
         export_labels();
         timer_stop();
     } else {
-        launch_persistent((const void *)sssp_batch_kernel, grid, block, args, st, false, dyn);
+        launch_persistent(pl.kernel, pl.grid, block, args, st, false, dyn);
         export_labels();
     }
     return !failed();
@@ -1910,7 +1918,7 @@ u32 sssp_batch_error(const Sssp_Batch_State *s, hipStream_t stream) {
 
 int sssp_batch_grid() {
     const int block = ctx().batch_sssp_block;
-    return cooperative_blocks((const void *)sssp_batch_kernel, block, q_lds_bytes(block));
+    return cooperative_blocks((const void *)sssp_batch_kernel<4>, block, q_lds_bytes(block));
 }
 
 }  // namespace g500
@@ -1969,7 +1977,7 @@ void oned_graph_sssp_batch_run_offsets(Worker_State *ws, const Oned_Graph *g, Ss
         // where the blocks stood: the fewest and most grid barriers passed, with the phase and tags of each
         static SsspBatchCtl h;
         g500_copy_to_host(&h, s->ctl, sizeof(h));
-        const int nb = std::min(launch_grid(g, nroots, sssp_batch_grid()), kMaxTraceBlocks);
+        const int nb = std::min(pick_launch(g, nroots, 0).grid, kMaxTraceBlocks);
         u32 lo = 0xFFFFFFFFu, hi = 0;
         int at_lo = 0, at_hi = 0;
         for (int b = 0; b < nb; ++b) {

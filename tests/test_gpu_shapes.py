@@ -193,3 +193,25 @@ def test_sssp_copy_of_step_weights(arena, oracle, n, ne, tight):
     finally:
         a.reserved = saved
     check_sssp_copy(arena, g)
+
+
+# both builds of the batched kernel, and both sides of the line between them
+# (entries times roots / 1024 = (1.5 resident roomy blocks)^2: between 18 and 19
+# roots here on 256 CUs)
+@pytest.mark.parametrize("scale,nroots", [(6, 1), (6, 32), (18, 16), (18, 18), (18, 20), (18, 32)])
+def test_batch_sssp_packed_and_roomy(arena, oracle, scale, nroots):
+    n = 1 << scale
+    g = arena.csr(arena.generate(scale), n)
+    ref = oracle.csr(n, *oracle.kronecker(scale))
+    roots = np.resize(oracle.roots(ref), nroots).astype(np.uint64)
+    sb, s1 = arena.sssp_batch_create(g, 0.05), arena.sssp_create(g, 0.05)
+    arena.sssp_batch(g, sb, roots)
+    for i, r in enumerate(roots):
+        d, p = arena.sssp_batch_result(g, sb, i)
+        if i in (0, nroots - 1):
+            want = oracle.dijkstra_f32(ref, int(r))[0]
+            assert oracle.sssp_check(ref, int(r), d, p) == 0, i
+        else:
+            arena.sssp(g, s1, int(r))
+            want = arena.sssp_result(s1)[0]
+        assert np.array_equal(d.view(np.uint32), want.view(np.uint32)), i
