@@ -158,8 +158,9 @@ struct Target {
 constexpr u32 kSCap = 64;
 constexpr int kSLists = 3;  // light tier 0, light tier 1, heavy wave tier
 struct StageLds {
-    u32 v[1024 / kWave][kSLists][kSCap];
-    u32 cnt[1024 / kWave][kSLists];
+    u32 v[512 / kWave][kSLists][kSCap];
+    u32 cnt[512 / kWave][kSLists];
+    u32 found[512 / kWave][2][2 * kWave];  // see Found
 };
 struct Stage {
     StageLds *L;
@@ -372,10 +373,10 @@ constexpr int kLocalRounds = 8;
 __device__ __forceinline__ void local_rounds(const SsspArgs &a, const Target &t, u64 &improved, volatile int *slot,
                                              Stage &sq) {
     for (int round = 0; round < kLocalRounds && sq.n[0]; ++round) {
-        const u32 n = sq.n[0];
+        const u32 n = min(sq.n[0], (u32)kWave);
+        sq.n[0] -= n;
         const bool mine = lane_id() < n;
-        const u32 u = mine ? ((volatile u32 *)sq.L->v[sq.w][0])[lane_id()] : 0;
-        sq.n[0] = 0;
+        const u32 u = mine ? ((volatile u32 *)sq.L->v[sq.w][0])[sq.n[0] + lane_id()] : 0;
         u64 b = 0, e = 0;
         u32 was = 0;
         if (mine) {
@@ -487,12 +488,13 @@ __device__ __forceinline__ void process_hubs(const SsspArgs &a, const u32 *hv, c
     }
 }
 
-// Calls f(v, probe distance bits) for every reached vertex that is not
+// Calls f(v, probe distance bits, last) for every reached vertex that is not
 // settled, with the whole wave converged: each lane reads one 64-vertex word
 // of reached & ~settled, a ballot picks the words with such vertices, and
 // the wave walks them one word at a time (lane = vertex of the word; lanes of
 // other vertices get +inf bits). Words in which everything is
-// settled or unreached cost one load per 64 of them.
+// settled or unreached cost one load per 64 of them. A last call, without
+// vertices, has `last` set.
 template <typename F>
 __device__ __forceinline__ void scan_open(const SsspArgs &a, F &&f) {
     const u64 gtid = (u64)blockIdx.x * blockDim.x + threadIdx.x, gthreads = (u64)gridDim.x * blockDim.x;
@@ -503,32 +505,64 @@ __device__ __forceinline__ void scan_open(const SsspArgs &a, F &&f) {
     // base + l * nwaves + g): open vertices cluster in the degree order, and
     // runs of 64 consecutive words per wave would leave most waves idle while
     // a few walk dense runs.
-    for (u64 base = 0; base < nwords; base += nwaves * kWave) {
-        const u64 w = base + (u64)lane * nwaves + wave_gid;
-        const u64 open_l = w < nwords ? (a.reached[w] & ~a.settled[w]) : 0ull;
-        u64 todo = ballot(open_l != 0);
-        // software pipelined: the next word's labels load while f runs
-        auto word_of = [&](int j) { return base + (u64)j * nwaves + wave_gid; };
-        auto take = [&](int &j, u32 &lbits) {
-            j = todo ? __ffsll((unsigned long long)todo) - 1 : -1;
-            todo &= todo - 1;
-            const u64 open = shfl64(open_l, j < 0 ? 0 : j);
-            const u64 v = word_of(j < 0 ? 0 : j) * 64 + lane;
-            lbits = (j >= 0 && ((open >> lane) & 1)) ? a.dl[v] : kInfBits;
-        };
-        int j;
-        u32 lbits;
-        take(j, lbits);
-        while (j >= 0) {
-            int jn;
-            u32 ln;
-            take(jn, ln);
-            f(word_of(j) * 64 + lane, lbits);
-            j = jn;
-            lbits = ln;
+    u64 base = 0, open_l = 0, todo = 0;
+    bool first = true;
+    auto take = [&](u64 &v, u32 &lbits) -> bool {  // the next word with open vertices and its labels
+        while (!todo) {
+            if (!first) base += nwaves * kWave;
+            first = false;
+            if (base >= nwords) return false;
+            const u64 w = base + (u64)lane * nwaves + wave_gid;
+            open_l = w < nwords ? (a.reached[w] & ~a.settled[w]) : 0ull;
+            todo = ballot(open_l != 0);
         }
+        const int j = __ffsll((unsigned long long)todo) - 1;
+        todo &= todo - 1;
+        v = (base + (u64)j * nwaves + wave_gid) * 64 + lane;
+        lbits = ((shfl64(open_l, j) >> lane) & 1) ? a.dl[v] : kInfBits;
+        return true;
+    };
+    u64 v = 0;
+    u32 lbits = kInfBits;
+    bool have = take(v, lbits);
+    for (;;) {  // software pipelined: the next word's labels load while f runs
+        u64 vn = 0;
+        u32 ln = kInfBits;
+        const bool more = have && take(vn, ln);
+        f(v, lbits, !have);
+        if (!have) break;
+        v = vn;
+        lbits = ln;
+        have = more;
     }
 }
+
+// Vertices that a wave finds in its words of a scan, kept in LDS until there
+// are 64 of them (L 0: of the bucket, 1: of the next bucket). What follows is
+// a chain of dependent loads and atomics, and most words hold one or two
+// such vertices: walked word by word, the chains of a wave's words add up.
+// us, delta 0.05, word by word / gathered: S19 1680 / 1497, S24 7434 / 6955, S26
+// 27260 / 25880, 700001 uniform vertices 1635 / 1409.
+struct Found {
+    u32 n[2];
+    template <int L>
+    __device__ __forceinline__ void put(Stage &sq, bool want, u32 v) {
+        const u64 m = ballot(want);
+        if (!m) return;
+        if (want) ((volatile u32 *)sq.L->found[sq.w][L])[n[L] + mask_rank(m)] = v;
+        n[L] += (u32)__popcll(m);
+    }
+    // up to 64 of them: false when fewer than 64 are there and more may come
+    template <int L>
+    __device__ __forceinline__ bool get(Stage &sq, bool last, bool &act, u32 &v) {
+        if (n[L] < (last ? 1u : (u32)kWave)) return false;
+        const u32 k = min(n[L], (u32)kWave);
+        n[L] -= k;
+        act = lane_id() < k;
+        v = act ? ((volatile u32 *)sq.L->found[sq.w][L])[n[L] + lane_id()] : 0u;
+        return true;
+    }
+};
 
 // Pull form of fused step x for the bucket [lo, hi): settles the bucket and
 // lowers every other unsettled vertex to its best candidate through a heavy
@@ -550,7 +584,14 @@ __device__ __forceinline__ void pull_step(const SsspArgs &a, u32 x, f32 lo, f32 
     sq.hs = hs;
     const u32 lo_b = __float_as_uint(lo), hi_b = __float_as_uint(hi), hi2_b = __float_as_uint(hi2);
     u64 nset = 0;
-    for (u64 v0 = wave_gid * kWave; v0 < a.nact; v0 += nwaves * kWave) {  // the wave owns the word of v0
+    Found found{};
+    for (u64 v0 = wave_gid * kWave;; v0 += nwaves * kWave) {  // the wave owns the word of v0
+        for (bool act, last = v0 >= a.nact;;) {
+            u32 v;
+            if (!found.get<1>(sq, last, act, v)) break;
+            push_light(a, act, v, t, sq);
+        }
+        if (v0 >= a.nact) break;
         const u64 v = v0 + lane, word = v0 >> 6;
         const u64 sw = a.settled[word];
         const bool open = v < a.nact && !((sw >> lane) & 1);
@@ -590,7 +631,7 @@ __device__ __forceinline__ void pull_step(const SsspArgs &a, u32 x, f32 lo, f32 
         }
         const u64 rm = ballot(imp && lb >= kInfBits);
         if (rm && lane == 0) atomicOr((unsigned long long *)&a.reached[word], (unsigned long long)rm);
-        push_light(a, act && !longrow && best >= hi_b && best < hi2_b, (u32)v, t, sq);
+        found.put<1>(sq, act && !longrow && best >= hi_b && best < hi2_b, (u32)v);
     }
     stage_flush(a, sq);
     {  // the block sums its waves' settled counts and makes one atomic (every thread is here)
@@ -647,7 +688,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
     const u64 gtid = (u64)blockIdx.x * blockDim.x + threadIdx.x, gthreads = (u64)gridDim.x * blockDim.x;
     const u64 nwaves = gthreads / kWave;
     const u32 lane = lane_id();
-    __shared__ int slots[1024 / kWave][kWave];
+    __shared__ int slots[512 / kWave][kWave];
     volatile int *slot = slots[threadIdx.x / kWave];
     __shared__ StageLds slds;
     Stage sq;
@@ -789,34 +830,37 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
             stage_to(t);
             sq.hs = hs;
             u64 nset_local = 0;
-            scan_open(a, [&](u64 v, u32 lbits) {
+            Found found{};
+            scan_open(a, [&](u64 v, u32 lbits, bool last) {
                 bool mine = false, next = false;
-                u64 b = 0, e = 0;
-                f32 dv = 0.f;
                 if (lbits < kInfBits) {
                     const f32 d = __uint_as_float(lbits);
-                    if (d >= lo && d < hi) {
-                        mine = true;
-                        dv = d;
-                        segment<false>(a, (u32)v, b, e);
-                    } else if (d >= hi && d < hi2) {
-                        next = true;
-                    }
+                    mine = d >= lo && d < hi;
+                    next = d >= hi && d < hi2;
                 }
-                if (!ballot(mine || next)) return;  // the word holds only later buckets
-                push_light(a, next, (u32)v, t, sq);
                 // the bucket's vertices are final now: the wave owns the word of v
                 const u64 sm = ballot(mine);
                 if (sm && lane == 0) {
                     a.settled[v >> 6] |= sm;
                     nset_local += (u64)__popcll(sm);
                 }
-                const u32 len = (u32)(e - b);
-                const bool medium = mine && len > kSmall && len <= kHub;
-                stage_push<2>(a, sq, medium, (u32)v);
-                hub_append(&ctl->hhub[hs].v, a.hqh, a.hq_off, a.hq_len, mine && len > kHub, (u32)v, len, a.n,
-                           &ctl->bar.error);
-                walk_segments(a, t, (u32)v, dv, b, mine && len <= kSmall ? len : 0, improved, slot, sq);
+                found.put<0>(sq, mine, (u32)v);
+                found.put<1>(sq, next, (u32)v);
+                bool act;
+                u32 u;
+                while (found.get<1>(sq, last, act, u)) push_light(a, act, u, t, sq);
+                while (found.get<0>(sq, last, act, u)) {
+                    u64 b = 0, e = 0;
+                    f32 du = 0.f;
+                    if (act) {
+                        segment<false>(a, u, b, e);
+                        du = __uint_as_float(a.dl[u]);
+                    }
+                    const u32 len = (u32)(e - b);
+                    stage_push<2>(a, sq, len > kSmall && len <= kHub, u);
+                    hub_append(&ctl->hhub[hs].v, a.hqh, a.hq_off, a.hq_len, len > kHub, u, len, a.n, &ctl->bar.error);
+                    walk_segments(a, t, u, du, b, len <= kSmall ? len : 0, improved, slot, sq);
+                }
             });
             if (bucket_items <= nwaves) local_rounds(a, t, improved, slot, sq);
             stage_flush(a, sq);
@@ -861,8 +905,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
         clear_ahead(x);
         {
             u32 bits = 0xFFFFFFFFu;
-            scan_open(a, [&](u64 v, u32 lbits) {
+            scan_open(a, [&](u64 v, u32 lbits, bool last) {
                 (void)v;
+                (void)last;
                 if (lbits < kInfBits && __uint_as_float(lbits) >= hi) bits = min(bits, lbits);
             });
             bits = wave_min(bits);
@@ -890,14 +935,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
         {
             const Target t = target(x, hi, lo);
             stage_to(t);
-            scan_open(a, [&](u64 v, u32 lbits) {
-                bool want = false;
-                if (lbits < kInfBits) {
-                    const f32 d = __uint_as_float(lbits);
-                    want = d >= lo && d < hi;
-                }
-                if (!ballot(want)) return;
-                push_light(a, want, (u32)v, t, sq);
+            Found found{};
+            scan_open(a, [&](u64 v, u32 lbits, bool last) {
+                const f32 d = __uint_as_float(lbits);
+                found.put<1>(sq, lbits < kInfBits && d >= lo && d < hi, (u32)v);
+                bool act;
+                u32 u;
+                while (found.get<1>(sq, last, act, u)) push_light(a, act, u, t, sq);
             });
         }
         stage_flush(a, sq);
