@@ -279,6 +279,16 @@ __device__ __forceinline__ u64 wave_min64(u64 v) {
     return wave_last(wave_scan(v, ~(u64)0, [](u64 x, u64 y) { return y < x ? y : x; }));
 }
 
+// Smallest value of the lane's row of 16 lanes (rotations within the row); all
+// lanes active.
+__device__ __forceinline__ u32 row_min(u32 v) {
+    constexpr int kDppRor = 0x120;
+    v = min(v, lane_before<kDppRor + 8, 0xF>(~0u, v));
+    v = min(v, lane_before<kDppRor + 4, 0xF>(~0u, v));
+    v = min(v, lane_before<kDppRor + 2, 0xF>(~0u, v));
+    return min(v, lane_before<kDppRor + 1, 0xF>(~0u, v));
+}
+
 __device__ __forceinline__ u64 shfl64(u64 v, int src) {
     u32 lo = __shfl((u32)v, src), hi = __shfl((u32)(v >> 32), src);
     return ((u64)hi << 32) | lo;

@@ -44,8 +44,7 @@
 // The SSSP rows are symmetric, so these are the same relaxations. The scan of
 // v stops at the first entry with fl(lo + w) >= v's best distance so far:
 // every later candidate fl(d_u + w') has d_u >= lo and w' >= w, and rounding
-// is monotone. Rows up to kPullLane heavy entries are scanned by one lane,
-// longer ones by a wave in chunks of 64.
+// is monotone.
 // Work is mapped by row-segment length: a lane per vertex (<= 32 entries), a
 // wave per vertex (<= 1024), or chunks of a flattened hub work space spread
 // over the whole grid (longer).
@@ -62,7 +61,18 @@
 namespace g500 {
 
 constexpr u32 kSmall = 32;
-constexpr u64 kPullLane = 32;
+// Pull form: rows up to kPullLane heavy entries take one lane, kPullStep
+// entries in flight, longer ones kPullLanes lanes, above kPullWide a wave. Most
+// scans end within the first entries, so a wave per row reads 64 to use a few,
+// and every row that is not a lane's goes through the list's one counter.
+// First pull of an S26 root, us, at kPullLane 8 / 16 / 32 / 64 / 128 (runs of
+// 64 in the list): 3040 / 2010 / 1450 / 1290 / -, another root's with runs of
+// 256: - / - / 2750 / 2140 / 2005; with a lane's entries one after another and
+// a wave per longer row (32) 1790 for the former.
+constexpr u64 kPullLane = 64;
+constexpr int kPullStep = 4;
+constexpr u32 kPullLanes = 16;
+constexpr u64 kPullWide = 512;
 constexpr u32 kHub = 1024;
 constexpr u32 kStepLog = 1024;
 
@@ -572,7 +582,7 @@ struct Found {
 // lowers every other unsettled vertex to its best candidate through a heavy
 // entry from the bucket; vertices ending in [hi, hi2) are queued for the next
 // bucket. Two phases: a lane per vertex (rows of up to kPullLane heavy
-// entries; longer rows go to the wave list), then a wave per listed vertex.
+// entries; longer rows go to a list), then 16 lanes or a wave per listed one.
 // Counters: settled vertices into nset[(x + 1) % 3], the wave list in
 // hlen[(x + 1) % 3]. Ends after the second barrier.
 __device__ __forceinline__ void pull_step(const SsspArgs &a, u32 x, f32 lo, f32 hi, f32 hi2, u64 &improved,
@@ -589,6 +599,18 @@ __device__ __forceinline__ void pull_step(const SsspArgs &a, u32 x, f32 lo, f32 
     const u32 lo_b = __float_as_uint(lo), hi_b = __float_as_uint(hi), hi2_b = __float_as_uint(hi2);
     u64 nset = 0;
     Found found{};
+    u64 swn = 0;
+    u32 lbn = 0;
+    RowRec recn{};
+    auto fetch = [&](u64 v0) {
+        const u64 v = v0 + lane;
+        if (v0 < a.nact) swn = a.settled[v0 >> 6];
+        if (v < a.nact) {
+            lbn = a.dl[v];
+            recn = load_rec(a.rows, (u32)v);
+        }
+    };
+    fetch(wave_gid * kWave);
     for (u64 v0 = wave_gid * kWave;; v0 += nwaves * kWave) {  // the wave owns the word of v0
         for (bool act, last = v0 >= a.nact;;) {
             u32 v;
@@ -597,9 +619,11 @@ __device__ __forceinline__ void pull_step(const SsspArgs &a, u32 x, f32 lo, f32 
         }
         if (v0 >= a.nact) break;
         const u64 v = v0 + lane, word = v0 >> 6;
-        const u64 sw = a.settled[word];
+        const u64 sw = swn;
+        const RowRec rec = recn;
         const bool open = v < a.nact && !((sw >> lane) & 1);
-        const u32 lb = open ? a.dl[v] : kInfBits;
+        const u32 lb = open ? lbn : kInfBits;
+        fetch(v0 + nwaves * kWave);
         const bool mine = open && lb >= lo_b && lb < hi_b;
         const u64 sm = ballot(mine);
         if (sm && lane == 0) {
@@ -608,21 +632,38 @@ __device__ __forceinline__ void pull_step(const SsspArgs &a, u32 x, f32 lo, f32 
         }
         const bool act = open && !mine;
         u64 b = 0, e = 0;
-        if (act) segment<false>(a, (u32)v, b, e);
+        if (act) {
+            b = rec.start + rec.light;
+            e = rec.start + rec.len;
+        }
         const bool longrow = act && e - b > kPullLane;
         stage_push<2>(a, sq, longrow, (u32)v);
         u32 best = lb, bu = 0;
         if (act && !longrow) {
-            for (u64 k = b; k < e; ++k) {
-                const f32 wk = a.w[k];
-                if (__float_as_uint(__fadd_rn(lo, wk)) >= best) break;
-                const u32 u = a.col[k];
-                const u32 du = a.dl[u];
-                if (du >= lo_b && du < hi_b) {
-                    const u32 c = __float_as_uint(__fadd_rn(__uint_as_float(du), wk));
-                    if (c < best) {
-                        best = c;
-                        bu = u;
+            for (u64 k = b; k < e; k += kPullStep) {
+                f32 wk[kPullStep];
+                u32 uk[kPullStep], dk[kPullStep];
+                bool ok[kPullStep];
+#pragma unroll
+                for (int q = 0; q < kPullStep; ++q) {
+                    const u64 kk = k + (u64)q < e ? k + (u64)q : k;
+                    wk[q] = a.w[kk];
+                    uk[q] = a.col[kk];
+                }
+                if (__float_as_uint(__fadd_rn(lo, wk[0])) >= best) break;
+#pragma unroll
+                for (int q = 0; q < kPullStep; ++q) {
+                    ok[q] = k + (u64)q < e && __float_as_uint(__fadd_rn(lo, wk[q])) < best;
+                    dk[q] = a.dl[ok[q] ? uk[q] : (u32)v];
+                }
+#pragma unroll
+                for (int q = 0; q < kPullStep; ++q) {
+                    if (ok[q] && dk[q] >= lo_b && dk[q] < hi_b) {
+                        const u32 c = __float_as_uint(__fadd_rn(__uint_as_float(dk[q]), wk[q]));
+                        if (c < best) {
+                            best = c;
+                            bu = uk[q];
+                        }
                     }
                 }
             }
@@ -647,38 +688,78 @@ __device__ __forceinline__ void pull_step(const SsspArgs &a, u32 x, f32 lo, f32 
         if (threadIdx.x == 0 && bset) atomicAdd((unsigned long long *)&ctl->nset[hs], (unsigned long long)bset);
     }
     sync_traced(ctl, kPhaseFused, lo_b, x);
-    // long rows: a wave per vertex, 64 entries per chunk, lightest chunk first
+    // longer rows: 16 lanes per vertex, lightest entries first; those of more
+    // than kPullWide entries by the whole wave
     const u32 nlong = min(ld_relaxed(&ctl->hlen[hs].v), (u32)a.n);
-    for (u64 i = wave_gid; i < nlong; i += nwaves) {
-        const u32 v = a.hq1[i];
-        if (v >= a.n) {
-            if (lane == 0) atomicOr(&ctl->bar.error, 4u);
-            continue;
+    constexpr u32 kRows = kWave / kPullLanes;
+    for (u64 i0 = wave_gid * kRows; i0 < nlong; i0 += nwaves * kRows) {
+        const u32 gl = lane % kPullLanes;
+        const u64 i = i0 + lane / kPullLanes;
+        u32 v = i < nlong ? a.hq1[i] : 0u;
+        bool live = i < nlong;
+        if (live && v >= a.n) {
+            if (gl == 0) atomicOr(&ctl->bar.error, 4u);
+            live = false;
+            v = 0;
         }
         const u32 lb = a.dl[v];
         u64 b, e;
         segment<false>(a, v, b, e);
-        u64 best = ((u64)lb << 32) | 0xFFFFFFFFull;  // (distance bits, parent)
-        for (u64 k0 = b; k0 < e; k0 += kWave) {
-            if (__float_as_uint(__fadd_rn(lo, a.w[k0])) >= (u32)(best >> 32)) break;
-            const u64 k = k0 + lane;
-            u64 c = ~0ull;
-            if (k < e) {
-                const f32 wk = a.w[k];
-                const u32 u = a.col[k];
-                const u32 du = a.dl[u];
-                if (du >= lo_b && du < hi_b) c = ((u64)__float_as_uint(__fadd_rn(__uint_as_float(du), wk)) << 32) | u;
+        u32 best = lb, bu = ~0u;  // bu: ~0 until lowered
+        const bool wide = live && e - b > kPullWide;
+        u64 wides = ballot(wide && gl == 0);
+        live = live && !wide && e > b;
+        for (u64 k0 = b; ballot(live); k0 += kPullLanes) {
+            const u64 k = k0 + gl;
+            const bool in = live && k < e;
+            const f32 wk = a.w[in ? k : 0];
+            const u32 u = a.col[in ? k : 0];
+            const bool near = in && __float_as_uint(__fadd_rn(lo, wk)) < best;
+            const u32 du = a.dl[near ? u : v];
+            u32 c = ~0u;
+            if (near && du >= lo_b && du < hi_b) c = __float_as_uint(__fadd_rn(__uint_as_float(du), wk));
+            const u32 m = row_min(c);
+            const u32 mu = row_min(c == m ? u : ~0u);
+            if (m < best) {
+                best = m;
+                bu = mu;
             }
-            best = wave_min64(best < c ? best : c);
+            // entries are in order of weight: one too heavy ends the row
+            const u64 heavy = ballot(in && !(__float_as_uint(__fadd_rn(lo, wk)) < best));
+            live = live && k0 + kPullLanes < e && !((heavy >> (lane & ~(kPullLanes - 1))) & ((1u << kPullLanes) - 1));
         }
-        const u32 bb = (u32)(best >> 32);
-        if (lane == 0 && bb < lb) {
-            a.dl[v] = bb;
-            a.lab[v] = best;
+        while (wides) {
+            const int src = __ffsll((unsigned long long)wides) - 1;
+            wides &= wides - 1;
+            const u64 bw = shfl64(b, src), ew = shfl64(e, src);
+            const u32 lw = __shfl(lb, src);
+            u64 bestw = ((u64)lw << 32) | 0xFFFFFFFFull;  // (distance bits, parent)
+            for (u64 k0 = bw; k0 < ew; k0 += kWave) {
+                if (__float_as_uint(__fadd_rn(lo, a.w[k0])) >= (u32)(bestw >> 32)) break;
+                const u64 k = k0 + lane;
+                u64 c = ~0ull;
+                if (k < ew) {
+                    const f32 wk = a.w[k];
+                    const u32 u = a.col[k];
+                    const u32 du = a.dl[u];
+                    if (du >= lo_b && du < hi_b)
+                        c = ((u64)__float_as_uint(__fadd_rn(__uint_as_float(du), wk)) << 32) | u;
+                }
+                bestw = wave_min64(bestw < c ? bestw : c);
+            }
+            if ((int)(lane & ~(kPullLanes - 1)) == src) {
+                best = (u32)(bestw >> 32);
+                bu = (u32)bestw;
+            }
+        }
+        const bool have = i < nlong && gl == 0 && e > b;
+        if (have && best < lb) {
+            a.dl[v] = best;
+            a.lab[v] = ((u64)best << 32) | bu;
             ++improved;
             if (lb >= kInfBits) atomicOr((unsigned long long *)&a.reached[v >> 6], 1ull << (v & 63));
         }
-        push_light(a, lane == 0 && bb >= hi_b && bb < hi2_b, v, t, sq);
+        push_light(a, have && best >= hi_b && best < hi2_b, v, t, sq);
     }
     stage_flush(a, sq);
     sync_traced(ctl, kPhaseHeavy, lo_b, x);

@@ -215,3 +215,37 @@ def test_batch_sssp_packed_and_roomy(arena, oracle, scale, nroots):
             arena.sssp(g, s1, int(r))
             want = arena.sssp_result(s1)[0]
         assert np.array_equal(d.view(np.uint32), want.view(np.uint32)), i
+
+
+# pulled buckets: rows on both sides of a lane's, 16 lanes' and a wave's, with
+# ties, infinite weights and scans that end at once or reach the last entry
+@pytest.mark.parametrize("length", [1, 3, 4, 5, 31, 62, 63, 64, 65, 127, 510, 511, 512, 513, 3000])
+@pytest.mark.parametrize("prune", [0, 1])
+def test_sssp_pull_rows_of_every_tier(arena, oracle, length, prune):
+    rng = np.random.default_rng(length)
+    n, e = two_stars(length)
+    e = np.concatenate([e, rng.integers(0, n, (n // 2, 2))]).astype(np.uint64)
+    for kind in ("heavy", "mixed", "equal"):
+        w = {"heavy": 0.5 + 0.4 * rng.random(len(e)), "mixed": rng.random(len(e)),
+             "equal": np.full(len(e), 0.75)}[kind].astype(np.float32)
+        if kind == "mixed":
+            w[::7] = np.inf
+        m = arena.mark()
+        saved = {k: arena.get_param(k) for k in ("sssp_pull", "sssp_prune")}
+        try:
+            arena.set_param("sssp_prune", prune)
+            g, ref = build(arena, n, e, w)
+            s = arena.sssp_create(g, 0.1)
+            for pull in (1e-9, 0.0, 0.3):
+                arena.set_param("sssp_pull", pull)
+                for root in (0, 2, length + 1):
+                    arena.sssp(g, s, root)
+                    d, p = arena.sssp_result(s)
+                    want, tree = oracle.dijkstra_f32(ref, root)
+                    assert np.array_equal(d.view(np.uint32), want.view(np.uint32)), (kind, pull, root)
+                    # an infinite entry between a reached and an unreached vertex counts in the oracle's own tree too
+                    assert oracle.sssp_check(ref, root, d, p) == oracle.sssp_check(ref, root, want, tree), (kind, root)
+        finally:
+            for k, x in saved.items():
+                arena.set_param(k, x)
+            arena.release(m)
