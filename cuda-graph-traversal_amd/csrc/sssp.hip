@@ -789,6 +789,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
     u64 improved = 0;
     u64 prev_total = 0;              // light-queue items of the step before (the same in every thread)
     u64 bucket_items = 0;            // light-queue items of the current bucket (the same in every thread)
+    u64 bucket_work = 0;             // the same, a hub as the lane items (kSmall entries) that its row would make
     u64 settled_total = 0;           // vertices settled so far (the same in every thread)
     u32 x = 0;                       // step
     f32 lo = 0.0f, hi = next_bound(0.0f, a.delta);
@@ -881,6 +882,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
             error = q.error;
             if (total == 0 || error) break;
             bucket_items += total;
+            bucket_work += total + hub_total(hub) / kSmall;
             if (gtid == 0) atomicAdd((unsigned long long *)&ctl->light_iters, 1ull);
             log_step(0, cnt[0], cnt[1], hub);
             const Target t = target(x, hi, lo);
@@ -902,8 +904,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
         if (gtid == 0) atomicAdd((unsigned long long *)&ctl->buckets, 1ull);
         log_step(1, 0, 0, 0);
         const f32 hi2 = next_bound(hi, a.delta);
+        // A hub pushes as much as the items of kSmall entries that its row makes,
+        // so it counts as those. Counted as one, the first bucket of an S26 root
+        // (8.2 million of 33 million vertices, 210 million heavy entries pushed
+        // into random labels: 9.1 ms) stayed below the share; pulled it takes 2.1.
         const u64 unsettled = a.nact > settled_total ? a.nact - settled_total : 0;
-        if (a.pull_ratio > 0.f && (f32)bucket_items >= a.pull_ratio * (f32)unsettled) {
+        if (a.pull_ratio > 0.f && (f32)bucket_work >= a.pull_ratio * (f32)unsettled) {
             pull_step(a, x, lo, hi, hi2, improved, sq);
             settled_total += ld_relaxed(&ctl->nset[(x + 1) % 3]);
             if (gtid == 0) atomicAdd((unsigned long long *)&ctl->pulls, 1ull);
@@ -980,7 +986,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
             if (q.total || q.nnext) {
                 lo = hi;
                 hi = hi2;
-                bucket_items = 0;
+                bucket_items = bucket_work = 0;
                 continue;
             }
             if (q.error) break;
@@ -1007,7 +1013,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
             break;
         }
         const f32 dmin = __uint_as_float(nm);
-        bucket_items = 0;
+        bucket_items = bucket_work = 0;
         lo = hi;
         hi = next_bound(lo, a.delta);
         while (dmin >= hi) {
