@@ -198,6 +198,18 @@ struct BTarget {
     const RootBuckets *rb;
 };
 
+// The target of relaxations. SCREEN: they read vmin before they lower it. The
+// roots of one entry all meet at their target's vmin, and most do not lower it;
+// where the atomics bound the steps the read saves more than it costs, in the
+// smaller grids of the roomy build it is one more load to wait for. us, without /
+// with: 32 roots S22 35000 / 32400, over 300001 uniform vertices 6330 / 6060, S19
+// 10900 / 10750, 16 roots S19 6590 / 6710; roomy 32 roots S16 5400 / 5480, 7 roots
+// S19 7990 / 8310; 7 roots S22 (packed) 22200 / 22500.
+template <bool SCREEN>
+struct RelaxTarget : BTarget {
+    static constexpr bool screen = SCREEN;
+};
+
 __device__ __forceinline__ int btier(u32 len) { return len <= kBSmall ? 0 : (len <= kBHub ? 1 : 2); }
 
 // Wave indices as wave-uniform (scalar) values: the compiler cannot tell on
@@ -407,12 +419,13 @@ __device__ __forceinline__ void relax_load(const SsspBatchArgs &a, f32 du, int r
 // phase at a time (probe atomics, label and mask updates, light-row counts,
 // pending-mask ORs, queue appends), so that the R atomics of a phase are in
 // flight together instead of one relaxation's chain after the other's.
-template <int R>
+template <int R, typename Target>
 __device__ __forceinline__ void relax_commit_push(const SsspBatchArgs &a, const u32 (&u)[R], const int (&r)[R],
-                                                  const Probe (&pr)[R], const bool (&act)[R], const BTarget &t,
+                                                  const Probe (&pr)[R], const bool (&act)[R], const Target &t,
                                                   u64 &improved, WaveQ &wq) {
     bool tried[R];
     u32 prev[R], out[R], ow[R], lw[R];
+    [[maybe_unused]] u32 vm[R];
     f32 below[R];
 #pragma unroll
     for (int h = 0; h < R; ++h) tried[h] = act[h] && pr[h].cur > pr[h].cb;
@@ -433,6 +446,10 @@ __device__ __forceinline__ void relax_commit_push(const SsspBatchArgs &a, const 
 #pragma unroll
     for (int h = 0; h < R; ++h)
         lw[h] = (tried[h] && __uint_as_float(pr[h].cb) < below[h]) ? a.split[pr[h].v] : 0u;
+    if constexpr (Target::screen) {  // as read it may be larger (see cur), which only lets an atomic through
+#pragma unroll
+        for (int h = 0; h < R; ++h) vm[h] = tried[h] ? a.vmin[pr[h].v] : 0u;
+    }
     u32 nimp = 0;  // lowered probes of this lane; summed per wave below (a wave-uniform counter)
 #pragma unroll
     for (int h = 0; h < R; ++h) {
@@ -441,7 +458,10 @@ __device__ __forceinline__ void relax_commit_push(const SsspBatchArgs &a, const 
         if (tried[h] && prev[h] > cb) {
             const f32 cand = __uint_as_float(cb);
             atomicMin((unsigned long long *)&a.lab[(u64)v * kBatchRoots + r[h]], ((unsigned long long)cb << 32) | u[h]);
-            atomicMin(&a.vmin[v], __float_as_uint(cand + t.rb->u[r[h]]));
+            const u32 reduced = __float_as_uint(cand + t.rb->u[r[h]]);
+            bool lower = true;
+            if constexpr (Target::screen) lower = reduced < vm[h];
+            if (lower) atomicMin(&a.vmin[v], reduced);
             if (prev[h] >= kInfBits) {  // v reached from root r: it has open work (again)
                 // bits are cleared only by dense scans, never during a relaxation phase, so a
                 // set bit read in this phase is current; a clear one may race a concurrent OR,
@@ -712,9 +732,9 @@ __device__ __forceinline__ void pull_clear(const SsspBatchArgs &a, u32 n0, u32 n
 // Tier 0 (segments <= 32 entries): a wave takes 64 items and walks their
 // concatenated pair ranges 64 pairs at a time. Light and long items read their
 // mask from pend and clear it; medium items carry it in the list entry.
-template <int K>
+template <int K, typename Target>
 __device__ __forceinline__ void group_tier(const SsspBatchArgs &a, u32 *pend, const u32 *lq, const u64 *hq, u32 count,
-                           const BTarget &t, u64 &improved, volatile int *slot, u64 *wk, WaveQ &wq,
+                           const Target &t, u64 &improved, volatile int *slot, u64 *wk, WaveQ &wq,
                            u32 keep = ~0u, u32 *grab = nullptr) {
     const u64 gthreads = (u64)gridDim.x * blockDim.x;
     const u32 lane = lane_id();
@@ -820,9 +840,9 @@ __device__ __forceinline__ PairLanes pair_lanes(u32 M) {
 }
 
 // Tier 1 (segments <= 1024 entries): a wave per item.
-template <int K>
+template <int K, typename Target>
 __device__ __forceinline__ void wave_tier(const SsspBatchArgs &a, u32 *pend, const u32 *lq, const u64 *hq, u32 count,
-                          const BTarget &t, u64 &improved, u64 *wk, WaveQ &wq, u32 keep = ~0u) {
+                          const Target &t, u64 &improved, u64 *wk, WaveQ &wq, u32 keep = ~0u) {
     const u64 gthreads = (u64)gridDim.x * blockDim.x;
     const u32 lane = lane_id();
     const u64 wave_gid = wave_index(), nwaves = gthreads / kWave;
@@ -875,9 +895,9 @@ __device__ __forceinline__ void wave_tier(const SsspBatchArgs &a, u32 *pend, con
 // Hub tier: chunks of the flattened work space. Light and long hubs read their
 // mask from pend (cleared by the item's last chunk; `aux` counts finished
 // chunks); medium hubs from `aux`.
-template <int K>
+template <int K, typename Target>
 __device__ __forceinline__ void hub_tier(const SsspBatchArgs &a, const u32 *hv, const u64 *hoff, const u32 *hlen, u32 *aux,
-                         u32 *pend, u64 packed, const BTarget &t, u64 &improved, u64 *wk, WaveQ &wq,
+                         u32 *pend, u64 packed, const Target &t, u64 &improved, u64 *wk, WaveQ &wq,
                          u32 keep = ~0u) {
     const u64 gthreads = (u64)gridDim.x * blockDim.x;
     const u32 lane = lane_id();
@@ -1085,7 +1105,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
     };
     // pushes of step `step`; lvl 0: queued below hi_r (floor lo_r), 1: below hi2_r (floor hi_r)
     auto target = [&](u32 step, int lvl) {
-        return BTarget{(int)((step + 1) & 1), (int)((step + 1) % 3), lvl, &rbk};
+        return RelaxTarget<WAVES == 4>{{(int)((step + 1) & 1), (int)((step + 1) % 3), lvl, &rbk}};
     };
     // Word-parallel pass over the vertices with open work: each lane reads one
     // word of openw, the wave walks the words that have open vertices, one
@@ -1211,7 +1231,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
             error = q.error;
             if (total == 0 || error) break;
             if (gtid == 0) atomicAdd((unsigned long long *)&ctl->light_iters, 1ull);
-            const BTarget t = target(x, 0);
+            const auto t = target(x, 0);
             const int buf = (int)(x & 1);
             light_dest(t);
             // selects, not runtime indexes into the argument struct (which would copy it to scratch)
@@ -1243,7 +1263,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
         if (gtid == 0) st_relaxed(&ctl->plen.v, 0u);
         __syncthreads();
         {
-            const BTarget t = target(x, 1);
+            const auto t = target(x, 1);
             const int hs = (int)((x + 1) % 3);
             light_dest(t);
             wq.hs = hs;
@@ -1539,7 +1559,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
         // collect step: queue every root's bucket [lo_r, hi_r)
         clear_ahead(x);
         {
-            const BTarget t = target(x, 0);
+            const auto t = target(x, 0);
             light_dest(t);
             scan_open(1, [&](u64 word, u64 v, u32 M, u32 B, u32 dmin, bool act, u32 R) {
                 (void)word;
