@@ -383,7 +383,14 @@ __device__ __forceinline__ void walk_segments(const SsspArgs &a, const Target &t
 // steps): S10 462 (15) / 408 (8), S14 769 (28) / 669 (12), S18 1562 (52) / 1295 (19),
 // S20 2402 (62) / 1928 (25), S22 3769 (64) / 3253 (26), S24 8668 (66) / 8295 (32);
 // without the conditions S12 568 / 593, S14 771 / 836.
+//
+// A round goes no further than one step of walk_segments: where a bucket starts
+// small but next to hubs, a wave would otherwise walk thousands of entries alone.
+// us without the limit / at 1024 / 512 / 256 / 128 entries: S16 802 / 808 / 692 /
+// 693 / 657, S12 (delta 0.05) 496 / 510 / 484 / 423 / 414, S19 1540 / 1422 / 1398 /
+// 1321 / 1381, 700001 uniform vertices 985 / 993 / 1004 / 985 / 1002.
 constexpr int kLocalRounds = 8;
+constexpr u32 kLocalEntries = kQ * kWave;
 __device__ __forceinline__ void local_rounds(const SsspArgs &a, const Target &t, u64 &improved, volatile int *slot,
                                              Stage &sq) {
     for (int round = 0; round < kLocalRounds && sq.n[0]; ++round) {
@@ -398,6 +405,11 @@ __device__ __forceinline__ void local_rounds(const SsspArgs &a, const Target &t,
             segment<true>(a, u, b, e);
         }
         asm volatile("s_waitcnt vmcnt(0)" : "+v"(was)::"memory");
+        if (wave_sum((u32)(e - b)) > kLocalEntries) {  // too much for one wave: back into the queue
+            const bool q = mine && atomicExch(&a.stamp[u], t.tag) != t.tag;  // unless queued again meanwhile
+            stage_push<0>(a, sq, q, u);
+            break;
+        }
         const f32 du = mine ? __uint_as_float(ld_relaxed(&a.dl[u])) : 0.f;
         walk_segments(a, t, u, du, b, (u32)(e - b), improved, slot, sq);
     }
