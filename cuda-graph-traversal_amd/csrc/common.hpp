@@ -38,7 +38,7 @@ struct Context {
     int bfs_hub_degree = 2048;    // frontier vertices above this degree are split grid-wide
     double batch_alpha = 15.0;    // the same two thresholds for the batched multi-root BFS
     double batch_beta = 18.0;
-    int batch_heavy_degree = 1 << 20; // batched bottom-up: vertices above this degree are split grid-wide
+    int batch_heavy_degree = 1 << 20; // batched bottom-up: vertices above this degree are split grid-wide (see heavy_bound)
     int sssp_block = 512;
     int batch_bfs_block = 512;    // threads per block of the batched BFS and batched SSSP kernels
     int batch_sssp_block = 512;
@@ -50,7 +50,8 @@ struct Context {
     double batch_pull = 0.2;       // batched SSSP pulls its far-class flush when the window's items >= this share
                                    // of the vertices with entries (0: never)
     double sssp_pull = 0.05;       // single-root SSSP pulls a bucket's heavy relaxations when the bucket's light
-                                  // items reach this share of the unsettled vertices (0: always push)
+                                  // items (a hub as the 32-entry items of its row) reach this share of the
+                                  // unsettled vertices (0: always push)
 };
 
 Context &ctx();
