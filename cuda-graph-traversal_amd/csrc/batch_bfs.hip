@@ -637,8 +637,9 @@ __global__ __launch_bounds__(256) void batch_depth_scatter(const u32 *__restrict
     }
 }
 
-// Degree above which a bottom-up level splits a vertex's row over the grid,
-// whatever the knob allows. The wave that owns 64 vertices of this degree
+// The degree above which a bottom-up level splits a vertex's row over the grid
+// when the knob leaves it to the library (kHeavyAuto; any other value of the
+// knob is the degree). The wave that owns 64 vertices of this degree
 // walks 64 times as many entries alone (the degree order puts them together),
 // so the bound grows with the number of vertex groups a wave has to amortise
 // that over; long rows cost a few dependent loads each, so it does not fall
@@ -707,7 +708,8 @@ bool bfs_batch_enqueue(const Oned_Graph *g, Bfs_Batch_State *b, const u64 *roots
     if (grid <= 0) grid = cooperative_blocks((const void *)batch_bfs_kernel, block, 0);
     grid = persistent_grid(a.m_total / 256, grid, block);
     if (failed()) return false;
-    a.heavy_degree = (u32)MIN((u64)c.batch_heavy_degree, heavy_bound(n, (u64)grid * (u64)block / kWave));
+    a.heavy_degree = c.batch_heavy_degree == kHeavyAuto ? (u32)heavy_bound(n, (u64)grid * (u64)block / kWave)
+                                                        : (u32)c.batch_heavy_degree;
     void *args[] = {&a};
     b->nroots = nroots;
     if (library) {

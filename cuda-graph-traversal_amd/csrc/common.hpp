@@ -18,6 +18,7 @@ namespace g500 {
 
 constexpr int kWave = 64;
 constexpr int kSsspBatchRoots = 32;  // roots (and label stride) of a batched SSSP launch
+constexpr int kHeavyAuto = 1 << 20;  // batch_heavy_degree's default: the library picks the degree (heavy_bound)
 
 struct Context {
     int device = -1;
@@ -38,7 +39,7 @@ struct Context {
     int bfs_hub_degree = 2048;    // frontier vertices above this degree are split grid-wide
     double batch_alpha = 15.0;    // the same two thresholds for the batched multi-root BFS
     double batch_beta = 18.0;
-    int batch_heavy_degree = 1 << 20; // batched bottom-up: vertices above this degree are split grid-wide (see heavy_bound)
+    int batch_heavy_degree = kHeavyAuto; // batched bottom-up: vertices above this degree are split grid-wide
     int sssp_block = 512;
     int batch_bfs_block = 512;    // threads per block of the batched BFS and batched SSSP kernels
     int batch_sssp_block = 512;

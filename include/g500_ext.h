@@ -292,6 +292,9 @@ void g500_copy_device(void *dst_device, const void *src_device, u64 bytes);
  * "batch_beta", "batch_heavy_degree", "bfs_block" and "sssp_block" (threads
  * per block of the persistent BFS / SSSP kernels, single and batched: 128,
  * 256 or 512), "gen_blocks", "coop_launch", "relabel"; read-only "num_cus", "sssp_batch_max").
+ * "batch_heavy_degree" is the degree above which a batched bottom-up level
+ * splits a vertex's row over the grid; its default, 1 << 20, leaves the degree
+ * to the library.
  * Returns 0 on success, -1 for an unknown name or a value out of range. */
 i32 g500_set_param(const char *name, f64 value);
 i32 g500_get_param(const char *name, f64 *value);
