@@ -36,3 +36,42 @@ def test_batch_heavy_degree_is_the_split_degree(arena, oracle, heavy):
     assert np.array_equal(np.sort(listed[listed > 0]), np.sort(degree[degree > heavy]))
     for i, r in enumerate(roots):
         assert np.array_equal(arena.batch_depth(g, b, i), oracle.bfs(ref, int(r))[1]), i
+
+
+def hub_row(weights):
+    """A vertex with an entry to random others for each of the weights."""
+    n = 1 << 20
+    other = np.random.default_rng(9).integers(1, n, len(weights))
+    return n, np.stack([np.zeros(len(weights), np.int64), other], 1), weights.astype(np.float32)
+
+
+def rows_ms(arena, tg, n):
+    """Device time of the rows alone (no copies), the least of five."""
+    old = arena.get_param("relabel")
+    arena.set_param("relabel", 0)
+    try:
+        ms = []
+        for _ in range(5):
+            m = arena.mark()
+            arena.csr(tg, n)
+            ms.append(arena.lib.g500_last_run_ms())
+            arena.release(m)
+        return min(ms)
+    finally:
+        arena.set_param("relabel", old)
+
+
+# One long row whose weights are not evenly spread: over-full bins, which blocks
+# sort. With squared uniform weights the first of 2605 bins holds 10^6 / sqrt(2605)
+# = 19600 entries (one block's radix sort, 40 ns an entry: 0.8 ms) and some 360 more
+# of 513 to 8000 are over-full; spread over the chip those cost no more than the
+# evenly spread row's whole construction (0.5 ms) again. So about 3.6 times that,
+# 6 with a margin; 13 when the blocks are as many as the long rows.
+def test_over_full_bins_of_one_row_are_sorted_side_by_side(arena, oracle):
+    u = np.random.default_rng(10).random(10**6)
+    n, e, w = hub_row(u * u)
+    g, ref = build(arena, n, e, w)
+    csr_equal(arena, g, ref)
+    even, skewed = (rows_ms(arena, arena.upload_tuples(e, x.astype(np.float32)), n) for x in (u, w))
+    print(f"[over-full bins] evenly spread {even:.3f} ms, squared {skewed:.3f} ms", flush=True)
+    assert skewed < 6 * even
