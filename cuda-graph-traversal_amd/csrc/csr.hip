@@ -529,23 +529,31 @@ __global__ __launch_bounds__(256) void sort_rows_wave(const u64 *__restrict__ rs
 
 // Segments that a wave does not sort: a block's bitonic sort in LDS up to
 // kSegBlock entries, a block's radix sort above. They are whole long rows, or
-// bins of rows whose weights are far from evenly spread (many equal ones).
+// bins of rows whose weights are far from evenly spread (many equal ones). A
+// bin's entries are still in the scratch pair, and its sort reads them there:
+// the wave that finds it too long would copy it alone (a row of 1e6 equal
+// weights: 6.9 of 24.3 ms).
 struct Segment {
     u64 at;       // in the columns and weights
-    u64 scratch;  // in the scratch pair (radix)
-    u32 len, pad;
+    u64 scratch;  // in the scratch pair (whole rows: radix only)
+    u32 len;
+    u32 in_scratch;  // where the entries are: 0 at, 1 scratch
 };
 constexpr u32 kSegThreads = 1024;
 __global__ __launch_bounds__(kSegThreads) void sort_segments_block(const Segment *__restrict__ segs, const u32 *__restrict__ nsegs,
-                                                           u32 *__restrict__ col, u32 *__restrict__ w) {
+                                                           u32 *__restrict__ col, u32 *__restrict__ w,
+                                                           const u32 *__restrict__ s_col,
+                                                           const u32 *__restrict__ s_w) {
     __shared__ u64 keys[kSegBlock];
     const u32 count = *nsegs;
     for (u32 r = blockIdx.x; r < count; r += gridDim.x) {
         const u64 b = segs[r].at;
         const u32 d = segs[r].len;
+        const u32 *from_col = segs[r].in_scratch ? s_col + segs[r].scratch : col + b;
+        const u32 *from_w = segs[r].in_scratch ? s_w + segs[r].scratch : w + b;
         u32 P = 128;
         while (P < d) P <<= 1;
-        for (u32 i = threadIdx.x; i < P; i += kSegThreads) keys[i] = i < d ? ((u64)w[b + i] << 32) | col[b + i] : ~0ull;
+        for (u32 i = threadIdx.x; i < P; i += kSegThreads) keys[i] = i < d ? ((u64)from_w[i] << 32) | from_col[i] : ~0ull;
         __syncthreads();
         for (u32 size = 2; size <= P; size <<= 1)
             for (u32 stride = size >> 1; stride > 0; stride >>= 1) {
@@ -570,8 +578,8 @@ __global__ __launch_bounds__(kSegThreads) void sort_segments_block(const Segment
 
 // Segments longer than kSegBlock entries, one 1024-thread block each, stable
 // LSD radix sort on 8-bit digits ping-ponging between the segment (column /
-// weight-bit arrays) and a scratch pair. Digits cover the column bits, then
-// the weight bits.
+// weight-bit arrays) and a scratch pair, from where the entries are. Digits
+// cover the column bits, then the weight bits.
 constexpr int kRadixBlock = 1024;
 constexpr int kRadixWaves = kRadixBlock / kWave;
 
@@ -591,10 +599,12 @@ __global__ __launch_bounds__(kRadixBlock) void sort_segments_radix(
         const u32 d = segs[r].len;
         u32 *a_lo = col + segs[r].at, *a_hi = wbits + segs[r].at;
         u32 *b_lo = s_lo + segs[r].scratch, *b_hi = s_hi + segs[r].scratch;
+        const int in_b = (int)segs[r].in_scratch;
         for (int pass = 0; pass < npass; ++pass) {
+            const bool from_b = (pass + in_b) & 1;
             const int shift = pass < col_passes ? 8 * pass : 32 + 8 * (pass - col_passes);
-            const u32 *src_lo = (pass & 1) ? b_lo : a_lo, *src_hi = (pass & 1) ? b_hi : a_hi;
-            u32 *dst_lo = (pass & 1) ? a_lo : b_lo, *dst_hi = (pass & 1) ? a_hi : b_hi;
+            const u32 *src_lo = from_b ? b_lo : a_lo, *src_hi = from_b ? b_hi : a_hi;
+            u32 *dst_lo = from_b ? a_lo : b_lo, *dst_hi = from_b ? a_hi : b_hi;
             if (threadIdx.x < 256) base[threadIdx.x] = 0;
             __syncthreads();
             for (u32 i = threadIdx.x; i < d; i += kRadixBlock)
@@ -650,7 +660,7 @@ __global__ __launch_bounds__(kRadixBlock) void sort_segments_radix(
                 __syncthreads();
             }
         }
-        if (npass & 1) {  // result sits in the scratch pair: copy back
+        if ((npass + in_b) & 1) {  // result sits in the scratch pair: copy back
             for (u32 i = threadIdx.x; i < d; i += kRadixBlock) {
                 a_lo[i] = b_lo[i];
                 a_hi[i] = b_hi[i];
@@ -828,8 +838,8 @@ __global__ __launch_bounds__(kLongBlock) void long_bin_kernel(LongRows a) {
     }
 }
 
-// Sorts every bin into its row; a bin too long for a wave is copied there and
-// listed for the block and radix sorts.
+// Sorts every bin into its row; a bin too long for a wave is listed for the
+// block and radix sorts.
 __global__ __launch_bounds__(256) void long_sort_bins(LongRows a, SortLists *L, Segment *__restrict__ block_segs,
                                                       Segment *__restrict__ radix_segs) {
     const u32 lane = lane_id();
@@ -844,16 +854,10 @@ __global__ __launch_bounds__(256) void long_sort_bins(LongRows a, SortLists *L, 
             wave_sort_segment<4>(a.s_col + from, a.s_w + from, a.col + to, a.w + to, len);
         } else if (len <= 8 * kWave) {
             wave_sort_segment<8>(a.s_col + from, a.s_w + from, a.col + to, a.w + to, len);
-        } else {
-            for (u32 i = lane; i < len; i += kWave) {
-                a.col[to + i] = a.s_col[from + i];
-                a.w[to + i] = a.s_w[from + i];
-            }
-            if (lane == 0) {
-                const Segment s = {to, from, len, 0};
-                if (len <= kSegBlock) block_segs[atomicAdd(&L->nblock.v, 1u)] = s;
-                else radix_segs[atomicAdd(&L->nradix.v, 1u)] = s;
-            }
+        } else if (lane == 0) {
+            const Segment s = {to, from, len, 1};
+            if (len <= kSegBlock) block_segs[atomicAdd(&L->nblock.v, 1u)] = s;
+            else radix_segs[atomicAdd(&L->nradix.v, 1u)] = s;
         }
     }
 }
@@ -1758,7 +1762,7 @@ static bool sort_rows(Worker_State *ws, Oned_Graph *g) {
         const u64 most_block = bins ? tier_cap(a.nchunks, h.long_entries.v, kLongRow + 1) : a.nrows;
         const u64 most_radix = bins ? tier_cap(a.nchunks, h.long_entries.v, kSegBlock + 1) : a.nrows;
         sort_segments_block<<<(unsigned)MIN(most_block, (u64)c.num_cus * 4), kSegThreads, 0, s>>>(
-            block_segs, &L->nblock.v, col, w);
+            block_segs, &L->nblock.v, col, w, a.s_col, a.s_w);
         if (bins || h.huge_entries.v) {
             int bits = 1;
             while (bits < 32 && (1ull << bits) < n) ++bits;
