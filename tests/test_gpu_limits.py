@@ -81,8 +81,9 @@ def test_over_full_bins_of_one_row_are_sorted_side_by_side(arena, oracle):
 # much per entry as a row of 131000 entries, which is short enough to be sorted as
 # it lies, and the construction's other costs grow slower than the entries: at most
 # the ratio of the entries, with 5 % for the clock. 9.0 to 7.6 when the bin is
-# copied by one wave first.
-@pytest.mark.parametrize("entries", [10**6])
+# copied by one wave first; 70 to 30.5 when a row with more bins than are counted in
+# LDS makes a global atomic per entry.
+@pytest.mark.parametrize("entries", [10**6, 4 * 10**6])
 def test_a_row_of_equal_weights_costs_a_sort_as_it_lies(arena, oracle, entries):
     ms = {}
     for k in (131000, entries):
@@ -92,3 +93,17 @@ def test_a_row_of_equal_weights_costs_a_sort_as_it_lies(arena, oracle, entries):
         ms[k] = rows_ms(arena, arena.upload_tuples(e, w), n)
     print(f"[equal weights] {ms}", flush=True)
     assert ms[entries] < 1.05 * entries / 131000 * ms[131000]
+
+
+# rows around one and two rounds of 8192 bins counted at a time (384 entries a
+# bin), alone and with a second row in the same span, evenly spread or not
+@pytest.mark.parametrize("entries", [384 * 8192, 384 * 8192 + 1, 2 * 384 * 8192 + 5000])
+def test_rows_of_more_bins_than_one_round(arena, oracle, entries):
+    rng = np.random.default_rng(entries)
+    u = rng.random(entries)
+    u[::3] *= u[::3]  # some over-full bins at the light end
+    n, e, w = hub_row(u)
+    second = np.stack([np.ones(600, np.int64), rng.integers(2, n, 600)], 1)  # its chunks follow the hub's
+    e, w = np.concatenate([e, second]), np.concatenate([w, rng.random(600).astype(np.float32)])
+    g, ref = build(arena, n, e, w)
+    csr_equal(arena, g, ref)
