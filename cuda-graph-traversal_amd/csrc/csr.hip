@@ -540,6 +540,30 @@ struct Segment {
     u32 in_scratch;  // where the entries are: 0 at, 1 scratch
 };
 constexpr u32 kSegThreads = 1024;
+__device__ __forceinline__ void block_sort(u64 *keys, const u32 *from_col, const u32 *from_w, u32 *col, u32 *w, u32 d) {
+    u32 P = 128;
+    while (P < d) P <<= 1;
+    for (u32 i = threadIdx.x; i < P; i += kSegThreads) keys[i] = i < d ? ((u64)from_w[i] << 32) | from_col[i] : ~0ull;
+    __syncthreads();
+    for (u32 size = 2; size <= P; size <<= 1)
+        for (u32 stride = size >> 1; stride > 0; stride >>= 1) {
+            for (u32 t = threadIdx.x; t < P / 2; t += kSegThreads) {
+                const u32 i = 2 * stride * (t / stride) + (t % stride), j = i + stride;
+                const bool up = (i & size) == 0;
+                const u64 a = keys[i], c = keys[j];
+                if ((a > c) == up) {
+                    keys[i] = c;
+                    keys[j] = a;
+                }
+            }
+            __syncthreads();
+        }
+    for (u32 i = threadIdx.x; i < d; i += kSegThreads) {
+        col[i] = (u32)keys[i];
+        w[i] = (u32)(keys[i] >> 32);
+    }
+    __syncthreads();
+}
 __global__ __launch_bounds__(kSegThreads) void sort_segments_block(const Segment *__restrict__ segs, const u32 *__restrict__ nsegs,
                                                            u32 *__restrict__ col, u32 *__restrict__ w,
                                                            const u32 *__restrict__ s_col,
@@ -548,31 +572,9 @@ __global__ __launch_bounds__(kSegThreads) void sort_segments_block(const Segment
     const u32 count = *nsegs;
     for (u32 r = blockIdx.x; r < count; r += gridDim.x) {
         const u64 b = segs[r].at;
-        const u32 d = segs[r].len;
         const u32 *from_col = segs[r].in_scratch ? s_col + segs[r].scratch : col + b;
         const u32 *from_w = segs[r].in_scratch ? s_w + segs[r].scratch : w + b;
-        u32 P = 128;
-        while (P < d) P <<= 1;
-        for (u32 i = threadIdx.x; i < P; i += kSegThreads) keys[i] = i < d ? ((u64)from_w[i] << 32) | from_col[i] : ~0ull;
-        __syncthreads();
-        for (u32 size = 2; size <= P; size <<= 1)
-            for (u32 stride = size >> 1; stride > 0; stride >>= 1) {
-                for (u32 t = threadIdx.x; t < P / 2; t += kSegThreads) {
-                    const u32 i = 2 * stride * (t / stride) + (t % stride), j = i + stride;
-                    const bool up = (i & size) == 0;
-                    const u64 a = keys[i], c = keys[j];
-                    if ((a > c) == up) {
-                        keys[i] = c;
-                        keys[j] = a;
-                    }
-                }
-                __syncthreads();
-            }
-        for (u32 i = threadIdx.x; i < d; i += kSegThreads) {
-            col[b + i] = (u32)keys[i];
-            w[b + i] = (u32)(keys[i] >> 32);
-        }
-        __syncthreads();
+        block_sort(keys, from_col, from_w, col + b, w + b, segs[r].len);
     }
 }
 
@@ -587,86 +589,153 @@ __device__ __forceinline__ u32 digit_of(u32 lo, u32 hi, int shift) {
     return shift < 32 ? (lo >> shift) & 0xFF : (hi >> (shift - 32)) & 0xFF;
 }
 
+struct RadixLds {
+    u32 base[256];
+    u32 wcnt[kRadixWaves][256];
+};
+// Sorts the d entries of pair a, or of pair b with in_b set, into a.
+__device__ __forceinline__ void block_radix(RadixLds &lds, u32 *a_lo, u32 *a_hi, u32 *b_lo, u32 *b_hi, int in_b, u32 d,
+                                            int col_passes) {
+    const int wave = threadIdx.x / kWave;
+    const int npass = col_passes + 4;
+    for (int pass = 0; pass < npass; ++pass) {
+        const bool from_b = (pass + in_b) & 1;
+        const int shift = pass < col_passes ? 8 * pass : 32 + 8 * (pass - col_passes);
+        const u32 *src_lo = from_b ? b_lo : a_lo, *src_hi = from_b ? b_hi : a_hi;
+        u32 *dst_lo = from_b ? a_lo : b_lo, *dst_hi = from_b ? a_hi : b_hi;
+        if (threadIdx.x < 256) lds.base[threadIdx.x] = 0;
+        __syncthreads();
+        for (u32 i = threadIdx.x; i < d; i += kRadixBlock)
+            atomicAdd(&lds.base[digit_of(src_lo[i], src_hi[i], shift)], 1u);
+        __syncthreads();
+        if (threadIdx.x < 256) {  // exclusive scan of the 256 bins, 4 waves
+            u32 x = lds.base[threadIdx.x];
+            const u32 incl = wave_inclusive_scan(x);
+            lds.wcnt[0][threadIdx.x] = incl;  // staging of wave-inclusive sums
+        }
+        __syncthreads();
+        if (threadIdx.x < 256) {
+            u32 add = 0;
+            for (int w = 0; w < (int)(threadIdx.x / kWave); ++w) add += lds.wcnt[0][w * kWave + kWave - 1];
+            lds.base[threadIdx.x] = add + lds.wcnt[0][threadIdx.x] - lds.base[threadIdx.x];
+        }
+        __syncthreads();
+        for (u32 t0 = 0; t0 < d; t0 += kRadixBlock) {
+            const u32 i = t0 + threadIdx.x;
+            const bool valid = i < d;
+            u32 lo = 0, hi = 0, dg = 0;
+            if (valid) {
+                lo = src_lo[i];
+                hi = src_hi[i];
+                dg = digit_of(lo, hi, shift);
+            }
+            for (int k = threadIdx.x; k < kRadixWaves * 256; k += kRadixBlock) (&lds.wcnt[0][0])[k] = 0;
+            u64 peers = ballot(valid);
+#pragma unroll
+            for (int bit = 0; bit < 8; ++bit) {
+                const u64 m = ballot((dg >> bit) & 1);
+                peers &= ((dg >> bit) & 1) ? m : ~m;
+            }
+            const u32 rank = mask_rank(peers);
+            __syncthreads();
+            if (valid && rank == 0) lds.wcnt[wave][dg] = (u32)__popcll(peers);
+            __syncthreads();
+            if (threadIdx.x < 256) {
+                u32 run = lds.base[threadIdx.x];
+                for (int w = 0; w < kRadixWaves; ++w) {
+                    const u32 c = lds.wcnt[w][threadIdx.x];
+                    lds.wcnt[w][threadIdx.x] = run;
+                    run += c;
+                }
+                lds.base[threadIdx.x] = run;
+            }
+            __syncthreads();
+            if (valid) {
+                const u32 pos = lds.wcnt[wave][dg] + rank;
+                dst_lo[pos] = lo;
+                dst_hi[pos] = hi;
+            }
+            __syncthreads();
+        }
+    }
+    if ((npass + in_b) & 1) {  // result sits in the scratch pair: copy back
+        for (u32 i = threadIdx.x; i < d; i += kRadixBlock) {
+            a_lo[i] = b_lo[i];
+            a_hi[i] = b_hi[i];
+        }
+    }
+    __syncthreads();
+}
 __global__ __launch_bounds__(kRadixBlock) void sort_segments_radix(
     const Segment *__restrict__ segs, const u32 *__restrict__ nsegs, u32 *__restrict__ col, u32 *__restrict__ wbits,
     u32 *__restrict__ s_lo, u32 *__restrict__ s_hi, int col_passes) {
-    __shared__ u32 base[256];
-    __shared__ u32 wcnt[kRadixWaves][256];
-    const int wave = threadIdx.x / kWave;
-    const int npass = col_passes + 4;
+    __shared__ RadixLds lds;
     const u32 count = *nsegs;
-    for (u32 r = blockIdx.x; r < count; r += gridDim.x) {
-        const u32 d = segs[r].len;
-        u32 *a_lo = col + segs[r].at, *a_hi = wbits + segs[r].at;
-        u32 *b_lo = s_lo + segs[r].scratch, *b_hi = s_hi + segs[r].scratch;
-        const int in_b = (int)segs[r].in_scratch;
-        for (int pass = 0; pass < npass; ++pass) {
-            const bool from_b = (pass + in_b) & 1;
-            const int shift = pass < col_passes ? 8 * pass : 32 + 8 * (pass - col_passes);
-            const u32 *src_lo = from_b ? b_lo : a_lo, *src_hi = from_b ? b_hi : a_hi;
-            u32 *dst_lo = from_b ? a_lo : b_lo, *dst_hi = from_b ? a_hi : b_hi;
-            if (threadIdx.x < 256) base[threadIdx.x] = 0;
-            __syncthreads();
-            for (u32 i = threadIdx.x; i < d; i += kRadixBlock)
-                atomicAdd(&base[digit_of(src_lo[i], src_hi[i], shift)], 1u);
-            __syncthreads();
-            if (threadIdx.x < 256) {  // exclusive scan of the 256 bins, 4 waves
-                u32 x = base[threadIdx.x];
-                const u32 incl = wave_inclusive_scan(x);
-                wcnt[0][threadIdx.x] = incl;  // staging of wave-inclusive sums
-            }
-            __syncthreads();
-            if (threadIdx.x < 256) {
-                u32 add = 0;
-                for (int w = 0; w < (int)(threadIdx.x / kWave); ++w) add += wcnt[0][w * kWave + kWave - 1];
-                base[threadIdx.x] = add + wcnt[0][threadIdx.x] - base[threadIdx.x];
-            }
-            __syncthreads();
-            for (u32 t0 = 0; t0 < d; t0 += kRadixBlock) {
-                const u32 i = t0 + threadIdx.x;
-                const bool valid = i < d;
-                u32 lo = 0, hi = 0, dg = 0;
-                if (valid) {
-                    lo = src_lo[i];
-                    hi = src_hi[i];
-                    dg = digit_of(lo, hi, shift);
-                }
-                for (int k = threadIdx.x; k < kRadixWaves * 256; k += kRadixBlock) (&wcnt[0][0])[k] = 0;
-                u64 peers = ballot(valid);
-#pragma unroll
-                for (int bit = 0; bit < 8; ++bit) {
-                    const u64 m = ballot((dg >> bit) & 1);
-                    peers &= ((dg >> bit) & 1) ? m : ~m;
-                }
-                const u32 rank = mask_rank(peers);
-                __syncthreads();
-                if (valid && rank == 0) wcnt[wave][dg] = (u32)__popcll(peers);
-                __syncthreads();
-                if (threadIdx.x < 256) {
-                    u32 run = base[threadIdx.x];
-                    for (int w = 0; w < kRadixWaves; ++w) {
-                        const u32 c = wcnt[w][threadIdx.x];
-                        wcnt[w][threadIdx.x] = run;
-                        run += c;
-                    }
-                    base[threadIdx.x] = run;
-                }
-                __syncthreads();
-                if (valid) {
-                    const u32 pos = wcnt[wave][dg] + rank;
-                    dst_lo[pos] = lo;
-                    dst_hi[pos] = hi;
-                }
-                __syncthreads();
-            }
-        }
-        if ((npass + in_b) & 1) {  // result sits in the scratch pair: copy back
-            for (u32 i = threadIdx.x; i < d; i += kRadixBlock) {
-                a_lo[i] = b_lo[i];
-                a_hi[i] = b_hi[i];
+    for (u32 r = blockIdx.x; r < count; r += gridDim.x)
+        block_radix(lds, col + segs[r].at, wbits + segs[r].at, s_lo + segs[r].scratch, s_hi + segs[r].scratch,
+                    (int)segs[r].in_scratch, segs[r].len, col_passes);
+}
+
+// ------------------------------------------------------------- without lists
+// For arenas that hold the rows but not the lists of them beside the sort's
+// scratch (up to 32 bytes a vertex and 1 an entry in 20): a block walks `per`
+// rows, its waves sort those of 17..512 entries and the block the longer ones.
+struct UnlistedCounts {
+    u64 notisolated, huge_entries, scratch_used;
+};
+__global__ __launch_bounds__(256) void count_rows(const u64 *__restrict__ rs, u64 n, UnlistedCounts *k) {
+    u64 nonzero = 0, huge = 0;
+    for (u64 v = (u64)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (u64)gridDim.x * blockDim.x) {
+        const u64 d = rs[v + 1] - rs[v];
+        nonzero += d > 0;
+        huge += d > kSegBlock ? d : 0;
+    }
+    nonzero = wave_sum(nonzero);
+    huge = wave_sum(huge);
+    if (lane_id() == 0 && nonzero) atomicAdd((unsigned long long *)&k->notisolated, (unsigned long long)nonzero);
+    if (lane_id() == 0 && huge) atomicAdd((unsigned long long *)&k->huge_entries, (unsigned long long)huge);
+}
+
+constexpr u32 kUnlistedRows = 1024;  // at most, per block at a time
+__global__ __launch_bounds__(kSegThreads) void sort_rows_unlisted(const u64 *__restrict__ rs, u64 n, u32 per, u32 *col,
+                                                                  u32 *w, u32 *s_col, u32 *s_w, UnlistedCounts *k,
+                                                                  int col_passes) {
+    static_assert(kSegThreads == (u32)kRadixBlock, "one block shape for both sorts");
+    __shared__ u64 keys[kSegBlock];
+    __shared__ RadixLds radix;
+    __shared__ u32 longs[kUnlistedRows], nlongs;
+    __shared__ u64 place;
+    const u32 wave = threadIdx.x / kWave;
+    for (u64 v0 = (u64)blockIdx.x * per; v0 < n; v0 += (u64)gridDim.x * per) {
+        if (threadIdx.x == 0) nlongs = 0;
+        __syncthreads();
+        for (u32 r = wave; r < per && v0 + r < n; r += kSegThreads / kWave) {
+            const u64 b = rs[v0 + r], d = rs[v0 + r + 1] - b;
+            u32 *c = col + b, *x = w + b;
+            if (d > kLongRow) {
+                if (lane_id() == 0) longs[atomicAdd(&nlongs, 1u)] = r;
+            } else if (d > 256) {
+                wave_sort_segment<8>(c, x, c, x, (u32)d);
+            } else if (d > 64) {
+                wave_sort_segment<4>(c, x, c, x, (u32)d);
+            } else if (d > 16) {
+                wave_sort_segment<1>(c, x, c, x, (u32)d);
             }
         }
         __syncthreads();
+        for (u32 i = 0; i < nlongs; ++i) {
+            const u64 b = rs[v0 + longs[i]];
+            const u32 d = (u32)(rs[v0 + longs[i] + 1] - b);
+            if (d <= kSegBlock) {
+                block_sort(keys, col + b, w + b, col + b, w + b, d);
+            } else {
+                if (threadIdx.x == 0)
+                    place = atomicAdd((unsigned long long *)&k->scratch_used, (unsigned long long)d);
+                __syncthreads();
+                block_radix(radix, col + b, w + b, s_col + place, s_w + place, 0, d, col_passes);
+            }
+        }
+        __syncthreads();  // nlongs is set again for the next rows
     }
 }
 
@@ -1686,6 +1755,46 @@ static bool fill_partitioned(Worker_State *ws, const Tuple_Graph *tg, Oned_Graph
 // entries in long rows) 1088 / 928, S15 1359 / 1155, S16 1745 / 1393.
 constexpr u64 kLongMin = 1 << 17;
 
+// 8-bit digits of the columns.
+static int column_passes(u64 n) {
+    int bits = 1;
+    while (bits < 32 && (1ull << bits) < n) ++bits;
+    return (bits + 7) / 8;
+}
+
+// sort_rows in the least room: three counters, and a scratch for the rows above
+// kSegBlock entries.
+static bool sort_rows_without_lists(Worker_State *ws, Oned_Graph *g) {
+    Context &c = ctx();
+    const hipStream_t s = c.stream;
+    const u64 n = g->nlocalverts, mark = ws->gpu_arena.used;
+    u32 *col = g->column, *w = (u32 *)g->weights;
+    UnlistedCounts *k = (UnlistedCounts *)arena_alloc(ws, sizeof(UnlistedCounts), "sort counts");
+    if (failed()) return false;
+    G500_HIP(hipMemsetAsync(k, 0, sizeof(UnlistedCounts), s));
+    count_rows<<<grid_for(n, 256, (u64)c.num_cus * 16), 256, 0, s>>>(g->rowstarts, n, k);
+    G500_HIP(hipGetLastError());
+    UnlistedCounts h = {};
+    G500_HIP(hipMemcpyAsync(&h, k, sizeof(h), hipMemcpyDeviceToHost, s));
+    sync();
+    if (failed()) return false;
+    g->notisolated = h.notisolated;
+    u32 *s_col = nullptr, *s_w = nullptr;
+    if (h.huge_entries) {
+        s_col = (u32 *)arena_alloc(ws, h.huge_entries * sizeof(u32), "sort scratch");
+        s_w = (u32 *)arena_alloc(ws, h.huge_entries * sizeof(u32), "sort scratch");
+        if (failed()) return false;
+    }
+    const u64 blocks = (u64)c.num_cus * 2;
+    const u32 per = (u32)MAX((u64)1, MIN((u64)kUnlistedRows, n / (4 * blocks)));
+    sort_rows_thread<<<grid_for(n, 256, (u64)c.num_cus * 32), 256, 0, s>>>(g->rowstarts, n, col, g->weights);
+    sort_rows_unlisted<<<grid_for(n, (int)per, blocks), kSegThreads, 0, s>>>(g->rowstarts, n, per, col, w, s_col, s_w, k,
+                                                                            column_passes(n));
+    G500_HIP(hipGetLastError());
+    ws->gpu_arena.used = mark;
+    return !failed();
+}
+
 // Sorts every row by (weight bits, column) and counts the rows with entries.
 static bool sort_rows(Worker_State *ws, Oned_Graph *g) {
     Context &c = ctx();
@@ -1693,16 +1802,21 @@ static bool sort_rows(Worker_State *ws, Oned_Graph *g) {
     const u64 n = g->nlocalverts, m = g->nlocaledges;
     const u64 mark = ws->gpu_arena.used;
     u32 *col = g->column, *w = (u32 *)g->weights;
-    SortLists *L = (SortLists *)arena_alloc(ws, sizeof(SortLists) + 256, "sort lists");
+    auto room = [&]() { return ws->gpu_arena.reserved - MIN(ws->gpu_arena.used + 255, ws->gpu_arena.reserved); };
+    u64 caps[kWaveTiers], lists = sizeof(SortLists) + (kWaveTiers + 6) * 256;
+    for (int q = 0; q < kWaveTiers; ++q) lists += (caps[q] = tier_cap(n, m, q ? 32u << q : 17)) * sizeof(u32);
     TierLists t;
-    for (int q = 0; q < kWaveTiers; ++q)
-        t.rows[q] = (u32 *)arena_alloc(ws, tier_cap(n, m, q ? 32u << q : 17) * sizeof(u32), "sort tier");
     t.long_cap = tier_cap(n, m, kLongRow + 1);
+    const u64 block_cap = tier_cap(m, m, kLongRow + 1), radix_cap = tier_cap(m, m, kSegBlock + 1);
+    lists += t.long_cap * (2 * sizeof(u32) + sizeof(u64)) + (block_cap + radix_cap) * sizeof(Segment);
+    if (lists > room()) return sort_rows_without_lists(ws, g);
+    SortLists *L = (SortLists *)arena_alloc(ws, sizeof(SortLists) + 256, "sort lists");
+    for (int q = 0; q < kWaveTiers; ++q) t.rows[q] = (u32 *)arena_alloc(ws, caps[q] * sizeof(u32), "sort tier");
     t.long_row = (u32 *)arena_alloc(ws, t.long_cap * sizeof(u32), "long rows");
     t.long_len = (u32 *)arena_alloc(ws, t.long_cap * sizeof(u32), "long row lengths");
     t.long_off = (u64 *)arena_alloc(ws, t.long_cap * sizeof(u64), "long row offsets");
-    Segment *block_segs = (Segment *)arena_alloc(ws, tier_cap(m, m, kLongRow + 1) * sizeof(Segment), "block segments");
-    Segment *radix_segs = (Segment *)arena_alloc(ws, tier_cap(m, m, kSegBlock + 1) * sizeof(Segment), "radix segments");
+    Segment *block_segs = (Segment *)arena_alloc(ws, block_cap * sizeof(Segment), "block segments");
+    Segment *radix_segs = (Segment *)arena_alloc(ws, radix_cap * sizeof(Segment), "radix segments");
     if (failed()) return false;
     u32 *error = (u32 *)(L + 1);
     G500_HIP(hipMemsetAsync(L, 0, sizeof(SortLists) + 256, s));
@@ -1713,6 +1827,10 @@ static bool sort_rows(Worker_State *ws, Oned_Graph *g) {
     G500_HIP(hipMemcpyAsync(&h, L, sizeof(h), hipMemcpyDeviceToHost, s));
     sync();
     if (failed()) return false;
+    if (2 * (MAX(h.huge_entries.v, (u64)1) * sizeof(u32) + 256) > room()) {
+        ws->gpu_arena.used = mark;
+        return sort_rows_without_lists(ws, g);
+    }
     g->notisolated = h.notisolated.v;
     TierCounts k;
     u64 nwave = 0;
@@ -1730,8 +1848,7 @@ static bool sort_rows(Worker_State *ws, Oned_Graph *g) {
         a.col = col;
         a.w = w;
         const u64 per_chunk = 3 * sizeof(u32) + sizeof(u64), slack = 16 * 256 + scan_tile_bytes(a.nchunks);
-        const u64 room = ws->gpu_arena.reserved - ws->gpu_arena.used;
-        const bool bins = h.long_entries.v >= kLongMin && h.long_entries.v * 8 + a.nchunks * per_chunk + a.nrows * 8 + slack <= room;
+        const bool bins = h.long_entries.v >= kLongMin && h.long_entries.v * 8 + a.nchunks * per_chunk + a.nrows * 8 + slack <= room();
         const u64 scratch = MAX(bins ? h.long_entries.v : h.huge_entries.v, (u64)1);
         a.s_col = (u32 *)arena_alloc(ws, scratch * sizeof(u32), "sort scratch");
         a.s_w = (u32 *)arena_alloc(ws, scratch * sizeof(u32), "sort scratch");
@@ -1768,12 +1885,9 @@ static bool sort_rows(Worker_State *ws, Oned_Graph *g) {
         const u64 most_radix = bins ? tier_cap(a.nchunks, h.long_entries.v, kSegBlock + 1) : a.nrows;
         sort_segments_block<<<(unsigned)MIN(most_block, (u64)c.num_cus * 4), kSegThreads, 0, s>>>(
             block_segs, &L->nblock.v, col, w, a.s_col, a.s_w);
-        if (bins || h.huge_entries.v) {
-            int bits = 1;
-            while (bits < 32 && (1ull << bits) < n) ++bits;
+        if (bins || h.huge_entries.v)
             sort_segments_radix<<<(unsigned)MIN(most_radix, (u64)c.num_cus * 2), kRadixBlock, 0, s>>>(
-                radix_segs, &L->nradix.v, col, w, a.s_col, a.s_w, (bits + 7) / 8);
-        }
+                radix_segs, &L->nradix.v, col, w, a.s_col, a.s_w, column_passes(n));
     }
     G500_HIP(hipGetLastError());
     ws->gpu_arena.used = mark;  // release the scratch

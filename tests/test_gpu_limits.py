@@ -107,3 +107,42 @@ def test_rows_of_more_bins_than_one_round(arena, oracle, entries):
     e, w = np.concatenate([e, second]), np.concatenate([w, rng.random(600).astype(np.float32)])
     g, ref = build(arena, n, e, w)
     csr_equal(arena, g, ref)
+
+
+def round256(x):
+    return (x + 255) // 256 * 256
+
+
+# A construction of rows alone needs, beside the CSR, 24 bytes a vertex for the sort's
+# lists and 8 an entry of rows above 4096 for its scratch, each array rounded to 256
+# bytes. Many entries per vertex (lists by entries would need more than that), rows of
+# every tier; with hubs, whose scratch is most of the room.
+@pytest.mark.parametrize("hubs", [0, 3])
+def test_rows_in_the_smallest_arena(arena, oracle, hubs):
+    rng = np.random.default_rng(hubs)
+    n = 3000
+    deg = np.concatenate([rng.integers(600, 1500, 1700), rng.integers(0, 40, 600), rng.integers(40, 500, 695),
+                          np.full(hubs, 60000), np.full(5 - hubs, 1)])
+    e = np.stack([np.repeat(np.arange(n), deg), rng.integers(0, n, deg.sum())], 1)
+    if not hubs:  # every row at most 4096 entries
+        assert np.bincount(e.ravel(), minlength=n).max() <= 4096
+    w = rng.random(len(e)).astype(np.float32)
+    tg = arena.upload_tuples(e, w)
+    ref = oracle.csr(n, e.astype(np.uint64), w)
+    degree = np.diff(ref.rowstarts.astype(np.int64))
+    m, huge = int(degree.sum()), int(degree[degree > 4096].sum())
+    assert (huge > 0) == (hubs > 0)
+    need = round256(8 * (n + 1)) + 2 * round256(4 * m)
+    need += 4 * round256(4 * n) + round256(8 * n) + 256 + 2 * round256(4 * huge)
+    a, saved, old = arena.ws.gpu_arena, arena.ws.gpu_arena.reserved, arena.get_param("relabel")
+    arena.set_param("relabel", 0)
+    a.reserved = round256(a.used) + need
+    try:
+        g = arena.csr(tg, n)
+        mark = a.used
+    finally:
+        a.reserved = saved
+        arena.set_param("relabel", old)
+    assert g.notisolated == int((degree > 0).sum())
+    assert mark <= g.weights + 4 * m - a.base + 255  # the scratch is released
+    csr_equal(arena, g, ref)
