@@ -1457,21 +1457,24 @@ void build_sssp_copy(Worker_State *ws, Oned_Graph *g, u64 nlong, u64 ntop) {
     const u64 kept_bytes = bits_bytes + off_bytes, count_bytes = align(ntiles * sizeof(u32)) + align(scan_tile_bytes(ntiles));
     const u64 table_bytes = align(n * kPruneHubs * sizeof(u32)), quant_bytes = align(n * kPruneHubs);
     const u64 entry_bytes = 2 * align(MAX(m, (u64)1) * sizeof(u32));
-    auto need = [&](u64 quant) {
-        return align((n + 1) * 8) + MAX(entry_bytes, kept_bytes + count_bytes + quant) + MAX(table_bytes, kept_bytes) + 1024;
-    };
-    // The copy is an optimization: without arena room for its largest moment
-    // (and a reserve of 8 bytes a vertex and 8 MiB) the graph keeps none, and
-    // SSSP relaxes the traversal copy. The 8-bit table fits beside that moment
-    // except on graphs of fewer than 5 entries a vertex.
-    const u64 room = ws->gpu_arena.reserved - ws->gpu_arena.used;
-    const u64 least = MAX(need(0), (n + 1) * 8 + m * 8 + n * kPruneHubs * 4 + n * 8 + (8u << 20));
-    if (least > room) {
+    // The copy is an optimization: without arena room for row offsets, entries
+    // at full size and the hub table (and a reserve of 8 bytes a vertex and
+    // 8 MiB) the graph keeps none, and SSSP relaxes the traversal copy. The bits
+    // and their counts always fit in that room, the 8-bit table beside them
+    // except on graphs of fewer than 5 entries a vertex. On graphs of hundreds of
+    // entries a vertex, whose bits outgrow the hub table, the room left for the
+    // entries may be less than full size: the kept ones are held against it.
+    const u64 start = ws->gpu_arena.used, room = ws->gpu_arena.reserved - start;
+    const u64 least = (n + 1) * 8 + m * 8 + n * kPruneHubs * 4 + n * 8 + (8u << 20);
+    auto no_room = [&](u64 bytes) {
         fprintf(stderr, "libg500: no arena room for the SSSP copy (%llu bytes); SSSP relaxes the traversal copy\n",
-                (unsigned long long)least);
-        return;
-    }
-    const bool quantised = need(quant_bytes) <= room;
+                (unsigned long long)bytes);
+        ws->gpu_arena.used = start;
+    };
+    if (least > room) return no_room(least);
+    const u64 high_bytes = MAX(table_bytes, kept_bytes);
+    const u64 low_room = room - (align((n + 1) * 8) + high_bytes + 1024);
+    const bool quantised = kept_bytes + count_bytes + quant_bytes <= low_room;
     // the hubs: the kPruneHubs largest degrees among the first max(ntop, kPruneHubs)
     // rows (every later row is no longer), ties to the smaller id
     const u64 nhead = MIN(n, MAX(ntop, (u64)kPruneHubs));
@@ -1496,8 +1499,9 @@ void build_sssp_copy(Worker_State *ws, Oned_Graph *g, u64 nlong, u64 ntop) {
     if (failed()) return;
     const u64 mark = ws->gpu_arena.used;
     const u64 quant_used = quantised ? quant_bytes : 0;
-    u8 *low = (u8 *)arena_alloc(ws, MAX(entry_bytes, kept_bytes + count_bytes + quant_used), "SSSP prune scratch");
-    u8 *high = (u8 *)arena_alloc(ws, MAX(table_bytes, kept_bytes), "SSSP prune hub table");
+    const u64 low_bytes = MIN(low_room, MAX(entry_bytes, kept_bytes + count_bytes + quant_used));
+    u8 *low = (u8 *)arena_alloc(ws, low_bytes, "SSSP prune scratch");
+    u8 *high = (u8 *)arena_alloc(ws, high_bytes, "SSSP prune hub table");
     if (failed()) return;
     u64 *bits = (u64 *)low, *tile_off = (u64 *)(low + bits_bytes);
     u32 *counts = (u32 *)(low + kept_bytes);
@@ -1523,6 +1527,8 @@ void build_sssp_copy(Worker_State *ws, Oned_Graph *g, u64 nlong, u64 ntop) {
     G500_HIP(hipMemcpyAsync(high, low, kept_bytes, hipMemcpyDeviceToDevice, s));
     sync();
     if (failed()) return;
+    const u64 kept_entries = 2 * align(MAX(m_s, (u64)1) * sizeof(u32));
+    if (kept_entries > low_bytes) return no_room(kept_entries - low_bytes + room);
     ws->gpu_arena.used = mark;
     u32 *col_s = (u32 *)arena_alloc(ws, MAX(m_s, (u64)1) * sizeof(u32), "SSSP columns");
     f32 *w_s = (f32 *)arena_alloc(ws, MAX(m_s, (u64)1) * sizeof(f32), "SSSP weights");

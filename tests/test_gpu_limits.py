@@ -146,3 +146,34 @@ def test_rows_in_the_smallest_arena(arena, oracle, hubs):
     assert g.notisolated == int((degree > 0).sum())
     assert mark <= g.weights + 4 * m - a.base + 255  # the scratch is released
     csr_equal(arena, g, ref)
+
+
+# The SSSP copy is built where 8 bytes an entry and 144 a vertex and 8 MiB are
+# free beside the traversal copy, also where the entries are so many (40000 a
+# vertex) that the bits of the kept ones, 1/7 byte each with their offsets, are
+# more than the hub table.
+def test_sssp_copy_of_a_dense_graph_in_little_room(arena):
+    scale = 11
+    n = 1 << scale
+    tg = arena.generate(scale, 20000)
+    a, saved, m0 = arena.ws.gpu_arena, arena.ws.gpu_arena.reserved, arena.mark()
+    kept = []  # entries kept per original vertex
+    for tight in (False, True):
+        arena.release(m0)
+        if tight:
+            m = int(g.nlocaledges)
+            rows = round256(8 * (n + 1)) + 2 * round256(4 * m)
+            traversal = 2 * round256(4 * n) + round256(8 * (n + 1)) + 2 * round256(4 * m)
+            a.reserved = round256(a.used) + rows + traversal + 256 + 8 * (n + 1) + 8 * m + 136 * n + (8 << 20)
+        try:
+            g = arena.csr(tg, n)
+        finally:
+            a.reserved = saved
+        assert g.rowstarts_s, tight
+        rs = arena.to_host(g.rowstarts_s, n + 1, np.uint64).astype(np.int64)
+        kept.append(np.diff(rs)[arena.to_host(g.perm, n, np.uint32)])
+    assert np.array_equal(*kept) and kept[0].sum() < m
+    s = arena.sssp_create(g, 0.1)
+    root = int(arena.roots(g)[0])
+    arena.sssp(g, s, root)
+    assert arena.sssp_check(g, s.dist, s.pred, root) == 0
