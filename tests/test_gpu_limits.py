@@ -177,3 +177,60 @@ def test_sssp_copy_of_a_dense_graph_in_little_room(arena):
     root = int(arena.roots(g)[0])
     arena.sssp(g, s, root)
     assert arena.sssp_check(g, s.dist, s.pred, root) == 0
+
+
+# Persistent kernels on every block that the device holds, with small blocks: the
+# grid barrier's largest member counts. Grids follow the work (entries / 512 or
+# 256, times roots), and S24's fills the device at these shapes: plain BFS
+# sqrt(5.3e8 / 512) x 512 / 128 = 4060 blocks wanted of 128 threads where 3072 are
+# resident, 2030 of 256 where 1536 are; the others hold fewer.
+@pytest.fixture(scope="module")
+def s24():
+    import g500
+    s = g500.Session(arena_bytes=64 << 30)
+    g = s.csr(s.generate(24), 1 << 24)
+    yield s, g, s.roots(g)[:6]
+    s.close()
+
+
+KNOBS = ("bfs_block", "sssp_block", "batch_bfs_block", "batch_sssp_block")
+
+
+def traversals(s, g, roots):
+    """Depths and distances by each of the four kernels."""
+    m, out, some = s.mark(), [], (0, len(roots) - 1)
+    b, p = s.bfs_create(g), s.sssp_create(g, 0.1)
+    for i in some:
+        s.bfs(g, b, roots[i])
+        assert s.bfs_validate(g, b, roots[i]) == (True, 0)
+        out.append(s.bfs_depth(g, b, roots[i]))
+        s.sssp(g, p, roots[i])
+        assert s.sssp_check(g, p.dist, p.pred, roots[i]) == 0
+        out.append(s.sssp_result(p)[0].view(np.uint32))
+    s.release(m)
+    bb = s.batch_create(g)
+    s.batch(g, bb, roots)
+    out += [s.batch_depth(g, bb, i) for i in some]
+    s.release(m)
+    sb = s.sssp_batch_create(g, 0.05)
+    s.sssp_batch(g, sb, roots)
+    out += [s.sssp_batch_result(g, sb, i)[0].view(np.uint32) for i in some]
+    s.release(m)
+    return out
+
+
+def test_small_blocks_on_the_whole_device(s24):
+    s, g, roots = s24
+    old = {k: s.get_param(k) for k in KNOBS}
+    want = traversals(s, g, roots)
+    for i in (0, 2):  # the batched kernels agree with the plain ones
+        assert np.array_equal(want[i], want[4 + i // 2]) and np.array_equal(want[i + 1], want[6 + i // 2])
+    try:
+        for block in (128, 256):
+            for k in KNOBS:
+                s.set_param(k, block)
+            for k, (x, y) in enumerate(zip(want, traversals(s, g, roots))):
+                assert np.array_equal(x, y), (block, k)
+    finally:
+        for k, v in old.items():
+            s.set_param(k, v)
