@@ -706,7 +706,7 @@ bool bfs_batch_enqueue(const Oned_Graph *g, Bfs_Batch_State *b, const u64 *roots
     a.hub_degree = (u32)c.bfs_hub_degree;
     const int block = ctx().batch_bfs_block;
     if (grid <= 0) grid = cooperative_blocks((const void *)batch_bfs_kernel, block, 0);
-    grid = persistent_grid(a.m_total / 256, grid, block);
+    grid = persistent_grid((a.m_total + 2 * n) / 256, grid, block);
     if (failed()) return false;
     a.heavy_degree = c.batch_heavy_degree == kHeavyAuto ? (u32)heavy_bound(n, (u64)grid * (u64)block / kWave)
                                                         : (u32)c.batch_heavy_degree;

@@ -530,8 +530,8 @@ void oned_graph_bfs_run(Worker_State *ws, const Oned_Graph *g, Bfs_State *bfs, u
     a.beta = (f32)c.bfs_beta;
     a.hub_degree = (u32)c.bfs_hub_degree;
     const int block = ctx().bfs_block;
-    const int grid =
-        persistent_grid(a.m_total / 512, cooperative_blocks((const void *)bfs_kernel, block, 0), block);
+    const int grid = persistent_grid((a.m_total + 8 * g->notisolated) / 512,
+                                     cooperative_blocks((const void *)bfs_kernel, block, 0), block);
     if (failed()) return;
     void *args[] = {&a};
     G500_HIP(hipMemsetAsync(bfs->ctl, 0, sizeof(BfsCtl), c.stream));

@@ -112,18 +112,29 @@ inline void sync() { G500_HIP(hipStreamSynchronize(ctx().stream)); }
 // the CU's LDS without allocation rounding is never taken.
 int cooperative_blocks(const void *kernel, int block, size_t dyn_lds);
 
-// Grid of a persistent kernel for a launch of `work` (entries times roots, in
-// units that take a block about as long as a barrier takes per block): at most
-// `full`, the co-resident grid of `block` threads. Every step costs its share
-// of the work, which falls with the blocks, and a barrier, which grows with
-// them (2.6 us at 32 blocks of 512 threads, 6.7 us at 512), so the best grid
-// grows with the square root of the work. Measured on Kronecker graphs, us at
-// 16 / 32 / 64 / 128 / 256 / 512 blocks: SSSP S12 432 / 435 / 446 / 469 / 516 / 606,
-// S16 1089 / 928 / 879 / 931 / 994 / 1158, S20 - / 4217 / 3033 / 2344 / 2131 / 2257,
-// S22 - / - / 12151 / 7865 / 5422 / 4806; BFS S12 104 / 105 / 108 / 111 / 124 / 143,
-// S20 - / 547 / 401 / 348 / 369 / 418; batched SSSP, 32 roots, S12
-// 5595 / 5238 / 5135 / 5214 / 5719 / 6848, S20 - / - / 54580 / 38302 / 31711 / 29702;
-// batched BFS S16 1073 / 873 / 779 / 776 / 803 / 849, S22 - / - / 13815 / 7318 / 4217 / 3389.
+// Grid of a persistent kernel for a launch of `work` (in units that take a
+// block about as long as a barrier takes per block): at most `full`, the
+// co-resident grid of `block` threads. Every step costs its share of the work,
+// which falls with the blocks, and a barrier, which grows with them (2.6 us at
+// 32 blocks of 512 threads, 6.7 us at 512), so the best grid grows with the
+// square root of the work. Work is entries (times roots) and vertices: a
+// vertex costs several entries when its labels are cleared, scanned or relaxed,
+// which decides on graphs of few entries a vertex. Measured, us at
+// 16 / 32 / 64 / 128 / 256 / 512 blocks (SSSP up to 256 the roomy build):
+// SSSP S12 326 / 308 / 312 / 329 / 359 / 472, S16 728 / 655 / 645 / 641 / 705 / 860,
+// S20 - / - / 2266 / 1800 / 1598 / 1865, S22 - / - / - / 4517 / 3209 / 3128,
+// 2e6 uniform edges over 2e6 vertices 14118 / 8305 / 5454 / 4166 / 3746 / 4449, 1e5
+// over 8e6 - / - / 215 / 142 / 111 / 185;
+// BFS S12 67 / 68 / 71 / 73 / 80 / 99, S20 - / - / 338 / 260 / 252 / 316, S22
+// - / - / - / 363 / 297 / 343, 2e6 over 2e6 5287 / 2823 / 1577 / 1069 / 1019 / 1343;
+// batched SSSP, 32 roots, S12 4363 / 4033 / 3988 / 4039 / 4336 / 5307, S20
+// - / - / - / 35820 / 28837 / 27609, one root 2e6 over 2e6
+// 95807 / 57411 / 37961 / 28438 / 24659 / 28396; batched BFS, 64 roots, S16
+// 888 / 726 / 652 / 655 / 679 / 705, S22 - / - / - / 4943 / 3302 / 3012, 1e5 over 8e6
+// - / - / 142 / 101 / 91 / 98.
+// Graphs that take few steps for their size want more blocks than any rule on
+// sizes gives (64 vertices joined to 5e5 by 3e6 edges, BFS from one of the 64 in
+// four levels: 816 at 144 blocks, 558 at 512).
 int persistent_grid(u64 work, int full, int block);
 
 // Kernel and grid of a persistent kernel that is built for four waves a SIMD

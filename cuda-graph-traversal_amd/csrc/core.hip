@@ -94,19 +94,23 @@ int cooperative_blocks(const void *kernel, int block, size_t dyn_lds) {
 
 int persistent_grid(u64 work, int full, int block) {
     // whole rounds over 8 XCDs; smaller blocks in proportion more
-    const f64 blocks = std::sqrt((f64)work) * 512.0 / block;
-    return (int)std::min<f64>(full, 8.0 * std::ceil(std::max(blocks, 1.0) / 8.0));
+    f64 blocks = 8.0 * std::ceil(std::max(std::sqrt((f64)work) * 512.0 / block, 1.0) / 8.0);
+    // a few blocks more than whole rounds over the CUs would only add a second (third) block to some of them
+    const f64 cus = ctx().num_cus * 512.0 / block, over = std::fmod(blocks, cus);
+    if (blocks > cus && over < cus / 2) blocks -= over;
+    return (int)std::min<f64>(full, blocks);
 }
 
 // The SSSP kernels hold about 200 registers a lane where four waves on a SIMD
 // get 128 each, and spill the rest; two waves a SIMD spill nothing but are half
 // as many. A grid that needs no more than the roomy blocks loses nothing by
 // them, and a somewhat larger one less than the spills cost it. us, packed ->
-// roomy, by the blocks wanted: SSSP S12 338 -> 316, S16 695 -> 675, S19 1555 ->
-// 1490; batched, 7 roots S12 (16 blocks) 1850 -> 1690, 32 roots S16 (256) 5690 ->
-// 5400, 7 roots S19 (344) 8360 -> 7920; past the line 32 roots over 300001
-// uniform vertices (416) 6450 -> 6880, 16 roots S19 (512) 6650 -> 7370, 32 roots
-// S22 35300 -> 41000.
+// roomy: SSSP S12 (32 blocks wanted) 342 -> 308, S16 (72) 684 -> 645, S20 1705 at 256
+// -> 1598; batched, 7 roots S12 (40) 2493 -> 2252, 7 roots S18 (264) 5099 at 256 ->
+// 4774, 32 roots S16 (264) 7737 at 256 -> 7375. Past the line, packed at 512 ->
+// roomy at 256: SSSP S22 3128 -> 3209, 32 roots over 300001 uniform vertices (472)
+// 7162 -> 7995, 32 roots S20 27600 -> 28800, 32 roots S22 57800 -> 68400; but 7
+// roots S20 12425 -> 11749.
 PersistentLaunch pick_persistent(const void *packed, const void *roomy, u64 work, int block, size_t dyn_lds) {
     const int want = persistent_grid(work, 1 << 30, block);
     const int most = cooperative_blocks(roomy, block, dyn_lds);

@@ -1252,7 +1252,7 @@ void oned_graph_sssp_run(Worker_State *ws, const Oned_Graph *g, Sssp_State *s, u
     a.dbound = g->rowstarts_s ? kPruneDistBound : __builtin_inff();
     const int block = ctx().sssp_block;
     const PersistentLaunch pl = pick_persistent((const void *)sssp_kernel<4>, (const void *)sssp_kernel<2>,
-                                                g->nlocaledges / 512, block, 0);
+                                                (g->nlocaledges + 8 * a.n) / 512, block, 0);
     if (failed()) return;
     void *args[] = {&a};
     G500_HIP(hipMemsetAsync(s->ctl, 0, sizeof(SsspCtl), c.stream));

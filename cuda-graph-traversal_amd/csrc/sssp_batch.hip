@@ -1797,7 +1797,7 @@ void sssp_batch_lags(const f32 *offsets, i32 nroots, f32 delta, u32 *lag, f32 *u
 static PersistentLaunch pick_launch(const Oned_Graph *g, i32 nroots, int grid) {
     const int block = ctx().batch_sssp_block;
     const void *packed = (const void *)sssp_batch_kernel<4>, *roomy = (const void *)sssp_batch_kernel<2>;
-    const u64 work = g->nlocaledges * (u64)nroots / 1024;
+    const u64 work = (g->nlocaledges * (u64)(nroots + 1) + 32 * g->notisolated) / 1024;
     // slots share the CUs: their share was counted in packed blocks
     if (grid > 0) return {packed, persistent_grid(work, grid, block), grid};
     return pick_persistent(packed, roomy, work, block, q_lds_bytes(block));

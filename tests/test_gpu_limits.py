@@ -234,3 +234,38 @@ def test_small_blocks_on_the_whole_device(s24):
     finally:
         for k, v in old.items():
             s.set_param(k, v)
+
+
+# A launch's blocks follow the vertices as well as the entries: with an entry per 40
+# vertices a launch is a pass over per-vertex arrays, about as much as a copy of 32
+# bytes a vertex (the labels, probes, stamps and row records that SSSP touches; the
+# batched BFS touches less). Both within twice that; 4 and 2.2 times with the 24 and
+# 32 blocks that the entries alone ask for.
+def test_few_entries_over_many_vertices(arena, oracle):
+    n = 8 * 10**6
+    e = np.random.default_rng(3).integers(0, n, (10**5, 2))
+    g, ref = build(arena, n, e)
+    root = int(e[0, 0])
+    m = arena.mark()
+    size = 32 * n
+    src = arena.lib._worker_arena_push_array(arena.ws, size, 1, 256, None)
+    dst = arena.lib._worker_arena_push_array(arena.ws, size, 1, 256, None)
+
+    def best(run):
+        run()
+        return min(run() for _ in range(5))
+
+    def copy():
+        arena.lib.g500_copy_device(dst, src, size)
+        return arena.lib.g500_last_run_ms()
+
+    ms = {"copy": best(copy)}
+    arena.release(m)
+    s, b = arena.sssp_create(g), arena.batch_create(g)
+    ms["sssp"] = best(lambda: arena.sssp(g, s, root))
+    ms["batch"] = best(lambda: arena.batch(g, b, np.array([root], np.uint64)))
+    print(f"[few entries] {ms}", flush=True)
+    want = oracle.dijkstra_f32(ref, root)[0]
+    assert np.array_equal(arena.sssp_result(s)[0].view(np.uint32), want.view(np.uint32))
+    assert np.array_equal(arena.batch_depth(g, b, 0), oracle.bfs(ref, root)[1])
+    assert max(ms["sssp"], ms["batch"]) < 2 * ms["copy"]
