@@ -43,10 +43,28 @@ __global__ __launch_bounds__(256) void validate_init_kernel(const i64 *__restric
 
 __device__ __forceinline__ i64 wrap_inc(i64 x) { return (i64)((u64)x + 1u); }
 
+// The row v whose slots hold slot k of the rows and their entries laid end to
+// end (row v's own slot is rs[v] + v, its entries' slots follow), for k < n + m.
+// All lanes search: 64 splits a round, four rounds up to 2^24 rows.
+__device__ __forceinline__ u64 row_of_slot(const u64 *rs, u64 n, u64 k) {
+    u64 lo = 0, hi = n;
+    while (hi - lo > 1) {
+        const u64 step = (hi - lo + kWave - 1) / kWave, v = lo + lane_id() * step;
+        const u64 below = ballot(v < hi && rs[v] + v <= k);  // a run of lanes from lane 0 on
+        lo += ((u64)__popcll(below) - 1) * step;
+        hi = min(lo + step, hi);
+    }
+    return lo;
+}
+
 // Rules 3-6 over every CSR entry (graph500_runner.cu:111-153). A wave takes
-// `per` source rows; 8 lanes walk each row of up to kValidateLong entries,
-// eight rows at a time, and the whole wave each longer one, with kValidateSteps
+// `span` slots of the rows and their entries laid end to end: it walks the rows
+// up to kValidateLong entries that start there, 8 lanes a row and eight rows at
+// a time, and the pieces there of longer rows, all lanes, with kValidateSteps
 // entries of a lane in flight: their depths are random reads, which bound it.
+// Rows by number instead would leave rows of hubs that follow each other to one
+// wave: validating 64 vertices joined to 5e5 others by 3e6 edges took 6.9 ms, now
+// 0.15, a star of 3e6 14.8, now 0.30, S20 0.93, now 0.40.
 // The reference also confirms d from an entry (s, d) with pred[d] == s; the
 // rows are symmetric, so d's own row holds s and confirms it there, and the
 // entries' parents need no reads. 700001 uniform vertices, 15.4e6 entries:
@@ -56,7 +74,7 @@ constexpr int kValidateSteps = 4;
 __global__ __launch_bounds__(256) void validate_edges_kernel(const u64 *__restrict__ rs, const u32 *__restrict__ col,
                                                              const i64 *__restrict__ pred, const i64 *__restrict__ dist,
                                                              u32 *__restrict__ confirmed, u64 *__restrict__ errors, u64 n,
-                                                             u32 per) {
+                                                             u64 slots, u64 span) {
     const u32 lane = lane_id();
     const u64 wave = ((u64)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
     const u64 nw = (u64)gridDim.x * blockDim.x / kWave;
@@ -89,32 +107,40 @@ __global__ __launch_bounds__(256) void validate_edges_kernel(const u64 *__restri
         }
         return self_ok;
     };
-    for (u64 s0 = wave * per; s0 < n; s0 += nw * per) {
-        const u64 s = s0 + lane;
-        const bool mine = lane < per && s < n;
-        const i64 sp = mine ? pred[s] : -1, sd = mine ? dist[s] : -1;
-        const u64 b = mine ? rs[s] : 0;
-        const u32 len = mine ? (u32)(rs[s + 1] - b) : 0;
-        for (u64 todo = ballot(len > 0 && len <= kValidateLong); todo;) {
-            int j = -1;
+    for (u64 k0 = wave * span; k0 < slots; k0 += nw * span) {
+        const u64 k1 = min(k0 + span, slots);
+        bool more = true;
+        for (u64 s0 = row_of_slot(rs, n, k0); more; s0 += kWave) {
+            const u64 s = s0 + lane;
+            const u64 b = s < n ? rs[s] : 0, at = b + s;  // the row's own slot
+            const bool mine = s < n && at < k1;
+            const u32 len = mine ? (u32)(rs[s + 1] - b) : 0;
+            const i64 sp = mine ? pred[s] : -1, sd = mine ? dist[s] : -1;
+            more = ballot(mine) == ~0ull;
+            for (u64 todo = ballot(at >= k0 && len > 0 && len <= kValidateLong); todo;) {
+                int j = -1;
 #pragma unroll
-            for (u32 q = 0; q < 8; ++q) {
-                const int jq = todo ? __ffsll((unsigned long long)todo) - 1 : -1;
-                todo &= todo - 1;
-                if (lane >> 3 == q) j = jq;
+                for (u32 q = 0; q < 8; ++q) {
+                    const int jq = todo ? __ffsll((unsigned long long)todo) - 1 : -1;
+                    todo &= todo - 1;
+                    if (lane >> 3 == q) j = jq;
+                }
+                const int js = j < 0 ? 0 : j;
+                const u32 lj = __shfl(len, js);
+                const bool ok = walk(s0 + js, (i64)shfl64((u64)sp, js), (i64)shfl64((u64)sd, js), shfl64(b, js),
+                                     j < 0 ? 0 : lj, lane & 7u, 8);
+                const u32 any = (u32)(ballot(ok) >> (lane & ~7u)) & 0xFFu;
+                if (any && (lane & 7u) == 0) confirm(confirmed, s0 + js);
             }
-            const int js = j < 0 ? 0 : j;
-            const u32 lj = __shfl(len, js);
-            const bool ok = walk(s0 + js, (i64)shfl64((u64)sp, js), (i64)shfl64((u64)sd, js), shfl64(b, js),
-                                 j < 0 ? 0 : lj, lane & 7u, 8);
-            const u32 any = (u32)(ballot(ok) >> (lane & ~7u)) & 0xFFu;
-            if (any && (lane & 7u) == 0) confirm(confirmed, s0 + js);
-        }
-        for (u64 todo = ballot(len > kValidateLong); todo; todo &= todo - 1) {
-            const int j = __ffsll((unsigned long long)todo) - 1;
-            const bool ok = walk(s0 + j, (i64)shfl64((u64)sp, j), (i64)shfl64((u64)sd, j), shfl64(b, j), __shfl(len, j),
-                                 lane, kWave);
-            if (ballot(ok) && lane == 0) confirm(confirmed, s0 + j);
+            for (u64 todo = ballot(len > kValidateLong); todo; todo &= todo - 1) {
+                const int j = __ffsll((unsigned long long)todo) - 1;
+                const u64 first = shfl64(at, j) + 1;  // the first entry's slot
+                const u64 from = max(k0, first) - first, to = min(k1 - min(k1, first), (u64)__shfl(len, j));
+                if (from >= to) continue;
+                const bool ok = walk(s0 + j, (i64)shfl64((u64)sp, j), (i64)shfl64((u64)sd, j), shfl64(b, j) + from,
+                                     (u32)(to - from), lane, kWave);
+                if (ballot(ok) && lane == 0) confirm(confirmed, s0 + j);
+            }
         }
     }
     err = wave_sum(err);
@@ -273,12 +299,14 @@ static u64 validate_enqueue(const Oned_Graph *g, const i64 *pred, const i64 *dis
     const u64 n = g->nlocalverts, nwords = (n + 31) / 32;
     const hipStream_t s = c.stream;
     const unsigned gv = grid_for(n, 256, (u64)c.num_cus * 32);
-    u32 per = kWave;  // source rows per wave, fewer on graphs that would leave waves idle
-    while (per > 1 && n / per < (u64)c.num_cus * 32) per /= 2;
-    const unsigned ge = grid_for((n + per - 1) / per * kWave, 256, (u64)c.num_cus * 32);
+    const u64 slots = n + g->nlocaledges;
+    u64 span = 1 << 16;  // less on graphs that would leave waves idle
+    while (span > 128 && slots / span < (u64)c.num_cus * 32) span /= 2;
+    const unsigned ge = grid_for((slots + span - 1) / span * kWave, 256, (u64)c.num_cus * 32);
     validate_clear_kernel<<<grid_for(nwords, 256, (u64)c.num_cus * 8), 256, 0, s>>>(confirmed, nwords, errors);
     validate_init_kernel<<<gv, 256, 0, s>>>(pred, dist, confirmed, errors, n, root);
-    validate_edges_kernel<<<ge, 256, 0, s>>>(g->rowstarts, g->column, pred, dist, confirmed, errors, n, per);
+    validate_edges_kernel<<<ge, 256, 0, s>>>(g->rowstarts, g->column, pred, dist, confirmed, errors, n, slots,
+                                            span);
     validate_confirmed_kernel<<<gv, 256, 0, s>>>(pred, dist, confirmed, errors, n, root);
     G500_HIP(hipGetLastError());
     u64 h = 0;

@@ -269,3 +269,51 @@ def test_few_entries_over_many_vertices(arena, oracle):
     assert np.array_equal(arena.sssp_result(s)[0].view(np.uint32), want.view(np.uint32))
     assert np.array_equal(arena.batch_depth(g, b, 0), oracle.bfs(ref, root)[1])
     assert max(ms["sssp"], ms["batch"]) < 2 * ms["copy"]
+
+
+# The validation's pieces: rows around the length that a whole wave walks, alone and
+# behind each other, and around the pieces of 128 rows and entries of small graphs
+@pytest.mark.parametrize("length", [1, 63, 125, 126, 127, 128, 129, 255, 256, 257, 5000])
+def test_validation_counts_in_pieces(arena, oracle, length):
+    n, edges = two_stars(length)
+    n += 200  # isolated vertices at the end
+    g, ref = build(arena, n, edges)
+    b = arena.bfs_create(g)
+    for root in (0, length + 1):
+        arena.bfs(g, b, root)
+        pred = arena.bfs_pred(b)
+        trees = [pred.copy() for _ in range(6)]
+        trees[1][1] = n - 1          # a centre's parent is no neighbour of it
+        trees[2][0 if root else 2] = n + 5
+        trees[3][length + 1] = length + 1
+        trees[4][[0, 1]] = [1, 0]    # a cycle of the two centres
+        trees[5][n - 2] = 1          # an isolated vertex with a parent
+        for k, t in enumerate(trees):
+            arena.to_device(b.pred, t)
+            ok, errors = arena.bfs_validate(g, b, root)
+            assert errors == oracle.bfs_validate(ref, t, root) and ok == (errors == 0), (root, k)
+
+
+# 64 hubs with following ids, and the same graph with its ids shuffled: the rows of the
+# hubs are cut into pieces either way. 17 times when one wave walks all of them.
+def test_validation_of_hubs_that_follow_each_other(arena):
+    import time
+    rng = np.random.default_rng(2)
+    n, ne = 500064, 3 * 10**6
+    e = np.stack([rng.integers(0, 64, ne), 64 + rng.integers(0, n - 64, ne)], 1)
+    ms = []
+    for ids in (np.arange(n), rng.permutation(n)):
+        m = arena.mark()
+        g = arena.csr(arena.upload_tuples(ids[e], rng.random(ne).astype(np.float32)), n)
+        b = arena.bfs_create(g)
+        root = int(ids[0])
+        arena.bfs(g, b, root)
+        times = []
+        for _ in range(6):
+            t0 = time.perf_counter()
+            assert arena.bfs_validate(g, b, root) == (True, 0)
+            times.append(time.perf_counter() - t0)
+        ms.append(1e3 * min(times))
+        arena.release(m)
+    print(f"[hub validate] ids in order {ms[0]:.3f} ms, shuffled {ms[1]:.3f} ms", flush=True)
+    assert ms[0] < 3 * ms[1]
