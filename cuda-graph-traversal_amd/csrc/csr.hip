@@ -270,24 +270,54 @@ __global__ __launch_bounds__(kPartThreads) void partition_kernel(PartArgs a) {
     }
 }
 
+// Words after pass 1's bucket counts.
+constexpr u32 kPartBad = kPartBins, kPartSeen = kPartBins + 1, kPartNear = kPartBins + 2, kPartWords = kPartBins + 3;
+
 // Entries per bucket of pass 1, from the tuples; flags endpoints out of range.
+// Every eighth block also counts its tuples with one before them in the wave,
+// and those of them whose endpoints both lie next to, but not on, the endpoints
+// of the one before (see tuples_are_near): a sample, since all waves' counts
+// would queue at these two words for longer than the pass takes.
+constexpr u64 kNearVertices = 16;  // a 64-byte line of the degrees
+__device__ __forceinline__ bool near_but_not_on(u64 a, u64 b) { return a - b + kNearVertices <= 2 * kNearVertices && a != b; }
 __global__ __launch_bounds__(1024) void partition_count_tuples(const Packed_Edge *__restrict__ edges, u64 ne, u64 n,
-                                                               u32 shift, u32 *__restrict__ counts,
-                                                               u32 *__restrict__ bad) {
-    __shared__ u32 h[kPartBins];
+                                                               u32 shift, u32 *__restrict__ counts) {
+    __shared__ u32 h[kPartBins], pairs[2];
     for (u32 b = threadIdx.x; b < kPartBins; b += blockDim.x) h[b] = 0;
+    if (threadIdx.x < 2) pairs[threadIdx.x] = 0;
     __syncthreads();
-    for (u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x; i < ne; i += (u64)gridDim.x * blockDim.x) {
-        const Packed_Edge e = edges[i];
+    const u32 lane = lane_id();
+    const u64 step = (u64)gridDim.x * blockDim.x;
+    u32 seen = 0, near = 0;
+    for (u64 i0 = (u64)blockIdx.x * blockDim.x + (threadIdx.x - lane); i0 < ne; i0 += step) {
+        const u64 i = i0 + lane;
+        const Packed_Edge e = edges[min(i, ne - 1)];
+        if (blockIdx.x % 8 == 0) {
+            const int before = lane ? (int)lane - 1 : 0;
+            const u64 p0 = shfl64(e.v0, before), p1 = shfl64(e.v1, before);
+            const bool pair = lane && i < ne;
+            seen += pair;
+            near += pair && near_but_not_on(e.v0, p0) && near_but_not_on(e.v1, p1);
+        }
+        if (i >= ne) continue;
         if (e.v0 >= n || e.v1 >= n) {
-            atomicOr(bad, 1u);
+            atomicOr(&counts[kPartBad], 1u);
             continue;
         }
         if (e.v0 == e.v1) continue;
         atomicAdd(&h[(u32)(e.v0 >> shift)], 1u);
         atomicAdd(&h[(u32)(e.v1 >> shift)], 1u);
     }
+    if (blockIdx.x % 8 == 0) {
+        seen = wave_sum(seen);
+        near = wave_sum(near);
+        if (lane == 0) {
+            atomicAdd(&pairs[0], seen);
+            atomicAdd(&pairs[1], near);
+        }
+    }
     __syncthreads();
+    if (threadIdx.x < 2 && pairs[threadIdx.x]) atomicAdd(&counts[threadIdx.x ? kPartNear : kPartSeen], pairs[threadIdx.x]);
     for (u32 b = threadIdx.x; b < kPartBins; b += blockDim.x)
         if (h[b]) atomicAdd(&counts[b], h[b]);
 }
@@ -1598,6 +1628,18 @@ void build_traversal_copy(Worker_State *ws, Oned_Graph *g) {
 // 876 / 800, S14 1259 / 1045, S16 2346 / 1762, S18 5046 / 3673, S20 14348 / 11278,
 // S22 47674 / 34400.
 constexpr u64 kPartitionTuples = 1ull << 16;
+// So do lists below this with at most two tuples a vertex, whose atomics seldom
+// meet: 1e5 tuples over 1e5 vertices, a path 378 / 432, uniform 379 / 398; 3e5 over
+// 1e5 uniform 417 / 406, 1e6 over 5e5 684 / 684, 2e6 over 2e6 1240 / 1078.
+constexpr u64 kPartitionSparse = 1ull << 18;
+// And lists of any length whose tuples lie near the ones before them (meshes,
+// paths and bands numbered along themselves): a wave's atomics and writes then
+// share lines, without meeting on a vertex, which the partition cannot better.
+// A 1000 x 1000 grid 633 / 771, 4000 x 4000 4585 / 6016, a path of 1e7 2439 / 3038, a
+// binary tree of 1e7 (half of the tuples near) 3100 / 3631; a band of five entries
+// after another at each vertex (one in five near) 1363 / 1141. Half of that last
+// but one case's share is the line.
+static bool tuples_are_near(u32 seen, u32 near) { return (u64)near * 8 >= (u64)seen * 3; }
 
 static bool bad_endpoints(u64 n) {
     fail("oned_graph_from_tuple_graph: tuple endpoint outside [0, %llu)", (unsigned long long)n);
@@ -1643,15 +1685,18 @@ static bool fill_direct(Worker_State *ws, const Tuple_Graph *tg, Oned_Graph *g) 
     return !failed();
 }
 
-// Whether the partition path is taken: large lists, whose counts fit 32 bits,
-// when the arena has room for its scratch (16 bytes an entry beside the
-// columns and weights; the copies built later need as much).
+// Whether the partition path is tried: lists above the limits whose entry counts
+// fit 32 bits (below 2^31 tuples), when the arena has room for its scratch (16
+// bytes an entry beside the columns and weights, 5 a vertex, and 64 MiB for
+// offsets and rounding; the copies built later need as much).
 static bool partition_pays(const Worker_State *ws, u64 n, u64 ne) {
     const u64 room = ws->gpu_arena.reserved - ws->gpu_arena.used;
-    return ne >= kPartitionTuples && 2 * ne < (1ull << 32) && 2 * ne * 24 + n * 5 + (64ull << 20) <= room;
+    return ne >= kPartitionTuples && (ne >= kPartitionSparse || ne > 2 * n) && 2 * ne < (1ull << 32) &&
+           2 * ne * 24 + n * 5 + (64ull << 20) <= room;
 }
 
-// The same arrays by partition (see partition_kernel).
+// The same arrays by partition (see partition_kernel), unless the tuples turn
+// out to be near each other.
 static bool fill_partitioned(Worker_State *ws, const Tuple_Graph *tg, Oned_Graph *g) {
     Context &c = ctx();
     const hipStream_t s = c.stream;
@@ -1664,19 +1709,21 @@ static bool fill_partitioned(Worker_State *ws, const Tuple_Graph *tg, Oned_Graph
     const u32 shift1 = bits - d1, shift2 = bits <= 18 ? 0 : shift1 / 2;
     const u64 nb1 = ((n - 1) >> shift1) + 1, nb2 = ((n - 1) >> shift2) + 1;
     // pass 1's counts, whose sum is the number of entries
-    std::vector<u32> h(nb1 + 1);
+    std::vector<u32> h(kPartWords);
     std::vector<u64> first(nb1 + 1);
-    u32 *count1 = (u32 *)arena_alloc(ws, (kPartBins + 1) * sizeof(u32), "CSR partition counts");
+    u32 *count1 = (u32 *)arena_alloc(ws, kPartWords * sizeof(u32), "CSR partition counts");
     if (failed()) return false;
-    G500_HIP(hipMemsetAsync(count1, 0, (kPartBins + 1) * sizeof(u32), s));
-    partition_count_tuples<<<(unsigned)c.num_cus * 2, 1024, 0, s>>>(tg->edges, ne, n, shift1, count1,
-                                                                   count1 + kPartBins);
+    G500_HIP(hipMemsetAsync(count1, 0, kPartWords * sizeof(u32), s));
+    partition_count_tuples<<<(unsigned)c.num_cus * 2, 1024, 0, s>>>(tg->edges, ne, n, shift1, count1);
     G500_HIP(hipGetLastError());
-    G500_HIP(hipMemcpyAsync(h.data(), count1, nb1 * sizeof(u32), hipMemcpyDeviceToHost, s));
-    G500_HIP(hipMemcpyAsync(&h[nb1], count1 + kPartBins, sizeof(u32), hipMemcpyDeviceToHost, s));
+    G500_HIP(hipMemcpyAsync(h.data(), count1, kPartWords * sizeof(u32), hipMemcpyDeviceToHost, s));
     sync();
     if (failed()) return false;
-    if (h[nb1]) return bad_endpoints(n);
+    if (h[kPartBad]) return bad_endpoints(n);
+    if (tuples_are_near(h[kPartSeen], h[kPartNear])) {
+        ws->gpu_arena.used = mark;
+        return fill_direct(ws, tg, g);
+    }
     u64 m = 0;
     for (u64 b = 0; b < nb1; ++b) {
         first[b] = m;
