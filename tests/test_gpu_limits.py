@@ -355,3 +355,36 @@ def test_orders_of_tuples(arena, oracle, ne, kind):
          "descending": np.stack([ne - i, ne - i + 16], 1), "far": np.stack([i * 17 % ne, i], 1)}[kind]
     g, ref = build(arena, ne + 20, e)
     csr_equal(arena, g, ref)
+
+
+# The SSSP copy of a graph without hubs: its rows are judged by the exact hub table,
+# 128 bytes a vertex written and read (one copy's time) and about as much again for the
+# passes over rows and entries. 2.15 copies on a path of 1e7 vertices; 2.8 with the 8-bit
+# table, which pays only where many rows reach a hub.
+def test_sssp_copy_of_a_graph_without_hubs(arena):
+    n = 10**7
+    e = np.stack([np.arange(n - 1), np.arange(1, n)], 1)
+    tg = arena.upload_tuples(e, np.random.default_rng(5).random(n - 1).astype(np.float32))
+
+    def best(run):
+        ms = []
+        for _ in range(6):
+            m = arena.mark()
+            run()
+            ms.append(arena.lib.g500_last_run_ms())
+            arena.release(m)
+        return min(ms)
+
+    old = arena.get_param("sssp_prune")
+    try:
+        ms = {}
+        for prune in (0, 1):
+            arena.set_param("sssp_prune", prune)
+            ms[prune] = best(lambda: arena.csr(tg, n))
+    finally:
+        arena.set_param("sssp_prune", old)
+    size = 128 * n
+    src, dst = (arena.lib._worker_arena_push_array(arena.ws, size, 1, 256, None) for _ in range(2))
+    ms["copy"] = best(lambda: arena.lib.g500_copy_device(dst, src, size))
+    print(f"[no hubs ms] {ms}", flush=True)
+    assert ms[1] - ms[0] < 2.5 * ms["copy"]
