@@ -234,9 +234,9 @@ __device__ __forceinline__ u32 wave_append(u32 *counter, bool want) {
 // kDppShr + n), or, for the rows in ROWS, the last lane of the row before
 // (kDppBcast15) or lane 31 (kDppBcast31). Lanes without a source take `old`.
 // A register move in the vector ALU, where a shuffle is a round trip through
-// the LDS pipe. Scans and sums by shuffles / by these, us: SSSP S12 523 / 504,
-// S19 1769 / 1658, batched SSSP of 7 roots S16 5016 / 4697, of 32 S22 39205 / 37589,
-// batched BFS S16 785 / 647.
+// the LDS pipe. Scans and sums by shuffles / by these, us: SSSP S12 338 / 316,
+// S19 1178 / 1157, batched SSSP of 7 roots S16 3772 / 3663, of 32 S22 58365 / 56946,
+// batched BFS S16 718 / 650.
 constexpr int kDppShr = 0x110, kDppBcast15 = 0x142, kDppBcast31 = 0x143;
 template <int CTRL, int ROWS, typename T>
 __device__ __forceinline__ T lane_before(T old, T v) {

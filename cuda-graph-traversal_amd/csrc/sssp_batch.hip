@@ -202,9 +202,11 @@ struct BTarget {
 // roots of one entry all meet at their target's vmin, and most do not lower it;
 // where the atomics bound the steps the read saves more than it costs, in the
 // smaller grids of the roomy build it is one more load to wait for. us, without /
-// with: 32 roots S22 35000 / 32400, over 300001 uniform vertices 6330 / 6060, S19
-// 10900 / 10750, 16 roots S19 6590 / 6710; roomy 32 roots S16 5400 / 5480, 7 roots
-// S19 7990 / 8310; 7 roots S22 (packed) 22200 / 22500.
+// with: packed 32 roots S22 with offsets 33070 / 31240, over 300001 uniform
+// vertices 7265 / 6800, S19 17690 / 18150, 7 roots S22 23360 / 23730, 16 roots S19
+// 11530 / 11820; roomy 32 roots S16 7180 / 7460, 7 roots S19 6930 / 7240. A serving
+// slot on a small graph is packed too and loses a little: a quarter of the device,
+// 7 roots with offsets, S12 1449 / 1444, S16 2700 / 2721, S20 8940 / 9116.
 template <bool SCREEN>
 struct RelaxTarget : BTarget {
     static constexpr bool screen = SCREEN;
@@ -397,10 +399,11 @@ struct Probe {
 // tiers (one item's row, so a round costs fewer registers there). With four
 // waves on a SIMD the kernel has 128 registers a lane and spills what does not
 // fit; more rounds spill more than their loads in flight hide (4 and 8 rounds
-// 188 spilled registers, 2 and 4 113). ms at 7 roots S12 / 7 roots S19 /
-// 32 roots S22: 4, 8 rounds 2.16 / 9.65 / 35.8; 4, 4 1.95 / 8.7 / 35.4; 2, 4
-// 1.87 / 8.5 / 35.2; 2, 2 1.85 / 8.6 / 36.6; 2, 5 1.88 / 8.6 / 35.7; 1, 2
-// 1.81 / 8.7 / 37.1.
+// 221 spilled registers, 2 and 4 121). ms at 7 roots S12 / 7 roots S19 (both roomy) /
+// 32 roots S22 with offsets / 32 over 300001 uniform vertices: 4, 8 rounds
+// 2.29 / 7.25 / 31.5 / 7.69; 4, 4 2.31 / 7.07 / 31.1 / 6.96; 2, 4 2.22 / 6.98 / 31.2 /
+// 6.80; 2, 5 2.28 / 6.98 / 31.7 / 7.07; 2, 2 2.21 / 7.10 / 32.4 / 6.73; 1, 2
+// 2.13 / 7.25 / 32.9 / 6.82.
 constexpr int kRounds = 2;
 constexpr int kWideRounds = 4;
 
